@@ -129,7 +129,8 @@ private:
 	std::vector<int32_t> partTexture_;
 	std::vector<size_t> partTextureOffset_;
 	bool alphaAny_ = false;
-	bool orthogonalAny_ = false;  // a task with an orthogonal camera
+	bool mixedCanvas_ = false;    // a canvas with tasks of both projections
+	std::vector<uint8_t> projections_;  // per canvas: 1 = a perspective task, 2 = an orthogonal one
 	bool oddCanvas_ = false;      // a canvas of odd height
 	bool wideCanvas_ = false;     // a canvas wider than the visibility raster's 16-bit row columns
 	int32_t commandCapacity_ = 0, pairCapacity_ = 0;
@@ -187,10 +188,10 @@ private:
 	uint64_t cleanGenerations_[3] = {0, 0, 0};
 	int32_t cleanTiles_ = 0, cleanCanvases_ = 0;
 	void dropGraph();
-	// The visibility raster reproduces the in-order result when every command is Solid and
-	// perspective and no canvas has an odd height.
+	// The visibility raster reproduces the in-order result when every command is Solid and each
+	// canvas's commands have one projection.
 	bool deferredRaster(const RenderOptions &o) const {
-		return o.rasterPath == 0 && !alphaAny_ && !orthogonalAny_ && !oddCanvas_ && !wideCanvas_;
+		return o.rasterPath == 0 && !alphaAny_ && !mixedCanvas_ && !wideCanvas_;
 	}
 };
 

@@ -63,7 +63,8 @@ void Frame::reset(int32_t tileConfig) {
 	partTexture_.clear();
 	partTextureOffset_.clear();
 	alphaAny_ = false;
-	orthogonalAny_ = false;
+	mixedCanvas_ = false;
+	projections_.clear();
 	occlusionGrid_ = nullptr;
 	gridW_ = gridH_ = 0;
 	oddCanvas_ = false;
@@ -86,9 +87,11 @@ int32_t Frame::addCanvas(const CanvasHost &c) {
 	d.visibility = c.visibility;
 	d.gradColor = c.gradColor;
 	d.diffStride = c.diffStride;
+	d.affine = 0;
 	if (c.height & 1) oddCanvas_ = true;
 	if (c.width > 32767) wideCanvas_ = true;
 	canvases_.push_back(d);
+	projections_.push_back(0);
 	canvasTileEnd_.push_back(d.tileBase + d.tilesX * d.tilesY);
 	return (int32_t)canvases_.size() - 1;
 }
@@ -131,7 +134,10 @@ int Frame::addTask(const ModelView &m, const float *transform, const CameraParam
 		partTexture_.push_back(textureSlot(m.partLight[p]));
 	}
 	if (m.filter != 0) alphaAny_ = true;
-	if (!camera.perspective) orthogonalAny_ = true;
+	uint8_t &projections = projections_[(size_t)canvas];
+	projections |= camera.perspective ? 1 : 2;
+	if (projections == 3) mixedCanvas_ = true;
+	if (!camera.perspective) canvases_[(size_t)canvas].affine = 1;
 	tasks_.push_back(t);
 	taskPointEnd_.push_back(t.pointBase + m.pointCount);
 	taskFanEnd_.push_back(t.fanBase + m.fanCount);
@@ -140,6 +146,24 @@ int Frame::addTask(const ModelView &m, const float *transform, const CameraParam
 
 static inline int32_t blocksOf(int64_t n, int32_t size) { return (int32_t)((n + size - 1) / size); }
 static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// The visibility raster of a frame with one tile shape: RGBA8 or differentiable, one workgroup per
+// tile or persistent, for even perspective canvases alone or for any (general).
+template <int TW, int TH, int P, bool GENERAL>
+static void launchDeferredForm(const FrameDev &f, int32_t grid, hipStream_t stream) {
+	if (f.mode == 1) hipLaunchKernelGGL((k_raster_deferred_diff<TW, TH, P, GENERAL>), dim3(grid), dim3(TW * TH / 4), 0, stream, f);
+	else hipLaunchKernelGGL((k_raster_deferred<TW, TH, P, GENERAL>), dim3(grid), dim3(TW * TH / 4), 0, stream, f);
+}
+template <int TW, int TH>
+static void launchDeferred(const FrameDev &f, int32_t grid, int32_t persistent, bool general, hipStream_t stream) {
+	if (persistent) {
+		if (general) launchDeferredForm<TW, TH, 1, true>(f, grid, stream);
+		else launchDeferredForm<TW, TH, 1, false>(f, grid, stream);
+	} else {
+		if (general) launchDeferredForm<TW, TH, 0, true>(f, grid, stream);
+		else launchDeferredForm<TW, TH, 0, false>(f, grid, stream);
+	}
+}
 
 int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks, int32_t tileBlocks, bool events, int parts,
                    bool skipBegin) {
@@ -182,39 +206,19 @@ int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks,
 		case 2: hipLaunchKernelGGL((k_raster_depth<32, 32>), dim3(xcdGrid(tileTotal)), dim3(32 * 32 / 4), 0, stream, f); break;
 		default: hipLaunchKernelGGL((k_raster_depth<16, 16>), dim3(xcdGrid(tileTotal)), dim3(16 * 16 / 4), 0, stream, f); break;
 		}
-	} else if (o.mode == 1) {
-		const bool deferred = deferredRaster(o);
-		switch (tileConfig_) {
-		case 1:
-			if (!deferred) hipLaunchKernelGGL((k_raster_diff<32, 16>), dim3(grid), dim3(128), 0, stream, f, persistent);
-			else if (persistent) hipLaunchKernelGGL((k_raster_deferred_diff<32, 16, 1>), dim3(grid), dim3(128), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred_diff<32, 16, 0>), dim3(grid), dim3(128), 0, stream, f);
-			break;
-		case 2:
-			if (!deferred) hipLaunchKernelGGL((k_raster_diff<32, 32>), dim3(grid), dim3(256), 0, stream, f, persistent);
-			else if (persistent) hipLaunchKernelGGL((k_raster_deferred_diff<32, 32, 1>), dim3(grid), dim3(256), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred_diff<32, 32, 0>), dim3(grid), dim3(256), 0, stream, f);
-			break;
-		default:
-			if (!deferred) hipLaunchKernelGGL((k_raster_diff<16, 16>), dim3(grid), dim3(64), 0, stream, f, persistent);
-			else if (persistent) hipLaunchKernelGGL((k_raster_deferred_diff<16, 16, 1>), dim3(grid), dim3(64), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred_diff<16, 16, 0>), dim3(grid), dim3(64), 0, stream, f);
-			break;
-		}
 	} else if (deferredRaster(o)) {
+		bool general = oddCanvas_;
+		for (uint8_t p : projections_) general = general || (p & 2) != 0;
 		switch (tileConfig_) {
-		case 1:
-			if (persistent) hipLaunchKernelGGL((k_raster_deferred<32, 16, 1>), dim3(grid), dim3(32 * 16 / 4), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred<32, 16, 0>), dim3(grid), dim3(32 * 16 / 4), 0, stream, f);
-			break;
-		case 2:
-			if (persistent) hipLaunchKernelGGL((k_raster_deferred<32, 32, 1>), dim3(grid), dim3(32 * 32 / 4), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred<32, 32, 0>), dim3(grid), dim3(32 * 32 / 4), 0, stream, f);
-			break;
-		default:
-			if (persistent) hipLaunchKernelGGL((k_raster_deferred<16, 16, 1>), dim3(grid), dim3(16 * 16 / 4), 0, stream, f);
-			else hipLaunchKernelGGL((k_raster_deferred<16, 16, 0>), dim3(grid), dim3(16 * 16 / 4), 0, stream, f);
-			break;
+		case 1: launchDeferred<32, 16>(f, grid, persistent, general, stream); break;
+		case 2: launchDeferred<32, 32>(f, grid, persistent, general, stream); break;
+		default: launchDeferred<16, 16>(f, grid, persistent, general, stream); break;
+		}
+	} else if (o.mode == 1) {
+		switch (tileConfig_) {
+		case 1: hipLaunchKernelGGL((k_raster_diff<32, 16>), dim3(grid), dim3(128), 0, stream, f, persistent); break;
+		case 2: hipLaunchKernelGGL((k_raster_diff<32, 32>), dim3(grid), dim3(256), 0, stream, f, persistent); break;
+		default: hipLaunchKernelGGL((k_raster_diff<16, 16>), dim3(grid), dim3(64), 0, stream, f, persistent); break;
 		}
 	} else switch (tileConfig_) {
 	case 1: hipLaunchKernelGGL((k_raster<32, 16>), dim3(grid), dim3(128), 0, stream, f, persistent); break;

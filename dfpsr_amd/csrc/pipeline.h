@@ -59,6 +59,7 @@ struct CanvasDev {
 	int32_t *visibility;
 	const float *gradColor;
 	int32_t diffStride;
+	int32_t affine;                    // its tasks' cameras are orthogonal (the smaller depth wins)
 };
 
 // One draw command: a (sub-)triangle that passed culling, clipping and the front-face test.
@@ -165,9 +166,9 @@ __global__ void k_scan_tiles_local(FrameDev f);
 __global__ void k_scan_tiles_add(FrameDev f);
 __global__ void k_bin_fill(FrameDev f);
 template <int TW, int TH> __global__ void k_raster(FrameDev f, int32_t persistent);
-template <int TW, int TH, int P> __global__ void k_raster_deferred(FrameDev f);
+template <int TW, int TH, int P, bool GENERAL> __global__ void k_raster_deferred(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_diff(FrameDev f, int32_t persistent);
-template <int TW, int TH, int P> __global__ void k_raster_deferred_diff(FrameDev f);
+template <int TW, int TH, int P, bool GENERAL> __global__ void k_raster_deferred_diff(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_depth(FrameDev f);
 __global__ void k_probe_edge_side(const int64_t *n, const int64_t *d, const int32_t *L, const int32_t *R, int32_t count, int32_t *out);
 __global__ void k_backward(FrameDev f, int32_t *head);

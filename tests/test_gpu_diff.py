@@ -112,6 +112,29 @@ def test_forward_visibility_raster_equals_in_order_raster(api):
                                       b.view(np.uint32) if b.dtype == np.float32 else b), f"run {k} view {i}"
 
 
+def test_forward_on_odd_heights_equals_in_order_raster(api):
+    """The same equality on canvases of odd height, whose last row the visibility raster walks in
+    submission order."""
+    views = S.sphere_views(6, 2, 75, 45, seed=8)
+    for v in views:  # near enough that the object reaches the last row
+        v.cam_location = S.look_at(np.asarray(v.cam_location[:3], np.float64) * 0.55)
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    out = []
+    for tile_config in (0, 1, 2):
+        for path in (0, 1):
+            gv = api.GpuViews(views)
+            r = api.DiffRenderer()
+            r.forward(gv.model, gv.views, tex, None, api.tuning(clear=True, raster_path=path, tile_config=tile_config))
+            torch.cuda.synchronize()
+            out.append([(gv.color[i].cpu().numpy(), gv.visibility[i].cpu().numpy(), gv.depth[i].cpu().numpy())
+                        for i in range(len(views))])
+    assert all((o[1][-1] >= 0).any() for o in out[0])
+    for k in range(1, len(out)):
+        for i in range(len(views)):
+            for a, b in zip(out[0][i], out[k][i]):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"run {k} view {i}"
+
+
 def test_adjoint_same_for_every_tile_shape(api):
     """The adjoint walks whatever tiles the forward used: texture and multiplier gradients agree
     across tile shapes up to the order of the float atomics."""

@@ -237,6 +237,60 @@ def test_visibility_raster_equals_in_order_raster(api, scene):
                   scene.name.endswith("_id_even"))
 
 
+def odd_scene(width, height, orthogonal, canvases, seed):
+    """Large overlapping triangles, whose spans' unclipped quads reach the odd canvas's last row, over
+    a depth canvas that holds ordinary values, infinities and NaN."""
+    sc = S.cube_soup(width=width, height=height, triangles=120, seed=seed, spread=0.9, cam_distance=2.0,
+                     name=f"odd_{width}x{height}_{'ortho' if orthogonal else 'persp'}_{canvases}")
+    sc.perspective = not orthogonal
+    sc.has_color, sc.has_depth = "c" in canvases, "d" in canvases
+    held = S.Rng(seed + 5).uniform(width * height, 0.0, 0.6 if not orthogonal else 4.0).reshape(height, width)
+    held.reshape(-1)[::7] = np.inf if orthogonal else 0.0
+    held.reshape(-1)[3::11] = np.nan
+    held.reshape(-1)[5::13] = -np.inf
+    sc.initial_depth = held
+    return sc
+
+
+@pytest.mark.parametrize("orthogonal", [False, True])
+@pytest.mark.parametrize("canvases", ["cd", "c", "d"])
+@pytest.mark.parametrize("size", [(1, 1), (61, 17), (33, 33), (130, 47), (64, 32)])
+def test_visibility_raster_of_odd_heights_and_orthogonal_cameras(api, size, canvases, orthogonal):
+    """The visibility raster walks an odd canvas's last row in order and reverses its depth order under
+    an orthogonal camera: the same canvases as the in-order raster, bit for bit, for every tile shape,
+    with and without persistent workgroups; and the oracle's."""
+    sc = odd_scene(size[0], size[1], orthogonal, canvases, seed=size[0] * 7 + size[1])
+    print(f"[gpu] odd rows {sc.name}", flush=True)
+    results = []
+    for tile_config in (0, 1, 2):
+        for path, persistent in ((1, 0), (0, 0), (0, 2)):
+            r = api.renderer_create()
+            api.renderer_setTuning(r, api.tuning(tile_config=tile_config, raster_path=path, persistent_per_cu=persistent))
+            results.append(api.render_scene(sc, r))
+    for c, d in results[1:]:
+        assert np.array_equal(c, results[0][0]) and np.array_equal(d.view(np.uint32), results[0][1].view(np.uint32))
+    assert_parity(sc, results[0], H.oracle_render(sc))
+
+
+def test_canvas_with_both_projections(api):
+    """A frame whose tasks mix perspective and orthogonal cameras on one canvas changes the direction of
+    the depth test between commands: both raster settings draw it in order."""
+    persp, ortho = odd_scene(90, 41, False, "cd", 3), odd_scene(90, 41, True, "cd", 4)
+    a, b = api.GpuScene(persp), api.GpuScene(ortho)
+    out = []
+    for path in (0, 1):
+        color, depth = np.zeros((41, 90), np.uint32), persp.initial_depth.copy()
+        r = api.renderer_create()
+        api.renderer_setTuning(r, api.tuning(raster_path=path))
+        api.renderer_begin(r, api.host_image(color), api.host_image(depth))
+        for g in (a, b, a):
+            g.give(r)
+        api.renderer_end(r)
+        out.append((color, depth))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1].view(np.uint32), out[1][1].view(np.uint32))
+    assert (out[0][0] != 0).any()
+
+
 def test_direct_bins_grow_to_the_longest_tile_list(api):
     """Tiles holding more commands than the direct bins' starting size (64) make the first frame
     overflow them: the renderer grows the bins to the longest list and draws the frame again
