@@ -87,7 +87,7 @@ int32_t Frame::addCanvas(const CanvasHost &c) {
 	d.visibility = c.visibility;
 	d.gradColor = c.gradColor;
 	d.diffStride = c.diffStride;
-	d.affine = 0;
+	d.affine = d.fans = d.dense = 0;
 	if (c.height & 1) oddCanvas_ = true;
 	if (c.width > 32767) wideCanvas_ = true;
 	canvases_.push_back(d);
@@ -137,7 +137,10 @@ int Frame::addTask(const ModelView &m, const float *transform, const CameraParam
 	uint8_t &projections = projections_[(size_t)canvas];
 	projections |= camera.perspective ? 1 : 2;
 	if (projections == 3) mixedCanvas_ = true;
-	if (!camera.perspective) canvases_[(size_t)canvas].affine = 1;
+	CanvasDev &cv = canvases_[(size_t)canvas];
+	if (!camera.perspective) cv.affine = 1;
+	cv.fans += m.fanCount;
+	cv.dense = (int64_t)cv.fans * DENSE_PIXELS_PER_FAN > (int64_t)cv.width * cv.height ? 1 : 0;
 	tasks_.push_back(t);
 	taskPointEnd_.push_back(t.pointBase + m.pointCount);
 	taskFanEnd_.push_back(t.fanBase + m.fanCount);
@@ -337,6 +340,8 @@ int Frame::run(const RenderOptions &o) {
 		f.tileH = tileConfigH(tileConfig_);
 		f.tileShiftW = f.tileW == 32 ? 5 : 4;
 		f.tileShiftH = f.tileH == 32 ? 5 : 4;
+		f.denseAny = 0;
+		for (const CanvasDev &cv : canvases_) f.denseAny |= cv.dense;
 		f.alphaAny = alphaAny_ ? 1 : 0;
 		// The differentiable frames fill in the raster only with 32-pixel-wide tiles: with 16x16
 		// tiles the separate fill kernel streams the float canvases faster than the one-wave
@@ -454,9 +459,10 @@ int Frame::run(const RenderOptions &o) {
 			}
 		}
 		if (overflow & 2) {
-			// Tile pairs no longer fit: the packed lists grow to the frame's pair count, the
-			// direct bins to the longest tile list with a quarter to spare.
-			pairCapacity_ = hostCounters_[1] + 1024;
+			// Tile pairs no longer fit: the packed lists grow to the frame's pair count (and its
+			// records, which count the tiles that a command's bound touches and its triangle
+			// misses), the direct bins to the longest tile list with a quarter to spare.
+			pairCapacity_ = std::max(hostCounters_[1], hostCounters_[7]) + 1024;
 			if (direct) {
 				const int64_t longest = hostCounters_[6];
 				binCapacity_ = (int32_t)std::min<int64_t>(((longest + longest / 4 + 15) / 16) * 16, BIN_ENTRY_LIMIT);

@@ -59,8 +59,15 @@ struct CanvasDev {
 	int32_t *visibility;
 	const float *gradColor;
 	int32_t diffStride;
+	int32_t fans;                      // fan triangles of its tasks
+	int32_t dense;                     // fewer than DENSE_PIXELS_PER_FAN pixels per fan triangle
 	int32_t affine;                    // its tasks' cameras are orthogonal (the smaller depth wins)
 };
+
+// Canvases with fewer pixels than this per fan triangle are dense: the setup tests each of their
+// (command, tile) pairs for coverage (pairCovers).  A 1080p terrain has 16 pixels per triangle and
+// gains nothing, 256x256 views of 20 480 triangles have 3.2 and gain a third of their time.
+constexpr int32_t DENSE_PIXELS_PER_FAN = 8;
 
 // One draw command: a (sub-)triangle that passed culling, clipping and the front-face test.
 struct __attribute__((aligned(16))) Command {
@@ -116,6 +123,7 @@ struct FrameDev {
 	int32_t *hostCounters;        // pinned host copy of counters[0..7], written by the raster kernel
 	int32_t tileW, tileH;
 	int32_t tileShiftW, tileShiftH;  // log2 of tileW and tileH (the tile sides are powers of two)
+	int32_t denseAny;             // any canvas is dense
 	int32_t alphaAny;             // any task uses the Alpha filter: tiles read colour first
 	// The visibility raster fills the canvases itself (image_fill) instead of a separate clear:
 	// it then visits every tile, and empty ones only take the fill values.

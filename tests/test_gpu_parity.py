@@ -315,6 +315,36 @@ def test_direct_bins_grow_to_the_longest_tile_list(api):
     assert_parity(sc, first, H.oracle_render(sc))
 
 
+@pytest.mark.parametrize("width,height,triangles,spread,distance,orthogonal", [
+    (37, 23, 3000, 0.02, 2.5, False),    # below a pixel: most cover no pixel centre
+    (37, 23, 3000, 0.02, 2.5, True),
+    (97, 40, 2500, 1.2, 0.7, False),     # long slivers far outside the canvas, clipped near the camera
+    (64, 33, 1500, 0.3, 1.6, False),     # a few tiles each, column 0 and the last row among them
+])
+def test_dense_canvas_pairs(api, width, height, triangles, spread, distance, orthogonal):
+    """On canvases with few pixels per triangle the setup drops the (command, tile) pairs that no row
+    covers: every tile shape, both ways of building the lists and both rasters still give the oracle's
+    depth bit for bit, and so does the depth-only draw."""
+    sc = S.cube_soup(width=width, height=height, triangles=triangles, seed=triangles + width, spread=spread, cam_distance=distance)
+    sc.perspective = not orthogonal
+    if orthogonal:
+        sc.initial_depth = np.full((height, width), np.inf, np.float32)
+    assert width * height < 8 * triangles
+    print(f"[gpu] dense pairs {width}x{height} {triangles} spread {spread}", flush=True)
+    ref = H.oracle_render(sc, threads=4)
+    pairs = set()
+    for tile_config in (0, 1, 2):
+        for path, binning in ((0, 0), (0, 1), (1, 0)):
+            r = api.renderer_create()
+            api.renderer_setTuning(r, api.tuning(tile_config=tile_config, raster_path=path, binning=binning))
+            assert_parity(sc, api.render_scene(sc, r), ref)
+            pairs.add((tile_config, int(r.stats()[1])))
+    assert len(pairs) == 3  # the same pairs whatever the lists and the raster
+    depth = api.render_scene_depth(sc)
+    want = H.oracle_render_depth(sc)
+    assert np.array_equal(depth.view(np.uint32), want.view(np.uint32))
+
+
 def test_packed_lists_grow_past_their_first_pair_capacity(api):
     """Commands whose bounds span the whole canvas touch every tile, so the frame makes more
     (tile, command) pairs than the packed lists' first capacity (four per command slot): the
