@@ -345,6 +345,24 @@ def test_dense_canvas_pairs(api, width, height, triangles, spread, distance, ort
     assert np.array_equal(depth.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("triangles", [120, 300, 600, 2600, 12000])
+def test_tile_lists_longer_than_a_round(api, triangles):
+    """A canvas of one tile whose triangles all reach it: lists below and above the 128, 256 and 1,024
+    commands that the rasters sort per round, in several rounds, against the oracle."""
+    sc = S.cube_soup(width=30, height=16, triangles=triangles, seed=triangles, spread=0.7, cam_distance=2.2)
+    # A second cluster of command indices far from the first: the middle half faces away.
+    a, b = triangles // 4, 3 * triangles // 4
+    sc.indices[a:b, :3] = sc.indices[a:b, 2::-1]
+    print(f"[gpu] long lists {triangles}", flush=True)
+    ref = H.oracle_render(sc, threads=4)
+    for tile_config, path in ((1, 0), (1, 1), (0, 0), (2, 1)):
+        r = api.renderer_create()
+        api.renderer_setTuning(r, api.tuning(tile_config=tile_config, raster_path=path))
+        assert_parity(sc, api.render_scene(sc, r), ref)
+    depth, want = api.render_scene_depth(sc), H.oracle_render_depth(sc)
+    assert np.array_equal(depth.view(np.uint32), want.view(np.uint32))
+
+
 def test_packed_lists_grow_past_their_first_pair_capacity(api):
     """Commands whose bounds span the whole canvas touch every tile, so the frame makes more
     (tile, command) pairs than the packed lists' first capacity (four per command slot): the
