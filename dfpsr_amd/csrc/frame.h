@@ -153,9 +153,14 @@ private:
 	// All per-frame tables in one upload, skipped when identical to the previous frame's.
 	std::vector<uint8_t> tables_, uploadedTables_;
 	DevBuf dTables_;
-	size_t offTasks_ = 0, offFanEnd_ = 0, offPointEnd_ = 0, offCanvases_ = 0, offTileEnd_ = 0, offTextures_ = 0;
+	size_t offTasks_ = 0, offFanEnd_ = 0, offPointEnd_ = 0, offCanvases_ = 0, offTileEnd_ = 0, offTextures_ = 0, offRegionEnd_ = 0;
 	bool prepared_ = false;
 	DevBuf dShaders_, dTriangleRows_;
+	// Differentiable frames: per command the shader's inputs, per canvas pixel the adjoint's record (none
+	// when there is no memory for them: the adjoint then derives the weights), and the forwards' count.
+	DevBuf dDiffInputs_, dDiffRecords_, dForwardNumber_;
+	std::vector<int32_t> canvasRegionEnd_;
+	int64_t recordTotal_ = 0;
 	DevBuf dCanvasBase_, dFanCount_, dBlockSums_, dCommands_, dCounters_, dTileCount_, dTileOffset_, dTileFill_, dTileList_, dTileQueue_, dPairRecords_;
 	int32_t *hostCounters_ = nullptr;
 	int32_t *hostCountersDevice_ = nullptr;

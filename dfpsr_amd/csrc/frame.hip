@@ -65,6 +65,8 @@ void Frame::reset(int32_t tileConfig) {
 	alphaAny_ = false;
 	mixedCanvas_ = false;
 	projections_.clear();
+	canvasRegionEnd_.clear();
+	recordTotal_ = 0;
 	occlusionGrid_ = nullptr;
 	gridW_ = gridH_ = 0;
 	oddCanvas_ = false;
@@ -88,10 +90,13 @@ int32_t Frame::addCanvas(const CanvasHost &c) {
 	d.gradColor = c.gradColor;
 	d.diffStride = c.diffStride;
 	d.affine = d.fans = d.dense = 0;
+	d.recordBase = recordTotal_;
+	recordTotal_ += (int64_t)c.width * c.height;
 	if (c.height & 1) oddCanvas_ = true;
 	if (c.width > 32767) wideCanvas_ = true;
 	canvases_.push_back(d);
 	projections_.push_back(0);
+	canvasRegionEnd_.push_back((canvasRegionEnd_.empty() ? 0 : canvasRegionEnd_.back()) + adjointRegions(c.width) * adjointRegions(c.height));
 	canvasTileEnd_.push_back(d.tileBase + d.tilesX * d.tilesY);
 	return (int32_t)canvases_.size() - 1;
 }
@@ -248,7 +253,8 @@ int Frame::prepare() {
 	offPointEnd_ = align256(offFanEnd_ + nT * 4);
 	offCanvases_ = align256(offPointEnd_ + nT * 4);
 	offTileEnd_ = align256(offCanvases_ + nC * sizeof(CanvasDev));
-	offTextures_ = align256(offTileEnd_ + nC * 4);
+	offRegionEnd_ = align256(offTileEnd_ + nC * 4);
+	offTextures_ = align256(offRegionEnd_ + nC * 4);
 	const size_t offParts = align256(offTextures_ + textures_.size() * sizeof(TextureDesc));
 	const size_t total = align256(offParts + partTexture_.size() * 4);
 	if (dTables_.ensure(total) != hipSuccess) return fail(-4, "device allocation failed");
@@ -260,6 +266,7 @@ int Frame::prepare() {
 	std::memcpy(&tables_[offPointEnd_], taskPointEnd_.data(), nT * 4);
 	std::memcpy(&tables_[offCanvases_], canvases_.data(), nC * sizeof(CanvasDev));
 	std::memcpy(&tables_[offTileEnd_], canvasTileEnd_.data(), nC * 4);
+	std::memcpy(&tables_[offRegionEnd_], canvasRegionEnd_.data(), nC * 4);
 	std::memcpy(&tables_[offTextures_], textures_.data(), textures_.size() * sizeof(TextureDesc));
 	std::memcpy(&tables_[offParts], partTexture_.data(), partTexture_.size() * 4);
 	if (tables_ != uploadedTables_) {
@@ -292,6 +299,23 @@ int Frame::run(const RenderOptions &o) {
 	    dCanvasBase_.ensure(2 * nC * 4) != hipSuccess)
 		return fail(-4, "device allocation failed");
 
+	bool keepRecords = false;
+	if (o.mode == 1) {
+		// New memory holds no record of any forward: numbers start at one over zeroed records.
+		const uint64_t records = dDiffRecords_.generation, number = dForwardNumber_.generation;
+		if (dForwardNumber_.ensure(4) != hipSuccess) return fail(-4, "device allocation failed");
+		if (dForwardNumber_.generation != number) HIP_TRY(hipMemsetAsync(dForwardNumber_.ptr, 0, 4, stream));
+		// Without a gradient of every canvas there is no adjoint to keep records for.
+		keepRecords = true;
+		for (const CanvasDev &cv : canvases_) keepRecords = keepRecords && cv.gradColor != nullptr;
+		const size_t bytes = (size_t)recordTotal_ * sizeof(DiffRecord);
+		if (keepRecords && dDiffRecords_.ensure(bytes) != hipSuccess) {
+			(void)hipGetLastError();
+			keepRecords = false;
+		}
+		if (dDiffRecords_.generation != records) HIP_TRY(hipMemsetAsync(dDiffRecords_.ptr, 0, dDiffRecords_.bytes, stream));
+	}
+
 	for (int pass = 1; pass <= 3; pass++) {
 		const bool single = singlePass(o, fanBlocks);
 		if (single && commandCapacity_ < fanBlocks * blockCapacity_) commandCapacity_ = fanBlocks * blockCapacity_;
@@ -300,6 +324,7 @@ int Frame::run(const RenderOptions &o) {
 		const size_t listEntries = direct ? (size_t)tileTotal * binCapacity_ : (size_t)pairCapacity_;
 		if (dCommands_.ensure((size_t)commandCapacity_ * sizeof(Command)) != hipSuccess ||
 		    (o.mode == 0 && dShaders_.ensure((size_t)commandCapacity_ * sizeof(ShaderInputs)) != hipSuccess) ||
+		    (o.mode == 1 && dDiffInputs_.ensure((size_t)commandCapacity_ * sizeof(DiffInputs)) != hipSuccess) ||
 		    dTriangleRows_.ensure((size_t)commandCapacity_ * sizeof(TriangleRows)) != hipSuccess ||
 		    dTileList_.ensure(listEntries * 4) != hipSuccess ||
 		    (!direct && dPairRecords_.ensure((size_t)pairCapacity_ * sizeof(PairRecord)) != hipSuccess))
@@ -354,6 +379,13 @@ int Frame::run(const RenderOptions &o) {
 		f.ftexLog2w = ftexLog2w_;
 		f.ftexLog2h = ftexLog2h_;
 		f.multipliers = multipliers_;
+		if (o.mode == 1) {
+			f.diffInputs = dDiffInputs_.as<DiffInputs>();
+			f.diffRecords = keepRecords ? dDiffRecords_.as<DiffRecord>() : nullptr;
+			f.forwardNumber = dForwardNumber_.as<int32_t>();
+			f.canvasRegionEnd = (const int32_t *)(base + offRegionEnd_);
+			f.regionTotal = canvasRegionEnd_.back();
+		}
 		f.blockCapacity = single ? blockCapacity_ : 0;
 		// The raster leaves the counts zeroed for the next frame on the common path: one pass of
 		// setup, direct bins, one workgroup per tile, no graph.  A frame may then skip the begin
@@ -508,16 +540,24 @@ int Frame::occludeExisting(float *deviceGrid, int32_t gridW, int32_t gridH) {
 	return 0;
 }
 
+static constexpr int32_t ADJOINT_UNITS_PER_CU = 8;
+
 int Frame::backward(float *gradTexture, float *gradMultipliers, const RenderOptions &o) {
 	if (!lastRunValid_ || lastRun_.mode != 1) return fail(-2, "backward needs a differentiable forward pass first");
 	FrameDev f = lastRun_;
 	f.gradTexture = gradTexture;
 	f.gradMultipliers = gradMultipliers;
-	int32_t *head = f.counters + 5;
-	const int32_t grid = o.persistentPerCU > 0 ? deviceCUs_ * o.persistentPerCU : f.tileTotal;
+	int32_t *heads = f.counters + 9;
+	// Regions are cut into bands of rows until every CU has some: fewer, larger ones empty their tables
+	// less often, but a few small views must not leave the chip idle.
+	f.regionBands = 1;
+	while (f.regionBands < 4 && f.regionTotal * f.regionBands < ADJOINT_UNITS_PER_CU * deviceCUs_) f.regionBands *= 2;
+	const int32_t units = f.regionTotal * f.regionBands;
+	const int32_t grid = o.persistentPerCU > 0 ? std::min(deviceCUs_ * o.persistentPerCU, units) : units;
 	auto enqueueBackward = [&]() -> int {
-		hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, stream, head, 1, 0);
-		hipLaunchKernelGGL(k_backward, dim3(grid), dim3(256), 0, stream, f, head);
+		hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, stream, heads, 3, 0);
+		if (f.diffRecords) hipLaunchKernelGGL(k_backward<false>, dim3(grid), dim3(256), 0, stream, f, heads);
+		hipLaunchKernelGGL(k_backward<true>, dim3(grid), dim3(256), 0, stream, f, heads);
 		HIP_TRY(hipGetLastError());
 		return 0;
 	};

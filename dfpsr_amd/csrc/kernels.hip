@@ -125,6 +125,21 @@ __device__ __forceinline__ void recordPair(const FrameDev &f, int32_t r, int32_t
 	else atomicOr(&f.counters[2], 2);
 }
 
+// The differentiable shader's inputs of a fan triangle of a task.
+__device__ __forceinline__ DiffInputs diffInputs(const TaskDev &task, int32_t fan) {
+	const FanRecord rec = task.fans[fan];
+	int32_t poly = rec.polygonFan >> 1, k = rec.polygonFan & 1;
+	const float *tc = task.texcoords + poly * 16;
+	const int32_t ca = 0, cb = (1 + k) * 4, cc = (2 + k) * 4;
+	DiffInputs d;
+	d.u = make3(tc[ca], tc[cb], tc[cc]);
+	d.v = make3(tc[ca + 1], tc[cb + 1], tc[cc + 1]);
+	d.point[0] = rec.corner[0];
+	d.point[1] = rec.corner[1];
+	d.point[2] = rec.corner[2];
+	return d;
+}
+
 // Writes draw command `index` with everything the raster needs of it -- the command, its row
 // setup and (for the RGBA8 shaders) its finished shader inputs -- and enters it into every tile
 // it can touch: the columns of cut(wholeBound, canvas), the rows of the aligned raster bound
@@ -138,6 +153,7 @@ __device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd
 	const TriangleRows tr = triangleRows(l2{cmd.fx[0], cmd.fy[0]}, l2{cmd.fx[1], cmd.fy[1]}, l2{cmd.fx[2], cmd.fy[2]}, canvasRect(cv));
 	f.triangleRows[index] = tr;
 	if (f.mode == 0) f.shaders[index] = si;
+	if (f.mode == 1) f.diffInputs[index] = diffInputs(f.tasks[cmd.task], cmd.fan);
 	int32_t tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;  // no tiles when the bound misses the canvas
 	if (tr.clipR > tr.clipL) {
 		// The columns and rows are at least 0 here, so shifts divide.
@@ -1052,39 +1068,21 @@ DH BilinearTaps bilinearTaps(int32_t log2w, int32_t log2h, float u, float v) {
 	return t;
 }
 
-// Inputs of the differentiable shader for one command's source triangle.
-struct DiffInputs {
-	f3 u, v;               // u1 and v1 at the three corners
-	int32_t point[3];      // model point of each corner (per-point multipliers)
-};
-
-__device__ __forceinline__ DiffInputs diffInputs(const TaskDev &task, int32_t fan) {
-	const FanRecord rec = task.fans[fan];
-	int32_t poly = rec.polygonFan >> 1, k = rec.polygonFan & 1;
-	const float *tc = task.texcoords + poly * 16;
-	const int32_t ca = 0, cb = (1 + k) * 4, cc = (2 + k) * 4;
-	DiffInputs d;
-	d.u = make3(tc[ca], tc[cb], tc[cc]);
-	d.v = make3(tc[ca + 1], tc[cb + 1], tc[cc + 1]);
-	d.point[0] = rec.corner[0];
-	d.point[1] = rec.corner[1];
-	d.point[2] = rec.corner[2];
-	return d;
-}
-
 __device__ __forceinline__ float multiplier(const FrameDev &f, int32_t point, int ch) {
 	return f.multipliers ? f.multipliers[point * 3 + ch] : 1.0f;
 }
 
-__device__ void drawCommandDiff(const FrameDev &f, const Command &cmd, int32_t commandIndex, const TaskDev &task,
-                                const QuadEval &e, QuadPixels<1> &q, bool depthRead, bool depthWrite) {
+// records: the adjoint record of the quad's upper left pixel, with recordStride records per row (null
+// when the frame keeps none).
+__device__ void drawCommandDiff(const FrameDev &f, const Command &cmd, int32_t c, int32_t commandIndex, DiffRecord *records,
+                                int32_t recordStride, const QuadEval &e, QuadPixels<1> &q, bool depthRead, bool depthWrite) {
 	const bool affine = (cmd.flags & 1) != 0;
 	bool vis[4];
 	if (!quadVisibility<1>(e, q, depthRead, affine, vis)) return;
-	const DiffInputs d = diffInputs(task, cmd.fan);
+	const DiffInputs d = f.diffInputs[c];
 	float m[3][3];
-	for (int c = 0; c < 3; c++)
-		for (int ch = 0; ch < 3; ch++) m[c][ch] = multiplier(f, d.point[c], ch);
+	for (int k = 0; k < 3; k++)
+		for (int ch = 0; ch < 3; ch++) m[k][ch] = multiplier(f, d.point[k], ch);
 	for (int l = 0; l < 4; l++) {
 		if (!vis[l]) continue;
 		float wa, wb, wc;
@@ -1105,6 +1103,7 @@ __device__ void drawCommandDiff(const FrameDev &f, const Command &cmd, int32_t c
 		put4(q.b, s, (wa * m[0][2] + wb * m[1][2] + wc * m[2][2]) * t[2]);
 		put4(q.a, s, t[3]);
 		put4(q.vis, s, commandIndex * 4 + l);
+		if (records) records[(s >> 1) * recordStride + (s & 1)] = DiffRecord{wb, wc, commandIndex * 4 + l, *f.forwardNumber};
 		q.colorDirty |= 1u << s;
 		if (depthWrite) {
 			put4(q.depth, s, e.l0[l]);
@@ -1234,16 +1233,20 @@ __device__ __forceinline__ void loadQuadColor(QuadPixels<0> &q, int s, bool in, 
 }
 __device__ __forceinline__ void loadQuadColor(QuadPixels<1> &, int, bool, const CanvasDev &, const FrameDev &, int32_t, int32_t) {}
 
-__device__ __forceinline__ void drawQuadCommand(const FrameDev &f, const Command &cmd, int32_t c, int32_t ci, const TaskDev &task,
-                                                const QuadEval &e, QuadPixels<0> &q, bool colorWrite, bool depthRead, bool depthWrite,
-                                                bool alphaFilter) {
+__device__ __forceinline__ void drawQuadCommand(const FrameDev &f, const Command &cmd, int32_t c, int32_t ci, const CanvasDev &cv,
+                                                int32_t px, int32_t py, const QuadEval &e, QuadPixels<0> &q, bool colorWrite,
+                                                bool depthRead, bool depthWrite, bool alphaFilter) {
 	(void)ci;
-	(void)task;
+	(void)cv;
+	(void)px;
+	(void)py;
 	drawCommand(f, cmd, c, e, q, colorWrite, depthRead, depthWrite, alphaFilter);
 }
-__device__ __forceinline__ void drawQuadCommand(const FrameDev &f, const Command &cmd, int32_t c, int32_t ci, const TaskDev &task,
-                                                const QuadEval &e, QuadPixels<1> &q, bool, bool depthRead, bool depthWrite, bool) {
-	drawCommandDiff(f, cmd, c - f.canvasCommandBase[ci], task, e, q, depthRead, depthWrite);
+__device__ __forceinline__ void drawQuadCommand(const FrameDev &f, const Command &cmd, int32_t c, int32_t ci, const CanvasDev &cv,
+                                                int32_t px, int32_t py, const QuadEval &e, QuadPixels<1> &q, bool, bool depthRead,
+                                                bool depthWrite, bool) {
+	DiffRecord *records = f.diffRecords ? f.diffRecords + cv.recordBase + (int64_t)py * cv.width + px : nullptr;
+	drawCommandDiff(f, cmd, c, c - f.canvasCommandBase[ci], records, cv.width, e, q, depthRead, depthWrite);
 }
 
 __device__ __forceinline__ void storeQuadColor(const QuadPixels<0> &q, int s, const CanvasDev &cv, int32_t x, int32_t y) {
@@ -1301,7 +1304,7 @@ __device__ void rasterTile(const FrameDev &f, int32_t tile, int32_t *list, RowIn
 			__syncthreads();
 			QuadEval e;
 			if (py >= alT && py < alB && evalQuad(cmd, rows[py - tileY0], rows[py + 1 - tileY0], px, py, cv.height, e)) {
-				drawQuadCommand(f, cmd, c, ci, task, e, q, colorWrite, depthRead, depthWrite, alphaFilter);
+				drawQuadCommand(f, cmd, c, ci, cv, px, py, e, q, colorWrite, depthRead, depthWrite, alphaFilter);
 			}
 		}
 		done += take;
@@ -1467,11 +1470,9 @@ static_assert(sizeof(TriangleRows) % 16 == 0 && sizeof(ShaderInputs) % 16 == 0 &
 
 // The differentiable shader (drawCommandDiff) for the lanes in mask of one command's quad at
 // (px, py), written straight to the float colour canvas with the visibility id base + lane.
-__device__ void shadeDiffLanes(const FrameDev &f, const CommandTail &ct, const QuadEval &e, uint32_t mask, uint32_t slots,
-                               int32_t idBase, const CanvasDev &cv, int32_t px, int32_t py) {
+__device__ void shadeDiffLanes(const FrameDev &f, const CommandTail &ct, const DiffInputs &d, const QuadEval &e, uint32_t mask,
+                               uint32_t slots, int32_t idBase, int32_t forward, const CanvasDev &cv, int32_t px, int32_t py) {
 	const bool affine = (ct.flags & 1) != 0;
-	const TaskDev &task = f.tasks[ct.task];
-	const DiffInputs d = diffInputs(task, ct.fan);
 	float m[3][3];
 	for (int c = 0; c < 3; c++)
 		for (int ch = 0; ch < 3; ch++) m[c][ch] = multiplier(f, d.point[c], ch);
@@ -1497,6 +1498,7 @@ __device__ void shadeDiffLanes(const FrameDev &f, const CommandTail &ct, const Q
 		                                                (wa * m[0][1] + wb * m[1][1] + wc * m[2][1]) * t[1],
 		                                                (wa * m[0][2] + wb * m[1][2] + wc * m[2][2]) * t[2], t[3]);
 		cv.visibility[p] = idBase + l;
+		if (f.diffRecords) f.diffRecords[cv.recordBase + (int64_t)y * cv.width + x] = DiffRecord{wb, wc, idBase + l, forward};
 	}
 }
 
@@ -1603,6 +1605,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 	const bool colorWrite = MODE == 0 && cv.color != nullptr;
 	const bool depthRead = cv.depth != nullptr;
 	const uint32_t flip = GENERAL && cv.affine ? ~0u : 0u;  // orthogonal canvases: the smaller depth wins
+	const int32_t forward = MODE == 1 && f.diffRecords ? *f.forwardNumber : 0;
 
 	for (int32_t p = t; p < NP; p += NT) {
 		if (f.clearInRaster) {
@@ -1860,7 +1863,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 						slots |= (uint32_t)sl << (2 * l);
 					}
 					const int32_t id = (s.list[c0 + j] - f.canvasCommandBase[ci]) * 4;
-					shadeDiffLanes(f, s.tail[j], e, mask, slots, id, cv, tileX0 + qx, tileY0 + qy);
+					shadeDiffLanes(f, s.tail[j], f.diffInputs[s.list[c0 + j]], e, mask, slots, id, forward, cv, tileX0 + qx, tileY0 + qy);
 				}
 			}
 			__syncthreads();
@@ -2107,25 +2110,35 @@ __device__ __forceinline__ void waveSync() {
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The adjoint of the differentiable forward with visibility fixed: each pixel re-derives the
-// interpolants of the (command, lane) that drew it -- the same rows and the same weight
-// stepping as the forward -- and scatters dL/dcolour into the four bilinear texels and the
-// three corners' RGB multipliers with float atomics.  Workgroups pull tiles from a queue
-// (all tiles of all views) until it is empty.  In tiles of 512 pixels and more a thread takes
-// two horizontally adjacent pixels of one quad: drawn by the same command they share the
-// quad's evaluation and one set of multiplier terms, and with the same four texels one set of
-// taps.  The multiplier
-// gradients of the pixels of one command are first added up in LDS (a small open-addressed
-// table of the tile's commands), so a tile makes one global atomic per (command, corner,
-// channel) instead of one per pixel; commands beyond the table's room add theirs directly.
-// Texture gradients are gathered the same way per texel (neighbouring pixels of a magnified
-// texture share their taps); taps that find no room are staged per wave in LDS and added with
+// The adjoint of the differentiable forward with visibility fixed: dL/dcolour of each drawn pixel goes
+// into the four bilinear texels and the three corners' RGB multipliers with float atomics, through the
+// weights of the (command, lane) that drew it.
+//
+// The forward leaves those weights in a record per drawn pixel.  Deriving them again -- two exact rows
+// and the weight chain per pixel pair, from 208 bytes of command gathered per lane -- was the larger
+// part of the kernel and kept it at three waves per SIMD.  A record counts only with the pixel's own
+// id and the number of the last forward; any other pixel (an id written by the caller, a canvas kept
+// from an earlier forward) raises a flag and is left to the DERIVE form, launched next, which ends at
+// once without the flag and otherwise derives the weights of those pixels as before.
+//
+// Workgroups pull bands of 32x32-pixel regions (all regions of all views, whatever the forward's tile
+// shape) from a queue until it is empty.  A thread takes two horizontally adjacent pixels: drawn by the
+// same command they share one set of multiplier terms, and with the same four texels one set of taps.
+// The multiplier gradients of the pixels of one command are first added up in LDS (a small
+// open-addressed table of the region's commands), so a region makes one global atomic per (command,
+// corner, channel) instead of one per pixel; commands beyond the table's room add theirs directly.
+// Texture gradients are gathered the same way per texel where neighbouring pixels share their taps (a
+// magnified texture); other taps, and those that find no room, are staged per wave in LDS and added with
 // one lane per channel, so that one atomic instruction covers the four channels of 16 texels
 // (L2 serves float atomics per cache line and request: four channels in one request instead
 // of four requests).
-constexpr int32_t BACKWARD_SLOTS = 64;
-constexpr int32_t TEXEL_SLOTS = 256;
-constexpr int32_t TEXEL_PROBES = 8;
+//
+// The tables add in 64 bits: an LDS float add (ds_add_f32) takes three cycles per active lane whatever
+// the addresses, 192 for a full wave, where the double add takes 8 to 32 as the addresses' banks allow.
+// Four of them per tap were 150 us of the 8-view fit's 460.
+constexpr int32_t BACKWARD_SLOTS = 128, BACKWARD_PROBES = 16;
+constexpr int32_t TEXEL_COLUMNS_LOG2 = 4, TEXEL_ROWS = 16, TEXEL_SLOTS = TEXEL_ROWS << TEXEL_COLUMNS_LOG2;
+constexpr int32_t POINT_SLOTS_LOG2 = 8, POINT_SLOTS = 1 << POINT_SLOTS_LOG2, POINT_PROBES = 16;
 
 // One pixel's share of the adjoint: its command (-1: none), the corners' points, its bilinear
 // taps, dL/dtexel per channel before the tap weights, and dL/dmultiplier per corner and channel.
@@ -2138,137 +2151,169 @@ struct AdjointTerms {
 	float mul[9];
 };
 
-// Three waves per SIMD (at most 168 VGPRs): the compiler's own choice of 189 registers left two,
-// and the third wave hides more of the adjoint's gather and atomic latency than the few values it
-// then keeps in scratch (and some private arrays it moves to LDS) cost.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_backward(FrameDev f, int32_t *head) {
-	__shared__ int32_t tileLds;
-	__shared__ int32_t slotCommand[BACKWARD_SLOTS];
-	__shared__ int32_t slotPoint[BACKWARD_SLOTS][3];
-	__shared__ float slotGrad[BACKWARD_SLOTS][9];
-	__shared__ int32_t texelKey[TEXEL_SLOTS];
-	__shared__ float4 texelGrad[TEXEL_SLOTS];
-	__shared__ int32_t stageTexel[256 * 4];
-	__shared__ float stageGrad[256 * 4 * 4];
-	const int32_t t = (int32_t)threadIdx.x;
+// The second and third corner's weights of lane `lane` of the command's quad over pixel (x, y), by the
+// forward's own rows and weight stepping; touches is 0 when the command does not touch the quad.
+struct DerivedWeights { float wb, wc; int32_t touches; };
+__device__ __forceinline__ DerivedWeights derivedWeights(const Command *commands, const TriangleRows *rows, int32_t c, int32_t lane,
+                                                         int32_t x, int32_t y, int32_t canvasHeight) {
+	const Command cmd = commands[c];
+	const int32_t py = y & ~1;
+	QuadEval e;
+	if (!evalQuad(cmd, triangleRow(rows[c], py), triangleRow(rows[c], py + 1), x & ~1, py, canvasHeight, e)) return DerivedWeights{0.0f, 0.0f, 0};
+	float wa[4], b[4], w[4];
+	for (int l = 0; l < 4; l++) laneWeights(e, l, (cmd.flags & 1) != 0, wa[l], b[l], w[l]);
+	return DerivedWeights{pick4(b, lane), pick4(w, lane), 1};
+}
 
-	// The taps of P (plus Q's, which then hit the same texels) into the tile's texel table, or
-	// staged and added one lane per channel.  Every lane of the wave calls it.
-	auto addTaps = [&](const AdjointTerms &P, const AdjointTerms &Q, bool any, bool withQ) {
-		for (int k = 0; k < 4; k++) stageTexel[t * 4 + k] = -1;
-		bool staged = false;
-		if (any)
-			for (int k = 0; k < 4; k++) {
-				if (P.weight[k] == 0.0f && !(withQ && Q.weight[k] != 0.0f)) continue;
-				float value[4];
-				for (int ch = 0; ch < 4; ch++) value[ch] = P.gt[ch] * P.weight[k] + (withQ ? Q.gt[ch] * Q.weight[k] : 0.0f);
-				const int32_t texel = (int32_t)P.texel[k];
-				int32_t slot = -1;
-				const int32_t h = (int32_t)(((uint32_t)texel * 2654435761u) >> 24);
-				for (int32_t q = 0; q < TEXEL_PROBES; q++) {
-					const int32_t i = (h + q) & (TEXEL_SLOTS - 1);
-					const int32_t old = atomicCAS(&texelKey[i], -1, texel);
-					if (old == -1 || old == texel) {
-						slot = i;
-						break;
-					}
-				}
-				if (slot >= 0) {
-					float *acc = (float *)&texelGrad[slot];
-					for (int ch = 0; ch < 4; ch++) atomicAdd(acc + ch, value[ch]);
-				} else {
-					stageTexel[t * 4 + k] = texel;
-					staged = true;
-					for (int ch = 0; ch < 4; ch++) stageGrad[(t * 4 + k) * 4 + ch] = value[ch];
-				}
-			}
-		if (__any(staged)) {
-			// The wave's 256 staged taps in 16 rounds of 16 taps x 4 channels; the stage is
-			// the wave's own, so a wave-scope barrier orders its writes and reads.
-			waveSync();
-			const int32_t lane = t & 63, ch = lane & 3, waveBase = (t & ~63) * 4;
-			for (int32_t r = 0; r < 16; r++) {
-				const int32_t e = waveBase + r * 16 + (lane >> 2);
-				const int32_t texel = stageTexel[e];
-				if (texel >= 0) unsafeAtomicAdd(f.gradTexture + (size_t)texel * 4 + ch, stageGrad[e * 4 + ch]);
-			}
+// heads: the queue heads of the two forms, then the flag.
+template <bool DERIVE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DERIVE ? 2 : 4, DERIVE ? 2 : 4))) k_backward(FrameDev f, int32_t *heads) {
+	if (DERIVE && f.diffRecords && heads[2] == 0) return;
+	__shared__ int32_t unitLds;
+	__shared__ int32_t slotCommand[BACKWARD_SLOTS];
+	__shared__ double slotGrad[9][BACKWARD_SLOTS];
+	__shared__ int32_t texelKey[TEXEL_SLOTS];
+	__shared__ double texelGrad[4][TEXEL_SLOTS];
+	__shared__ int32_t stageTexel[256 * 4];
+	__shared__ float4 stageGrad[256 * 4];
+	static_assert(POINT_SLOTS <= 256 * 4 && POINT_SLOTS * 3 * sizeof(double) <= sizeof(stageGrad), "the points' table fits the stage");
+	const int32_t t = (int32_t)threadIdx.x;
+	const int32_t forward = f.diffRecords ? *f.forwardNumber : 0;
+	bool unknown = false;  // a pixel of this thread is left to the DERIVE form
+
+	// One of the four taps of a pixel into the region's texel table; false when another texel has its place.
+	auto addToTable = [&](int32_t texel, const float4 &value) -> bool {
+		const int32_t i = (((texel >> f.ftexLog2w) & (TEXEL_ROWS - 1)) << TEXEL_COLUMNS_LOG2) | (texel & ((1 << TEXEL_COLUMNS_LOG2) - 1));
+		// Most taps find their texel there already: a plain read, which lanes with one address share.
+		if (((volatile int32_t *)texelKey)[i] != texel) {
+			const int32_t old = atomicCAS(&texelKey[i], -1, texel);
+			if (old != -1 && old != texel) return false;
 		}
-		waveSync();
+		unsafeAtomicAdd(&texelGrad[0][i], (double)value.x);
+		unsafeAtomicAdd(&texelGrad[1][i], (double)value.y);
+		unsafeAtomicAdd(&texelGrad[2][i], (double)value.z);
+		unsafeAtomicAdd(&texelGrad[3][i], (double)value.w);
+		return true;
+	};
+	// The taps of a thread's two pixels: the upper two of each, then the lower two.  same: both pixels
+	// hit the same texels, and the left one's taps carry the right one's share.  What the table does
+	// not take is staged in the order of the columns, so that one instruction adds the four channels
+	// of 16 taps of eight neighbouring pixels and one texel row: as few L2 requests as they have
+	// lines.  Every lane of the wave calls it.
+	auto addTaps = [&](const AdjointTerms &P, const AdjointTerms &Q, bool any, bool second, bool same, bool table) {
+		const int32_t lane = t & 63, ch = lane & 3, waveBase = (t & ~63) * 4;
+#pragma unroll
+		for (int row = 0; row < 2; row++) {
+			bool staged = false;
+#pragma unroll
+			for (int k = 0; k < 4; k++) {
+				const AdjointTerms &T = k < 2 ? P : Q;
+				const int tap = row * 2 + (k & 1);
+				const float other = k < 2 && same ? Q.weight[tap] : 0.0f;
+				bool due = (k < 2 ? any : second) && !(T.weight[tap] == 0.0f && other == 0.0f);
+				float4 value;
+				value.x = T.gt[0] * T.weight[tap] + (k < 2 && same ? Q.gt[0] * other : 0.0f);
+				value.y = T.gt[1] * T.weight[tap] + (k < 2 && same ? Q.gt[1] * other : 0.0f);
+				value.z = T.gt[2] * T.weight[tap] + (k < 2 && same ? Q.gt[2] * other : 0.0f);
+				value.w = T.gt[3] * T.weight[tap] + (k < 2 && same ? Q.gt[3] * other : 0.0f);
+				if (due && table && addToTable((int32_t)T.texel[tap], value)) due = false;
+				stageTexel[t * 4 + k] = due ? (int32_t)T.texel[tap] : -1;
+				if (due) stageGrad[t * 4 + k] = value;
+				staged = staged || due;
+			}
+			if (__any(staged)) {
+				// The stage is the wave's own, so a wave-scope barrier orders its writes and reads.
+				waveSync();
+#pragma unroll 4
+				for (int32_t r = 0; r < 16; r++) {
+					const int32_t e = waveBase + r * 16 + (lane >> 2);
+					const int32_t to = stageTexel[e];
+					if (to >= 0) unsafeAtomicAdd(f.gradTexture + (size_t)to * 4 + ch, ((const float *)stageGrad)[e * 4 + ch]);
+				}
+			}
+			waveSync();
+		}
 	};
 	auto addMultipliers = [&](const AdjointTerms &P) {
 		int32_t slot = -1;
-		const int32_t h = (int32_t)(((uint32_t)P.c * 2654435761u) >> 26);
-		for (int32_t k = 0; k < BACKWARD_SLOTS; k++) {
+		const int32_t h = (int32_t)(((uint32_t)P.c * 2654435761u) >> 25);
+		for (int32_t k = 0; k < BACKWARD_PROBES; k++) {
 			const int32_t i = (h + k) & (BACKWARD_SLOTS - 1);
-			const int32_t old = atomicCAS(&slotCommand[i], -1, P.c);
-			if (old == -1) {
-				for (int c3 = 0; c3 < 3; c3++) slotPoint[i][c3] = P.point[c3];
-				slot = i;
-				break;
-			}
-			if (old == P.c) {
+			int32_t old = ((volatile int32_t *)slotCommand)[i];
+			if (old == -1) old = atomicCAS(&slotCommand[i], -1, P.c);
+			if (old == -1 || old == P.c) {
 				slot = i;
 				break;
 			}
 		}
+#pragma unroll
 		for (int c3 = 0; c3 < 3; c3++)
+#pragma unroll
 			for (int ch = 0; ch < 3; ch++) {
-				if (slot >= 0) atomicAdd(&slotGrad[slot][c3 * 3 + ch], P.mul[c3 * 3 + ch]);
+				if (slot >= 0) unsafeAtomicAdd(&slotGrad[c3 * 3 + ch][slot], (double)P.mul[c3 * 3 + ch]);
 				else unsafeAtomicAdd(f.gradMultipliers + P.point[c3] * 3 + ch, P.mul[c3 * 3 + ch]);
 			}
 	};
 
+	const int32_t rows = ADJOINT_REGION / f.regionBands;
 	while (true) {
-		const int32_t t = opaqueThreadIndex();  // values derived from it are computed per tile
-		if (t == 0) tileLds = atomicAdd(head, 1);
-		if (t < BACKWARD_SLOTS) slotCommand[t] = -1;
-		for (int32_t i = t; i < BACKWARD_SLOTS * 9; i += 256) (&slotGrad[0][0])[i] = 0.0f;
-		for (int32_t i = t; i < TEXEL_SLOTS; i += 256) {
-			texelKey[i] = -1;
-			texelGrad[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-		}
+		if (t == 0) unitLds = atomicAdd(&heads[DERIVE ? 1 : 0], 1);
+		for (int32_t i = t; i < BACKWARD_SLOTS; i += 256) slotCommand[i] = -1;
+		for (int32_t i = t; i < BACKWARD_SLOTS * 9; i += 256) (&slotGrad[0][0])[i] = 0.0;
+		for (int32_t i = t; i < TEXEL_SLOTS; i += 256) texelKey[i] = -1;
+		for (int32_t i = t; i < TEXEL_SLOTS * 4; i += 256) (&texelGrad[0][0])[i] = 0.0;
 		__syncthreads();
-		const int32_t tile = tileLds;
-		if (tile >= f.tileTotal) break;
-		const int32_t ci = findSegment(f.canvasTileEnd, f.canvasCount, tile);
-		const CanvasDev cv = f.canvases[ci];
-		const int32_t local = tile - cv.tileBase;
-		// Pixel pairs (x even, x + 1) per thread and round, or single pixels in tiles of 256
-		// pixels (every thread busy): 256 or 512 items a tile, whole rounds for every wave.
-		const int32_t span = f.tileW * f.tileH >= 512 ? 2 : 1;
-		const int32_t across = f.tileW / span;
-		for (int32_t item = t; item < across * f.tileH; item += 256) {
-			const int32_t x = (local % cv.tilesX) * f.tileW + span * (item % across);
-			const int32_t y = (local / cv.tilesX) * f.tileH + item / across;
+		const int32_t unit = __builtin_amdgcn_readfirstlane(unitLds);
+		if (unit >= f.regionTotal * f.regionBands) break;
+		const int32_t region = unit / f.regionBands, band = unit % f.regionBands;
+		const int32_t ci = findSegment(f.canvasRegionEnd, f.canvasCount, region);
+		const CanvasDev &cv = f.canvases[ci];
+		const int32_t local = region - (ci > 0 ? f.canvasRegionEnd[ci - 1] : 0), across = adjointRegions(cv.width);
+		const int32_t x0 = (local % across) * ADJOINT_REGION, y0 = (local / across) * ADJOINT_REGION + band * rows;
+		const int32_t commandBase = f.canvasCommandBase[ci];
+		for (int32_t item = t; item < ADJOINT_REGION / 2 * rows; item += 256) {
+			const int32_t x = x0 + 2 * (item % (ADJOINT_REGION / 2)), y = y0 + item / (ADJOINT_REGION / 2);
 			AdjointTerms a[2];
-			a[0].c = -1;
-			a[1].c = -1;
-			QuadEval e;
-			int32_t evaluated = -1;  // the command whose quad e holds
+			float weightB[2], weightC[2];
 #pragma unroll
 			for (int i = 0; i < 2; i++) {
-				if (i >= span || x + i >= cv.width || y >= cv.height) continue;
-				const size_t p = (size_t)y * cv.diffStride + x + i;
-				const int32_t id = cv.visibility[p];
+				a[i].c = -1;
+				if (x + i >= cv.width || y >= cv.height) continue;
+				const int32_t id = cv.visibility[(size_t)y * cv.diffStride + x + i];
 				if (id < 0) continue;
-				const int32_t c = (id >> 2) + f.canvasCommandBase[ci], lane = id & 3;
-				const Command cmd = f.commands[c];
-				if (c != evaluated) {
-					evaluated = -1;
-					const TriangleRows &tr = f.triangleRows[c];
-					const int32_t py = y & ~1;
-					RowInterval upper = triangleRow(tr, py);
-					RowInterval lower = triangleRow(tr, py + 1);
-					if (!evalQuad(cmd, upper, lower, x & ~1, py, cv.height, e)) continue;
-					evaluated = c;
+				const int32_t c = (id >> 2) + commandBase;
+				bool known = false;
+				if (f.diffRecords) {
+					const DiffRecord rec = f.diffRecords[cv.recordBase + (int64_t)y * cv.width + x + i];
+					known = rec.id == id && rec.forward == forward;
+					weightB[i] = rec.wb;
+					weightC[i] = rec.wc;
 				}
-				const bool affine = (cmd.flags & 1) != 0;
-				float wa, wbw, wc;
-				laneWeights(e, lane, affine, wa, wbw, wc);
-				const DiffInputs d = diffInputs(f.tasks[cmd.task], cmd.fan);
+				if (!DERIVE) {
+					unknown = unknown || !known;
+					if (!known) continue;
+				} else {
+					if (known) continue;
+					const DerivedWeights derived = derivedWeights(f.commands, f.triangleRows, c, id & 3, x + i, y, cv.height);
+					if (!derived.touches) continue;
+					weightB[i] = derived.wb;
+					weightC[i] = derived.wc;
+				}
+				a[i].c = c;
+			}
+#pragma unroll
+			for (int i = 0; i < 2; i++) {
+				AdjointTerms &o = a[i];
+				const int32_t c = o.c;
+				if (c < 0) continue;
+				const size_t p = (size_t)y * cv.diffStride + x + i;
+				const float wbw = weightB[i], wc = weightC[i], wa = 1.0f - (wbw + wc);
+				const float4 g = *(const float4 *)(cv.gradColor + p * 4);
+				const DiffInputs d = f.diffInputs[c];
 				const float u = interp(d.u, wa, wbw, wc), v = interp(d.v, wa, wbw, wc);
 				const BilinearTaps taps = bilinearTaps(f.ftexLog2w, f.ftexLog2h, u, v);
 				float tx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
 				for (int k = 0; k < 4; k++) {
 					const float4 texel = *(const float4 *)(f.ftexTexels + (size_t)taps.index[k] * 4);
 					tx[0] += taps.weight[k] * texel.x;
@@ -2276,14 +2321,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
 					tx[2] += taps.weight[k] * texel.z;
 					tx[3] += taps.weight[k] * texel.w;
 				}
-				const float4 g = *(const float4 *)(cv.gradColor + p * 4);
 				const float w3[3] = {wa, wbw, wc};
 				float mixed[3];
+#pragma unroll
 				for (int ch = 0; ch < 3; ch++)
 					mixed[ch] = wa * multiplier(f, d.point[0], ch) + wbw * multiplier(f, d.point[1], ch) + wc * multiplier(f, d.point[2], ch);
-				AdjointTerms &o = a[i];
-				o.c = c;
+#pragma unroll
 				for (int c3 = 0; c3 < 3; c3++) o.point[c3] = d.point[c3];
+#pragma unroll
 				for (int k = 0; k < 4; k++) {
 					o.texel[k] = taps.index[k];
 					o.weight[k] = taps.weight[k];
@@ -2293,23 +2338,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
 				o.gt[2] = g.z * mixed[2];
 				o.gt[3] = g.w;
 				const float gm[3] = {g.x * tx[0], g.y * tx[1], g.z * tx[2]};
+#pragma unroll
 				for (int c3 = 0; c3 < 3; c3++)
+#pragma unroll
 					for (int ch = 0; ch < 3; ch++) o.mul[c3 * 3 + ch] = gm[ch] * w3[c3];
 			}
 			const bool v0 = a[0].c >= 0, v1 = a[1].c >= 0;
 			if (f.gradTexture) {
 				bool same = v0 && v1;
+#pragma unroll
 				for (int k = 0; k < 4; k++) same = same && a[0].texel[k] == a[1].texel[k];
-				// First the left pixel's taps (with the right one's when they hit the same
-				// texels) or the right pixel's alone, then the right pixel's when still due.
+				// The table pays where a pair's taps overlap: the right pixel starts at a texel of the
+				// left one's, as in most of the wave's pairs of a magnified texture.
+				const bool near = v0 && v1 && (a[1].texel[0] == a[0].texel[0] || a[1].texel[0] == a[0].texel[1] || a[1].texel[0] == a[0].texel[2] ||
+				                               a[1].texel[0] == a[0].texel[3] || a[0].texel[0] == a[1].texel[1] || a[0].texel[0] == a[1].texel[2]);
+				const bool table = 2 * __popcll(__ballot(near)) >= __popcll(__ballot(v0 && v1));
 				AdjointTerms first = a[1];
 				if (v0) first = a[0];
-				addTaps(first, a[1], v0 || v1, same);
-				const bool second = v0 && v1 && !same;
-				if (__any(second)) addTaps(a[1], a[1], second, false);
+				addTaps(first, a[1], v0 || v1, v0 && v1 && !same, same, table);
 			}
 			if (f.gradMultipliers) {
 				if (v0 && v1 && a[0].c == a[1].c) {
+#pragma unroll
 					for (int m = 0; m < 9; m++) a[0].mul[m] += a[1].mul[m];
 					addMultipliers(a[0]);
 				} else {
@@ -2322,16 +2372,48 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
 		if (f.gradTexture)
 			for (int32_t i = t; i < TEXEL_SLOTS * 4; i += 256) {
 				const int32_t texel = texelKey[i >> 2];
-				if (texel >= 0) unsafeAtomicAdd(f.gradTexture + (size_t)texel * 4 + (i & 3), (&texelGrad[i >> 2].x)[i & 3]);
+				if (texel >= 0) unsafeAtomicAdd(f.gradTexture + (size_t)texel * 4 + (i & 3), (float)texelGrad[i & 3][i >> 2]);
 			}
-		if (f.gradMultipliers)
-			for (int32_t i = t; i < BACKWARD_SLOTS * 9; i += 256) {
-				const int32_t slot = i / 9, m = i % 9;
-				if (slotCommand[slot] >= 0) unsafeAtomicAdd(f.gradMultipliers + slotPoint[slot][m / 3] * 3 + m % 3, slotGrad[slot][m]);
+		if (f.gradMultipliers) {
+			// The points' table lies in the stage, which no wave uses before the next region.
+			int32_t *pointKey = stageTexel;
+			double *pointGrad = (double *)stageGrad;
+			for (int32_t i = t; i < POINT_SLOTS; i += 256) pointKey[i] = -1;
+			for (int32_t i = t; i < POINT_SLOTS * 3; i += 256) pointGrad[i] = 0.0;
+			__syncthreads();
+			for (int32_t i = t; i < BACKWARD_SLOTS * 3; i += 256) {
+				const int32_t slot = i / 3, corner = i % 3;
+				if (slotCommand[slot] < 0) continue;
+				const int32_t point = f.diffInputs[slotCommand[slot]].point[corner];
+				const int32_t h = (int32_t)(((uint32_t)point * 2654435761u) >> (32 - POINT_SLOTS_LOG2));
+				int32_t at = -1;
+				for (int32_t q = 0; q < POINT_PROBES; q++) {
+					const int32_t k = (h + q) & (POINT_SLOTS - 1);
+					const int32_t old = atomicCAS(&pointKey[k], -1, point);
+					if (old == -1 || old == point) {
+						at = k;
+						break;
+					}
+				}
+				for (int ch = 0; ch < 3; ch++) {
+					const double grad = slotGrad[corner * 3 + ch][slot];
+					if (at >= 0) unsafeAtomicAdd(&pointGrad[at * 3 + ch], grad);
+					else unsafeAtomicAdd(f.gradMultipliers + point * 3 + ch, (float)grad);
+				}
 			}
+			__syncthreads();
+			for (int32_t i = t; i < POINT_SLOTS * 3; i += 256) {
+				const int32_t point = pointKey[i / 3];
+				if (point >= 0) unsafeAtomicAdd(f.gradMultipliers + point * 3 + i % 3, (float)pointGrad[i]);
+			}
+		}
 		__syncthreads();
 	}
+	if (!DERIVE && unknown) atomicOr(&heads[2], 1);
 }
+
+template __global__ void k_backward<false>(FrameDev, int32_t *);
+template __global__ void k_backward<true>(FrameDev, int32_t *);
 
 // The start of a frame: zeroed counters, tile counts and fill cursors, unset canvas command
 // bases, and the projection of every model point (modelAPI.cpp:237-242), in one launch.
@@ -2340,6 +2422,7 @@ __global__ void k_frame_begin(FrameDev f) {
 	if (i < COUNTERS) f.counters[i] = 0;
 	if (i < 2 * f.tileTotal + 1) f.tileCount[i] = 0;
 	if (i < f.canvasCount) f.canvasCommandBase[i] = 0x7FFFFFFF;
+	if (i == 0 && f.forwardNumber) f.forwardNumber[0]++;
 }
 
 // renderer_occludeFromExistingTriangles (rendererAPI.cpp:241-258): the Solid draw commands of

@@ -59,6 +59,7 @@ struct CanvasDev {
 	int32_t *visibility;
 	const float *gradColor;
 	int32_t diffStride;
+	int64_t recordBase;                // differentiable frames: the canvas's first adjoint record
 	int32_t fans;                      // fan triangles of its tasks
 	int32_t dense;                     // fewer than DENSE_PIXELS_PER_FAN pixels per fan triangle
 	int32_t affine;                    // its tasks' cameras are orthogonal (the smaller depth wins)
@@ -75,6 +76,22 @@ struct __attribute__((aligned(16))) Command {
 	f3 start, dx, dy;      // weight planes
 	int32_t task, fan;     // source: task and fan triangle within the task's model
 	int32_t canvas, flags; // canvas slot; bit 0 = affine (orthogonal camera)
+};
+
+// What the differentiable shader and its adjoint need of a draw command's source triangle, written by
+// the setup: u1, v1 and the model point of each corner.
+struct __attribute__((aligned(16))) DiffInputs {
+	f3 u, v;
+	int32_t point[3];
+	int32_t pad[3];
+};
+
+// What a differentiable forward leaves for the adjoint at a pixel it draws: the second and third
+// corner's weights of the winning lane, its visibility id, and the number of the forward.
+struct __attribute__((aligned(16))) DiffRecord {
+	float wb, wc;
+	int32_t id;
+	int32_t forward;
 };
 
 // A (tile, command) pair of the packed lists: the command's slot in the tile's list, from the
@@ -100,9 +117,10 @@ struct FrameDev {
 	TriangleRows *triangleRows;   // per command: edges and bounds of its rows
 	int32_t commandCapacity;
 	int32_t *counters;            // [0] commands, [1] pairs, [2] overflow flags, [3] tiles with commands,
-	                              // [5] backward head, [6] longest tile list when a bin overflowed,
+	                              // [6] longest tile list when a bin overflowed,
 	                              // [7] pair records, [8] most commands of one setup block when a
-	                              // single-pass block overflowed, [QUEUE_HEADS + 32 x] XCD x's raster head
+	                              // single-pass block overflowed, [9..11] the adjoint's queue heads
+	                              // and flag, [QUEUE_HEADS + 32 x] XCD x's raster head
 	int32_t blockCapacity;        // single-pass setup: command slots per setup block (0: two passes)
 	int32_t selfClean;            // the raster leaves zeroed counts for the next frame (resetNextCounters)
 	int32_t *nextCounters;        // selfClean: the counter set of the next frame
@@ -138,12 +156,21 @@ struct FrameDev {
 	const float *multipliers;
 	float *gradTexture;
 	float *gradMultipliers;
+	DiffInputs *diffInputs;           // per command
+	DiffRecord *diffRecords;          // width x height per canvas from its recordBase on, or null
+	int32_t *forwardNumber;           // grows by one with every forward (k_frame_begin)
+	// The adjoint's work: regions of ADJOINT_REGION^2 pixels, each cut into regionBands bands of rows.
+	const int32_t *canvasRegionEnd;   // inclusive prefix of regions per canvas
+	int32_t regionTotal, regionBands;
 	// Occlusion grid of a renderer frame (one canvas), gridW x gridH cells of 16 x 16 pixels;
 	// null when the frame has no occluders.  The setup drops each command it covers
 	// (completeOcclusion); k_occlude_existing lowers it.
 	float *occlusionGrid;
 	int32_t gridW, gridH;
 };
+
+constexpr int32_t ADJOINT_REGION = 32;
+DH int32_t adjointRegions(int32_t pixels) { return (pixels + ADJOINT_REGION - 1) / ADJOINT_REGION; }
 
 // First entry of tile t's command list.
 DH const int32_t *tileListOf(const FrameDev &f, int32_t tile) {
@@ -179,7 +206,7 @@ template <int TW, int TH> __global__ void k_raster_diff(FrameDev f, int32_t pers
 template <int TW, int TH, int P, bool GENERAL> __global__ void k_raster_deferred_diff(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_depth(FrameDev f);
 __global__ void k_probe_edge_side(const int64_t *n, const int64_t *d, const int32_t *L, const int32_t *R, int32_t count, int32_t *out);
-__global__ void k_backward(FrameDev f, int32_t *head);
+template <bool DERIVE> __global__ void k_backward(FrameDev f, int32_t *heads);
 __global__ void k_fill(int32_t *p, int32_t n, int32_t value);
 __global__ void k_clear_canvases(FrameDev f, uint32_t color, float depth);
 __global__ void k_downsample(uint32_t *texels, TextureDesc t, uint32_t targetLevel);

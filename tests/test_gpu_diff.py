@@ -135,6 +135,59 @@ def test_forward_on_odd_heights_equals_in_order_raster(api):
                 assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"run {k} view {i}"
 
 
+def test_adjoint_of_kept_and_changed_visibility(api):
+    """The adjoint takes a pixel's weights from the forward's record only where the pixel still shows what
+    that forward drew there, and derives them again otherwise.  Masked pixels are left out; two pixels of
+    one quad that trade their ids and gradients, and canvases kept from an earlier forward (not cleared,
+    so that the second forward draws nothing), give the gradients they gave before.  Sums of some 10^4
+    single-precision terms in any order differ by about 1e-6 of their norm; the bound is 2e-5."""
+    views = small_views()
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    gv = api.GpuViews(views)
+    for i, g in enumerate(gv.grad):
+        g.copy_(torch.from_numpy(S.Rng(100 + i).uniform(g.numel(), -1.0, 1.0).reshape(tuple(g.shape))))
+    r = api.DiffRenderer()
+
+    def adjoint():
+        gt, gm = torch.zeros_like(tex), torch.zeros((gv.point_count, 3), device="cuda")
+        r.backward(gt, gm)
+        torch.cuda.synchronize()
+        return gt.cpu().double(), gm.cpu().double()
+
+    def assert_close(got, want, what):
+        for a, b in zip(got, want):
+            assert float((a - b).norm()) <= 2e-5 * float(b.norm()), what
+
+    for path in (0, 1):
+        r.forward(gv.model, gv.views, tex, None, api.tuning(clear=True, raster_path=path))
+        base = adjoint()
+        vis, grad = [v.clone() for v in gv.visibility], [g.clone() for g in gv.grad]
+        swapped = 0
+        for v, g in zip(gv.visibility, gv.grad):  # columns 2k and 2k + 1 of one command
+            left, right = v[:, 0::2].clone(), v[:, 1::2].clone()
+            trade = (left >= 0) & (right >= 0) & ((left >> 2) == (right >> 2))
+            v[:, 0::2], v[:, 1::2] = torch.where(trade, right, left), torch.where(trade, left, right)
+            gl, gr = g[:, 0::2].clone(), g[:, 1::2].clone()
+            g[:, 0::2], g[:, 1::2] = torch.where(trade[..., None], gr, gl), torch.where(trade[..., None], gl, gr)
+            swapped += int(trade.sum())
+        assert swapped > 1000
+        assert_close(adjoint(), base, "traded ids")
+        for i, v in enumerate(gv.visibility):
+            v.copy_(vis[i])
+            gv.grad[i].copy_(grad[i])
+            v[::3, ::2] = -1
+        masked = adjoint()
+        for i, v in enumerate(gv.visibility):
+            v.copy_(vis[i])
+            gv.grad[i][::3, ::2] = 0.0
+        assert_close(masked, adjoint(), "masked pixels")
+        for i, g in enumerate(gv.grad):
+            g.copy_(grad[i])
+        r.forward(gv.model, gv.views, tex, None, api.tuning(raster_path=path))
+        assert all(torch.equal(a, b) for a, b in zip(vis, gv.visibility))
+        assert_close(adjoint(), base, "kept canvases")
+
+
 def test_adjoint_same_for_every_tile_shape(api):
     """The adjoint walks whatever tiles the forward used: texture and multiplier gradients agree
     across tile shapes up to the order of the float atomics."""
