@@ -147,10 +147,10 @@ __device__ __forceinline__ DiffInputs diffInputs(const TaskDev &task, int32_t fa
 // any order: the raster sorts each list); otherwise the tile's count grows here and a pair
 // record (tile, slot, command) keeps the slot until the counts are scanned and the list is
 // filled from the records.
-__device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd, const CanvasDev &cv,
+__device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd, const Projected *P, const CanvasDev &cv,
                             const ShaderInputs &si, BinTally &tally, BinJob *jobs, int32_t jobBase) {
 	f.commands[index] = cmd;
-	const TriangleRows tr = triangleRows(l2{cmd.fx[0], cmd.fy[0]}, l2{cmd.fx[1], cmd.fy[1]}, l2{cmd.fx[2], cmd.fy[2]}, canvasRect(cv));
+	const TriangleRows tr = triangleRows(P[0].flat, P[1].flat, P[2].flat, canvasRect(cv));
 	f.triangleRows[index] = tr;
 	if (f.mode == 0) f.shaders[index] = si;
 	if (f.mode == 1) f.diffInputs[index] = diffInputs(f.tasks[cmd.task], cmd.fan);
@@ -313,11 +313,9 @@ __device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, i
 			if (EMIT) {
 				Command c;
 				const f2 is[3] = {P[0].is, P[1].is, P[2].is};
-				Projection pr = weightPlanes(is, make3(P[0].cs.z, P[1].cs.z, P[2].cs.z), make3(0.0f, 1.0f, 0.0f), make3(0.0f, 0.0f, 1.0f), perspective);
-				for (int q = 0; q < 3; q++) { c.fx[q] = P[q].flat.x; c.fy[q] = P[q].flat.y; }
-				c.start = pr.start; c.dx = pr.dx; c.dy = pr.dy;
-				c.task = ti; c.fan = local; c.canvas = t.canvas; c.flags = perspective ? 0 : 1;
-				emitCommand(f, offset, c, cv, si, tally, jobs, jobBase);
+				c.plane = weightPlanes(is, make3(P[0].cs.z, P[1].cs.z, P[2].cs.z), make3(0.0f, 1.0f, 0.0f), make3(0.0f, 0.0f, 1.0f), perspective);
+				c.task = ti; c.fan = local; c.flags = perspective ? 0 : 1;
+				emitCommand(f, offset, c, P, cv, si, tally, jobs, jobBase);
 			}
 			count = 1;
 		}
@@ -342,12 +340,10 @@ __device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, i
 				if (EMIT) {
 					Command c;
 					const f2 is[3] = {S[0].is, S[1].is, S[2].is};
-					Projection pr = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), make3(va.subB, vb.subB, vc.subB),
-					                             make3(va.subC, vb.subC, vc.subC), perspective);
-					for (int q = 0; q < 3; q++) { c.fx[q] = S[q].flat.x; c.fy[q] = S[q].flat.y; }
-					c.start = pr.start; c.dx = pr.dx; c.dy = pr.dy;
-					c.task = ti; c.fan = local; c.canvas = t.canvas; c.flags = perspective ? 0 : 1;
-					emitCommand(f, offset + count, c, cv, si, tally, jobs, jobBase);
+					c.plane = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), make3(va.subB, vb.subB, vc.subB),
+					                       make3(va.subC, vb.subC, vc.subC), perspective);
+					c.task = ti; c.fan = local; c.flags = perspective ? 0 : 1;
+					emitCommand(f, offset + count, c, S, cv, si, tally, jobs, jobBase);
 				}
 				count++;
 			}
@@ -908,7 +904,7 @@ __device__ __forceinline__ bool evalQuad(const Projection &cmd, RowInterval uppe
 
 __device__ __forceinline__ bool evalQuad(const Command &cmd, RowInterval upper, RowInterval lower, int32_t px, int32_t py,
                                          int32_t canvasHeight, QuadEval &e) {
-	return evalQuad(Projection{cmd.start, cmd.dx, cmd.dy}, upper, lower, px, py, canvasHeight, e);
+	return evalQuad(cmd.plane, upper, lower, px, py, canvasHeight, e);
 }
 
 // The integer part of evalQuad: whether the command touches the quad at (px, py) and, per lane,
@@ -1456,21 +1452,12 @@ template <int TW, int TH, int CH> struct DeferShape {
 
 constexpr int32_t LDS_TEXTURES = 16;  // texture tables up to this size are read from LDS
 
-// The bytes of a draw command from its weight planes to its end (Command::start ..).
-struct __attribute__((aligned(16))) CommandTail {
-	Projection plane;
-	int32_t task, fan, canvas, flags;
-	int32_t pad[3];
-};
-constexpr int32_t COMMAND_TAIL_OFFSET = 48;  // bytes of Command before start
-static_assert(offsetof(Command, start) == COMMAND_TAIL_OFFSET && offsetof(Command, flags) == COMMAND_TAIL_OFFSET + 48 &&
-              sizeof(CommandTail) == sizeof(Command) - COMMAND_TAIL_OFFSET, "CommandTail mirrors the tail of Command");
-static_assert(sizeof(TriangleRows) % 16 == 0 && sizeof(ShaderInputs) % 16 == 0 && sizeof(CommandTail) % 16 == 0,
+static_assert(sizeof(TriangleRows) % 16 == 0 && sizeof(ShaderInputs) % 16 == 0 && sizeof(Command) % 16 == 0,
               "staged records are whole 16-byte units");
 
 // The differentiable shader (drawCommandDiff) for the lanes in mask of one command's quad at
 // (px, py), written straight to the float colour canvas with the visibility id base + lane.
-__device__ void shadeDiffLanes(const FrameDev &f, const CommandTail &ct, const DiffInputs &d, const QuadEval &e, uint32_t mask,
+__device__ void shadeDiffLanes(const FrameDev &f, const Command &ct, const DiffInputs &d, const QuadEval &e, uint32_t mask,
                                uint32_t slots, int32_t idBase, int32_t forward, const CanvasDev &cv, int32_t px, int32_t py) {
 	const bool affine = (ct.flags & 1) != 0;
 	float m[3][3];
@@ -1518,7 +1505,7 @@ template <int TW, int TH, int CH, int MODE> struct DeferLds {
 		unsigned long long keys[TW * TH];        // then the pixels' (depth, command) keys
 	};
 	ShaderInputs si[RGBA ? S::CHUNK : 1];        // shader inputs,
-	CommandTail tail[S::CHUNK];                  // weight planes and flags
+	Command command[S::CHUNK];                  // weight planes and flags
 	RowSpan rows[S::CHUNK * TH];                 // chunk command j, tile row r
 	union {
 		struct {                                 // during the rows:
@@ -1541,13 +1528,11 @@ template <int TW, int TH, int CH, int MODE> struct DeferLds {
 	int32_t slot;
 };
 
-// Copies the 16-byte units [offset, offset + sizeof(T)) of element list[c0 + j] of a global
-// array with `stride` bytes per element into dst[j], for every chunk command j, with loads that
-// write LDS directly (no registers hold the data).  Each wave instruction fills 64
-// consecutive units of dst.  The caller waits for them (stageWait) before reading dst.
+// Copies element list[c0 + j] of a global array of T into dst[j], for every chunk command j, with loads
+// that write LDS directly (no registers hold the data), 16 bytes per lane.  Each wave instruction fills
+// 64 consecutive units of dst.  The caller waits for them (stageWait) before reading dst.
 template <int NT, typename T>
-__device__ __forceinline__ void stageToLds(T *dst, const uint8_t *src, int32_t stride, int32_t offset,
-                                           const int32_t *list, int32_t c0, int32_t cn) {
+__device__ __forceinline__ void stageToLds(T *dst, const uint8_t *src, const int32_t *list, int32_t c0, int32_t cn) {
 	constexpr int32_t UNITS = (int32_t)(sizeof(T) / 16);
 	const int32_t total = cn * UNITS;
 	const int32_t lane = (int32_t)(threadIdx.x & 63);
@@ -1555,7 +1540,7 @@ __device__ __forceinline__ void stageToLds(T *dst, const uint8_t *src, int32_t s
 		const int32_t q = base + lane;
 		if (q < total) {
 			const int32_t j = q / UNITS, u = q % UNITS;
-			const uint8_t *g = src + (size_t)list[c0 + j] * stride + offset + u * 16;
+			const uint8_t *g = src + (size_t)list[c0 + j] * sizeof(T) + u * 16;
 			__builtin_amdgcn_global_load_lds((const void *)g, (void *)((uint8_t *)dst + (size_t)base * 16), 16, 0, 0);
 		}
 	}
@@ -1631,9 +1616,9 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 			const int32_t t = opaqueThreadIndex();
 			const int32_t cn = take - c0 < CHUNK ? take - c0 : CHUNK;
 			// The chunk's row setups, shader inputs and weight planes into LDS.
-			stageToLds<NT>(s.tr, (const uint8_t *)f.triangleRows, (int32_t)sizeof(TriangleRows), 0, s.list, c0, cn);
-			if (colorWrite) stageToLds<NT>(s.si, (const uint8_t *)f.shaders, (int32_t)sizeof(ShaderInputs), 0, s.list, c0, cn);
-			stageToLds<NT>(s.tail, (const uint8_t *)f.commands, (int32_t)sizeof(Command), COMMAND_TAIL_OFFSET, s.list, c0, cn);
+			stageToLds<NT>(s.tr, (const uint8_t *)f.triangleRows, s.list, c0, cn);
+			if (colorWrite) stageToLds<NT>(s.si, (const uint8_t *)f.shaders, s.list, c0, cn);
+			stageToLds<NT>(s.command, (const uint8_t *)f.commands, s.list, c0, cn);
 			stageWait();
 			__syncthreads();
 			// Rows of every chunk command in the tile: empty outside the command's aligned bound,
@@ -1714,7 +1699,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				const int32_t py = tileY0 + 2 * rp;
 				if (GENERAL && py + 1 >= cv.height) continue;  // walked below
 				QuadEval e;
-				const bool ok = evalQuad(s.tail[j].plane, rowInterval(s.rows[j * TH + 2 * rp]), rowInterval(s.rows[j * TH + 2 * rp + 1]),
+				const bool ok = evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + 2 * rp]), rowInterval(s.rows[j * TH + 2 * rp + 1]),
 				                         px, py, cv.height, e);
 				if (!ok) continue;
 				for (int l = 0; l < 4; l++) {
@@ -1740,7 +1725,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 					const RowSpan upperRow = s.rows[j * TH + py - tileY0];
 					if (upperRow.right <= upperRow.left) continue;
 					QuadEval e;
-					if (!evalQuad(s.tail[j].plane, rowInterval(upperRow), rowInterval(s.rows[j * TH + py - tileY0 + 1]), px, py, cv.height, e)) continue;
+					if (!evalQuad(s.command[j].plane, rowInterval(upperRow), rowInterval(s.rows[j * TH + py - tileY0 + 1]), px, py, cv.height, e)) continue;
 #pragma unroll
 					for (int i = 0; i < 2; i++) {
 						const float old = held[i];
@@ -1796,7 +1781,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 					const int32_t j = pr / RP, rp = pr % RP;
 					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
 					QuadEval e;
-					if (!evalQuad(s.tail[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
+					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
 					              tileY0 + qy, cv.height, e))
 						continue;
 					int32_t pixel[4];
@@ -1808,7 +1793,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 						if (!fillAll) atomicOr(&s.dirty[pixel[l] >> 5], 1u << (pixel[l] & 31));
 					}
 					if (colorWrite) {
-						const bool affine = (s.tail[j].flags & 1) != 0;
+						const bool affine = (s.command[j].flags & 1) != 0;
 						float wa[4], wb[4], wc[4];
 						for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
 						const uint32_t mip = quadMip(s.si[j], textures, wa, wb, wc);
@@ -1840,7 +1825,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 					const int32_t j = pr / RP, rp = pr % RP;
 					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
 					QuadEval e;
-					if (!evalQuad(s.tail[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
+					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
 					              tileY0 + qy, cv.height, e))
 						continue;
 					uint32_t mask = 0;
@@ -1863,7 +1848,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 						slots |= (uint32_t)sl << (2 * l);
 					}
 					const int32_t id = (s.list[c0 + j] - f.canvasCommandBase[ci]) * 4;
-					shadeDiffLanes(f, s.tail[j], f.diffInputs[s.list[c0 + j]], e, mask, slots, id, forward, cv, tileX0 + qx, tileY0 + qy);
+					shadeDiffLanes(f, s.command[j], f.diffInputs[s.list[c0 + j]], e, mask, slots, id, forward, cv, tileX0 + qx, tileY0 + qy);
 				}
 			}
 			__syncthreads();
@@ -1993,7 +1978,7 @@ template <int TW, int TH> struct DepthLds {
 	int32_t list[LIST];
 	unsigned long long keys[TW * TH];
 	TriangleRows tr[CHUNK];
-	CommandTail tail[CHUNK];
+	Command command[CHUNK];
 	int32_t rowFirst[CHUNK];
 	int32_t rowStart[CHUNK + 1];
 	int32_t roundInfo[4];
@@ -2027,8 +2012,8 @@ __device__ void depthTile(const FrameDev &f, int32_t tile, DepthLds<TW, TH> &s) 
 		const int32_t take = nextRound<NT, S::LIST>(src, n, done, last, s.list, s.roundInfo, (int32_t *)s.tr);
 		for (int32_t c0 = 0; c0 < take; c0 += CHUNK) {
 			const int32_t cn = take - c0 < CHUNK ? take - c0 : CHUNK;
-			stageToLds<NT>(s.tr, (const uint8_t *)f.triangleRows, (int32_t)sizeof(TriangleRows), 0, s.list, c0, cn);
-			stageToLds<NT>(s.tail, (const uint8_t *)f.commands, (int32_t)sizeof(Command), COMMAND_TAIL_OFFSET, s.list, c0, cn);
+			stageToLds<NT>(s.tr, (const uint8_t *)f.triangleRows, s.list, c0, cn);
+			stageToLds<NT>(s.command, (const uint8_t *)f.commands, s.list, c0, cn);
 			stageWait();
 			__syncthreads();
 			// Each command's rows inside the tile and inside the canvas, and their prefix.
@@ -2059,7 +2044,7 @@ __device__ void depthTile(const FrameDev &f, int32_t tile, DepthLds<TW, TH> &s) 
 				const RowInterval row = triangleRow(s.tr[j], y);
 				const int32_t x1 = tmin(row.right, tileX0 + TW);
 				if (row.left >= x1 || row.right <= tileX0) continue;
-				const Projection &pl = s.tail[j].plane;
+				const Projection &pl = s.command[j].plane;
 				const float dx = pl.dx.x;
 				float value = weightAtPixel(pl, row.left, y).x;
 				int32_t x = row.left;

@@ -70,13 +70,15 @@ struct CanvasDev {
 // gains nothing, 256x256 views of 20 480 triangles have 3.2 and gain a third of their time.
 constexpr int32_t DENSE_PIXELS_PER_FAN = 8;
 
-// One draw command: a (sub-)triangle that passed culling, clipping and the front-face test.
+// One draw command, a (sub-)triangle that passed culling, clipping and the front-face test, as the
+// rasters read it: 48 bytes, three 16-byte units (its corners are only needed by the setup, which
+// reduces them to TriangleRows; with them it was 112 bytes).
 struct __attribute__((aligned(16))) Command {
-	int64_t fx[3], fy[3];  // corners in sub-pixels (256 per pixel)
-	f3 start, dx, dy;      // weight planes
+	Projection plane;      // weight planes
 	int32_t task, fan;     // source: task and fan triangle within the task's model
-	int32_t canvas, flags; // canvas slot; bit 0 = affine (orthogonal camera)
+	int32_t flags;         // bit 0 = affine (orthogonal camera)
 };
+static_assert(sizeof(Command) == 48, "three 16-byte units");
 
 // What the differentiable shader and its adjoint need of a draw command's source triangle, written by
 // the setup: u1, v1 and the model point of each corner.
