@@ -443,23 +443,50 @@ DH int64_t divTrunc64(int64_t n, int64_t d) {
 
 DH bool sameCorner(const l2 &a, const l2 &b) { return a.x == b.x && a.y == b.y; }
 
-// An edge as the rows read it: a left or right edge (kind 1, 2) keeps a = offsetX,
-// b = offsetY, c = limitTop; a horizontal edge (kind 3) keeps a = threshold, b = offsetY,
-// c = valueTop; an edge without effect (kind 0) keeps nothing.
-struct EdgeRows { int64_t a, b, c; };
+// An edge as the rows read it.  Row r of the aligned bound cuts a left or right edge (kind 1, 2) at
+// trunc(m / a) + 1 with m = c - b * r and a > 0 (a left edge's signs are turned round); a horizontal
+// edge (kind 3) empties the rows with m < 0; an edge without effect (kind 0) keeps nothing.
+//
+// c and b are whole numbers held in double: below 2^52 the fused c - b * r and the remainder of an
+// estimated quotient are exact, at the rate of single precision on this chip, where 64-bit integer
+// products and compares take several instructions each.  a is exact in float (256 times less than
+// 2^24), inverse is 1 / a.  Triangles with larger terms keep the integers (wide) and take wideRow.
+struct EdgeRows {
+	union {
+		struct { double c, b; float a, inverse; } exact;
+		struct { int64_t a, b, c; } wide;  // kind 1, 2: offsetX, offsetY, limitTop; 3: threshold, offsetY, valueTop
+	};
+};
 
-DH EdgeRows edgeRows(const EdgeSetup &st) {
+// Whether the edge's terms fit the double form over the bound's rows and columns.  Quotients of 2^30
+// and more stay with the integers, which wrap them to int32 as the reference does.
+DH bool edgeFitsDouble(const EdgeSetup &st, int32_t rows) {
+	const double a = fabs((double)st.offsetX), b = fabs((double)st.offsetY) * rows, c = fabs((double)(st.kind == 3 ? st.valueTop : st.limitTop));
+	if (st.kind == 0) return true;
+	if (!(b < 2251799813685248.0 && c < 2251799813685248.0 && a < 4294967296.0)) return false;  // 2^51, 2^32
+	return st.kind == 3 || b + c < 1073741824.0 * a;  // 2^30
+}
+
+DH EdgeRows edgeRows(const EdgeSetup &st, bool wide) {
 	EdgeRows e;
-	e.a = st.kind == 3 ? st.threshold : st.offsetX;
-	e.b = st.offsetY;
-	e.c = st.kind == 3 ? st.valueTop : st.limitTop;
+	if (wide) {
+		e.wide.a = st.kind == 3 ? st.threshold : st.offsetX;
+		e.wide.b = st.offsetY;
+		e.wide.c = st.kind == 3 ? st.valueTop : st.limitTop;
+		return e;
+	}
+	const bool leftEdge = st.kind == 1;
+	e.exact.c = (double)(st.kind == 3 ? st.threshold - st.valueTop : (leftEdge ? -(st.limitTop + 1) : st.limitTop));
+	e.exact.b = (double)(leftEdge ? -st.offsetY : st.offsetY);
+	e.exact.a = st.kind == 1 || st.kind == 2 ? (float)(leftEdge ? -st.offsetX : st.offsetX) : 1.0f;
+	e.exact.inverse = 1.0f / e.exact.a;
 	return e;
 }
 
 // What every row of a triangle needs (ITriangle2D.cpp:70-176): the three edges of
 // rasterizeTriangle, the clipped columns and the aligned row bound.  Set up once per draw
 // command; rows are then independent of each other.  flags: the edges' kinds in bits 0-1,
-// 2-3 and 4-5, bit 6 = two equal corners.
+// 2-3 and 4-5, bit 6 = two equal corners, bit 7 = wide edges.
 struct __attribute__((aligned(16))) TriangleRows {
 	EdgeRows edges[3];
 	int32_t clipL, clipR, alT, alB;
@@ -473,15 +500,17 @@ DH TriangleRows triangleRows(const l2 &A, const l2 &B, const l2 &C, const Rect &
 	const Rect rowClip = rectSides(clipR.l, al.t, clipR.right(), al.bottom());
 	const EdgeSetup e0 = edgeSetup(A, B, rowClip), e1 = edgeSetup(B, C, rowClip), e2 = edgeSetup(C, A, rowClip);
 	TriangleRows tr;
-	tr.edges[0] = edgeRows(e0);
-	tr.edges[1] = edgeRows(e1);
-	tr.edges[2] = edgeRows(e2);
+	const int32_t rows = al.h;
+	const bool wide = !(edgeFitsDouble(e0, rows) && edgeFitsDouble(e1, rows) && edgeFitsDouble(e2, rows)) || clipR.right() > 65536;
+	tr.edges[0] = edgeRows(e0, wide);
+	tr.edges[1] = edgeRows(e1, wide);
+	tr.edges[2] = edgeRows(e2, wide);
 	tr.clipL = clipR.l;
 	tr.clipR = clipR.right();
 	tr.alT = al.t;
 	tr.alB = al.bottom();
 	const bool degenerate = sameCorner(A, B) || sameCorner(B, C) || sameCorner(C, A);
-	tr.flags = e0.kind | (e1.kind << 2) | (e2.kind << 4) | (degenerate ? 64 : 0);
+	tr.flags = e0.kind | (e1.kind << 2) | (e2.kind << 4) | (degenerate ? 64 : 0) | (wide ? 128 : 0);
 	return tr;
 }
 
@@ -517,6 +546,36 @@ __device__ __forceinline__ int32_t edgeSide(int64_t n, int64_t d, int32_t L, int
 	return tmin(tmax(L, (int32_t)(divTrunc64(n, d) + 1)), R);
 }
 
+// clamp(trunc(m / a) + 1, L, R) for m a whole number below 2^52 in double, a and inverse as EdgeRows
+// has them, |m / a| below 2^30 and columns L and R of at most 65 536.  The float estimate of |m / a|
+// is within 2^-22 of it relatively, so that, truncated, it is at most one off where the columns do not
+// decide; the remainder, one fused operation and exact, tells.
+__device__ __forceinline__ int32_t rowSide(double m, float a, float inverse, int32_t L, int32_t R) {
+	const double size = fabs(m), divisor = (double)a;
+	const float estimate = truncf((float)size * inverse);
+	const double remainder = __builtin_fma(-(double)estimate, divisor, size);
+	const int32_t q = (int32_t)estimate + (remainder >= divisor ? 1 : 0) - (remainder < 0.0 ? 1 : 0);
+	return tmin(tmax(L, (m < 0.0 ? -q : q) + 1), R);
+}
+
+// The same row from the 64-bit integers, for the triangles whose terms leave the doubles' range.  A
+// function of its own: it is rare, and its divisions would triple the size of every caller's row code.
+__device__ __attribute__((noinline)) RowInterval wideRow(const EdgeRows *edges, int32_t flags, int32_t rowIndex, int32_t L, int32_t R) {
+	RowInterval row{L, R};
+	const int64_t r = rowIndex;
+	for (int k = 0; k < 3; k++) {
+		const EdgeRows &e = edges[k];
+		const int32_t kind = (flags >> (2 * k)) & 3;
+		const int64_t along = e.wide.b * r;
+		const bool sloped = kind == 1 || kind == 2;
+		const int32_t side = edgeSide(e.wide.c - along + (kind == 1 ? 1 : 0), sloped ? e.wide.a : 1, L, R);
+		if (kind == 1) row.left = tmax(row.left, side);
+		if (kind == 2) row.right = tmin(row.right, side);
+		if (kind == 3 && e.wide.c + along > e.wide.a) { row.left = R; row.right = L; }
+	}
+	return row;
+}
+
 // Row y of the triangle (rasterizeTriangle, ITriangle2D.cpp:150-169, row y - alT of the
 // aligned bound); empty outside the aligned bound.
 __device__ __forceinline__ RowInterval triangleRow(const TriangleRows &tr, int32_t y) {
@@ -524,20 +583,21 @@ __device__ __forceinline__ RowInterval triangleRow(const TriangleRows &tr, int32
 	if (y < tr.alT || y >= tr.alB) return row;
 	const int32_t L = tr.clipL, R = tr.clipR;
 	if (tr.flags & 64) { row.left = R; row.right = L; return row; }
-	const int64_t r = y - tr.alT;
+	if (tr.flags & 128) return wideRow(tr.edges, tr.flags, y - tr.alT, L, R);
+	const double r = (double)(y - tr.alT);
 	row.left = L;
 	row.right = R;
 	// Every edge takes the same steps whatever its kind (lanes of one wavefront hold edges of
 	// different kinds); the kind picks which result is kept.
+#pragma unroll
 	for (int k = 0; k < 3; k++) {
 		const EdgeRows &e = tr.edges[k];
 		const int32_t kind = (tr.flags >> (2 * k)) & 3;
-		const int64_t along = e.b * r;
-		const bool sloped = kind == 1 || kind == 2;
-		const int32_t side = edgeSide(e.c - along + (kind == 1 ? 1 : 0), sloped ? e.a : 1, L, R);
+		const double m = __builtin_fma(-e.exact.b, r, e.exact.c);
+		const int32_t side = rowSide(m, e.exact.a, e.exact.inverse, L, R);
 		if (kind == 1) row.left = tmax(row.left, side);
 		if (kind == 2) row.right = tmin(row.right, side);
-		if (kind == 3 && e.c + along > e.a) { row.left = R; row.right = L; }
+		if (kind == 3 && m < 0.0) { row.left = R; row.right = L; }
 	}
 	return row;
 }

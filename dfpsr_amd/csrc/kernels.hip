@@ -69,31 +69,29 @@ __device__ __forceinline__ int32_t jobOfPair(const BinJob *jobs, int32_t count, 
 // 96 views of 256x256: raster 632 -> 358 us.  Where triangles are larger the test does not pay: a
 // 1080p terrain loses a quarter of its pairs, but its raster gains 2 us and its setup loses as much.
 //
-// An edge cuts a row at trunc(n / a) with n = c - b * row (triangleRow), so it keeps column x >= 1
-// exactly when n >= a * x; column 0 takes every n > -a from a right edge (truncation), and no more
-// than n >= 0 from a left one.  n is linear in the row: if the best of the tile's first and last row
-// fails at the tile's best column, the edge keeps nothing of the tile.  Edges whose quotients could
-// pass int32, which the rows wrap as the reference does, are not tested.  What is left of few rows
-// is decided by the rows themselves.
+// A right edge ends row r at trunc(m / a), m = c - b * r (EdgeRows), so it keeps column x >= 1 exactly
+// when m >= a * x, and column 0 when m > -a (truncation); a left edge starts it after trunc(m / a) and
+// keeps column x >= 1 when m < a * x, column 0 when m <= -a.  m is linear in the row: if the best of
+// the tile's first and last row fails at the tile's best column, the edge keeps nothing of the tile.
+// What is left of few rows is decided by the rows themselves.
 constexpr int32_t PAIR_EXACT_ROWS = 4;
 __device__ __forceinline__ bool pairCovers(const TriangleRows &tr, int32_t x0, int32_t y0, int32_t w, int32_t h) {
 	if (tr.flags & 64) return false;
 	const int32_t left = tmax(x0, tr.clipL), right = tmin(x0 + w, tr.clipR);
 	const int32_t top = tmax(y0, tr.alT), bottom = tmin(y0 + h, tr.alB);
 	if (left >= right || top >= bottom) return false;
-	const int64_t big = (int64_t)1 << 40, wide = (int64_t)1 << 60;
+	if (tr.flags & 128) return true;
 	bool missed = false;
 #pragma unroll
 	for (int k = 0; k < 3; k++) {
 		const EdgeRows e = tr.edges[k];
 		const int32_t kind = (tr.flags >> (2 * k)) & 3;
-		const bool tested = kind != 0 && e.a < big && e.a > -big && e.b < big && e.b > -big && e.c < wide && e.c > -wide;
-		const int64_t first = e.b * (top - tr.alT), last = e.b * (bottom - 1 - tr.alT);
-		const int64_t nearest = e.c - tmin(first, last), farthest = e.c - tmax(first, last);
-		const float limit = 1.0e9f * fabsf((float)e.a);
-		const bool small = fabsf((float)nearest) < limit && fabsf((float)farthest) < limit;
-		const bool sloped = kind == 2 && left == 0 ? nearest <= -e.a : nearest < e.a * (kind == 2 ? left : right - 1);
-		missed = missed || (tested && (kind == 3 ? e.c + tmin(first, last) > e.a : small && sloped));
+		const double first = __builtin_fma(-e.exact.b, (double)(top - tr.alT), e.exact.c);
+		const double last = __builtin_fma(-e.exact.b, (double)(bottom - 1 - tr.alT), e.exact.c);
+		const double least = fmin(first, last), most = fmax(first, last), a = (double)e.exact.a;
+		if (kind == 1) missed = missed || (right > 1 ? least >= a * (right - 1) : least > -a);
+		if (kind == 2) missed = missed || (left > 0 ? most < a * left : most <= -a);
+		if (kind == 3) missed = missed || most < 0.0;
 	}
 	if (missed) return false;
 	if (bottom - top > PAIR_EXACT_ROWS) return true;
@@ -2449,11 +2447,16 @@ __global__ void k_occlude_top_rows(const float *depth, int32_t width, int32_t he
 	if (farthest < grid[cell]) grid[cell] = farthest;
 }
 
-// The side a row takes from one edge (edgeSide) for count (n, d, L, R) inputs: the check of
-// the row intervals' quotient against exact integer arithmetic.
+// The side a row takes from one edge for count (n, d, L, R) inputs -- by the double form where its
+// operands fit it, as the rows do, by the integers otherwise: the check of the row intervals' quotient
+// against exact integer arithmetic.
 __global__ void k_probe_edge_side(const int64_t *n, const int64_t *d, const int32_t *L, const int32_t *R, int32_t count, int32_t *out) {
 	const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < count) out[i] = edgeSide(n[i], d[i], L[i], R[i]);
+	if (i >= count) return;
+	const double m = d[i] < 0 ? -(double)n[i] : (double)n[i], a = fabs((double)d[i]);
+	const bool fits = fabs(m) < 4503599627370496.0 && a < 4294967296.0 && (double)(float)a == a && fabs(m) < 1073741824.0 * a &&
+	                  L[i] >= -65536 && L[i] <= 65536 && R[i] >= -65536 && R[i] <= 65536;
+	out[i] = fits ? rowSide(m, (float)a, 1.0f / (float)a, L[i], R[i]) : edgeSide(n[i], d[i], L[i], R[i]);
 }
 
 __global__ void k_fill(int32_t *p, int32_t n, int32_t value) {

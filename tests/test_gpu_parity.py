@@ -291,6 +291,28 @@ def test_canvas_with_both_projections(api):
     assert (out[0][0] != 0).any()
 
 
+@pytest.mark.parametrize("log2_reach", [12, 19, 23, 24, 27])
+def test_rows_of_far_corners(api, renderer, log2_reach):
+    """Corners up to 2^27 sub-pixels away, some edges nearly horizontal or vertical: below 2^24 a row's
+    sides come from doubles, beyond that from 64-bit integers, and both give the oracle's rows."""
+    n = 150
+    sc = projected_by_oracle(S.cube_soup(width=120, height=75, triangles=n, seed=log2_reach, cam_distance=2.0, spread=0.6))
+    rng = S.Rng(1000 + log2_reach)
+    reach = 1 << log2_reach
+    flat = rng.integers(n * 6, -reach, reach).reshape(n, 3, 2) + np.array([60, 37]) * 256
+    flat[::3, 1, 1] = flat[::3, 0, 1] + rng.integers((n + 2) // 3, -1, 2)   # an edge of at most 1 / 256 row
+    flat[1::3, 2, 0] = flat[1::3, 0, 0] + rng.integers((n + 1) // 3, -1, 2)
+    sc.projected = sc.projected.copy()
+    sc.projected["flat"] = flat
+    print(f"[gpu] far corners 2^{log2_reach}", flush=True)
+    ref = H.oracle_render(sc)
+    assert (ref[1] > 0).any()
+    for path in (0, 1):
+        r = api.renderer_create()
+        api.renderer_setTuning(r, api.tuning(tile_config=1, raster_path=path))
+        assert_parity(sc, api.render_scene(sc, r), ref)
+
+
 def test_direct_bins_grow_to_the_longest_tile_list(api):
     """Tiles holding more commands than the direct bins' starting size (64) make the first frame
     overflow them: the renderer grows the bins to the longest list and draws the frame again
