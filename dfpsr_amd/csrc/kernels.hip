@@ -905,43 +905,6 @@ __device__ __forceinline__ bool evalQuad(const Command &cmd, RowInterval upper, 
 	return evalQuad(cmd.plane, upper, lower, px, py, canvasHeight, e);
 }
 
-// The integer part of evalQuad: whether the command touches the quad at (px, py) and, per lane,
-// the pixel it writes and whether the row's sides keep it -- without the weight chains.
-struct QuadLanes {
-	int slot[4];
-	bool clip[4];
-	bool clipSides;
-};
-
-__device__ __forceinline__ bool quadLanes(RowInterval upper, RowInterval lower, int32_t px, int32_t py, int32_t canvasHeight,
-                                          QuadLanes &q) {
-	const int32_t outerStart = tmin(upper.left, lower.left);
-	const int32_t outerEnd = tmax(upper.right, lower.right);
-	const int32_t innerStart = tmax(upper.left, lower.left);
-	const int32_t innerEnd = tmin(upper.right, lower.right);
-	const int32_t outerBlockStart = (int32_t)((uint32_t)outerStart & ~1u);
-	const int32_t outerBlockEnd = (int32_t)(((uint32_t)outerEnd + 1u) & ~1u);
-	const int32_t innerBlockStart = (int32_t)(((uint32_t)innerStart + 1u) & ~1u);
-	const int32_t innerBlockEnd = (int32_t)((uint32_t)innerEnd & ~1u);
-	if (py + 1 >= canvasHeight) lower.right = lower.left;
-	const bool hasTop = upper.right > upper.left;
-	const bool hasBottom = lower.right > lower.left;
-	if (!(hasTop || hasBottom)) return false;
-	if (px < outerBlockStart || px >= outerBlockEnd) return false;
-	const bool inner = innerBlockEnd > innerBlockStart && px >= innerBlockStart && px < innerBlockEnd;
-	q.clipSides = !inner;
-	q.slot[0] = hasTop ? 0 : 2;
-	q.slot[1] = hasTop ? 1 : 3;
-	q.slot[2] = hasBottom ? 2 : 0;
-	q.slot[3] = hasBottom ? 3 : 1;
-	const int32_t x2 = px + 1;
-	q.clip[0] = px >= upper.left && px < upper.right;
-	q.clip[1] = x2 >= upper.left && x2 < upper.right;
-	q.clip[2] = px >= lower.left && px < lower.right;
-	q.clip[3] = x2 >= lower.left && x2 < lower.right;
-	return true;
-}
-
 // Vertex weights of a lane (fillRowSuper, fillerTemplates.h:222-238): perspective divides the
 // depth-divided weights by 1/W.
 __device__ __forceinline__ void laneWeights(const QuadEval &e, int l, bool affine, float &wa, float &wb, float &wc) {
@@ -1422,8 +1385,8 @@ template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 
 // Keys order depths as floats compare: larger depth, larger key; -0 equals +0.
 __device__ __forceinline__ uint32_t depthOrder(float d) {
-	uint32_t u = __float_as_uint(d == 0.0f ? 0.0f : d);
-	return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+	const uint32_t u = __float_as_uint(d + 0.0f);  // -0 + 0 = +0
+	return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
 // A row interval in LDS: columns fit 16 bits (the visibility raster takes canvases up to
@@ -1548,12 +1511,9 @@ __device__ __forceinline__ void stageToLds(T *dst, const uint8_t *src, const int
 __device__ __forceinline__ void stageWait() { __builtin_amdgcn_s_waitcnt(0); }
 
 
-// The chunk command that won a pixel's key, or -1.
-__device__ __forceinline__ int32_t keyWinner(unsigned long long key, bool depthRead) {
-	if (!depthRead) return (int32_t)key - 1;
-	const uint32_t low = (uint32_t)key;
-	return low == 0xFFFFFFFFu ? -1 : (int32_t)(0xFFFFFFFEu - low);
-}
+// The low half of a key of chunk command j, below which the canvas's own value (all ones) ranks first
+// and equal depths go to the earlier command.  Without a depth canvas the high half is j + 1.
+__device__ __forceinline__ uint32_t keyOfCommand(int32_t j) { return 0xFFFFFFFEu - (uint32_t)j; }
 
 // Index of the segment holding item it in an exclusive prefix of count + 1 entries.
 template <typename T>
@@ -1566,17 +1526,28 @@ __device__ __forceinline__ int32_t segmentOf(const T *offset, int32_t count, int
 	return lo;
 }
 
+// The lanes of command j's quad, whose upper left pixel has its key at key[0], that won their pixels.
+// A lane's pixel is the lane's own except in an odd canvas's last row (oddRow), where the key's high
+// half says which of a column's two lanes wrote it.
+template <int TW, bool GENERAL>
+__device__ __forceinline__ uint32_t lanesWon(const unsigned long long *key, int32_t j, bool oddRow) {
+	const uint32_t *half = (const uint32_t *)key;
+	const uint32_t own = keyOfCommand(j);
+	if (GENERAL && oddRow)
+		return (half[0] == own ? 1u << (2 * (half[1] & 1u)) : 0u) | (half[2] == own ? 2u << (2 * (half[3] & 1u)) : 0u);
+	return (half[0] == own ? 1u : 0u) | (half[2] == own ? 2u : 0u) | (half[2 * TW] == own ? 4u : 0u) | (half[2 * TW + 2] == own ? 8u : 0u);
+}
+
 // MODE 0: the RGBA8 shaders into the colour canvas.  MODE 1: the differentiable float shader
 // into the float colour canvas plus the visibility id of each pixel's winning lane.
 template <int TW, int TH, int MODE, bool GENERAL, int CH>
-__device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW, TH, CH, MODE> &s, const TextureDesc *textures) {
+__device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW, TH, CH, MODE> &s, const TextureTable &textures) {
 	using S = DeferShape<TW, TH, CH>;
 	constexpr int32_t NT = S::NT, CHUNK = S::CHUNK;
 	constexpr int32_t NP = TW * TH, RP = TH / 2;
 	constexpr int32_t PAIRS = DeferLds<TW, TH, CH, MODE>::PAIRS;
 	constexpr int32_t ITEM_TABLE = DeferLds<TW, TH, CH, MODE>::ITEM_TABLE;
 	constexpr int32_t PAIRS_PER_THREAD = PAIRS / NT > 0 ? PAIRS / NT : 1;
-	static_assert(PAIRS * (TW / 2) <= 32 * NT, "a thread's items fit the 32 four-bit masks of pass 2a");
 	const int32_t n = f.tileCount[tile];
 	const int32_t ci = findSegment(f.canvasTileEnd, f.canvasCount, tile);
 	const CanvasDev cv = f.canvases[ci];
@@ -1700,16 +1671,14 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				const bool ok = evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + 2 * rp]), rowInterval(s.rows[j * TH + 2 * rp + 1]),
 				                         px, py, cv.height, e);
 				if (!ok) continue;
+				// A lane whose row misses the quad is clipped, so a lane that counts is its own pixel.
+				unsigned long long *key = &s.keys[2 * rp * TW + px - tileX0];
+#pragma unroll
 				for (int l = 0; l < 4; l++) {
-					if (e.clipSides && !e.clip[l]) continue;
-					const int32_t sl = e.slot[l];
-					const int32_t p = (py - tileY0 + (sl >> 1)) * TW + (px - tileX0 + (sl & 1));
-					if (depthRead) {
-						const float d = e.l0[l];
-						if (d == d) atomicMax(&s.keys[p], ((unsigned long long)(depthOrder(d) ^ flip) << 32) | (unsigned long long)(0xFFFFFFFEu - (uint32_t)j));
-					} else {
-						atomicMax(&s.keys[p], (unsigned long long)(j + 1));
-					}
+					const float d = e.l0[l];
+					const bool offers = (!e.clipSides || e.clip[l]) && (!depthRead || d == d);
+					const uint32_t rank = depthRead ? depthOrder(d) ^ flip : (uint32_t)(j + 1);
+					if (offers) atomicMax(&key[(l >> 1) * TW + (l & 1)], ((unsigned long long)rank << 32) | keyOfCommand(j));
 				}
 			}
 			// The odd canvas's last row: both lanes of a column test the depth held before the
@@ -1741,70 +1710,58 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 #pragma unroll
 				for (int i = 0; i < 2; i++)
 					if (winner[i] >= 0)
-						s.keys[(py - tileY0) * TW + 2 * t + i] = ((unsigned long long)lower[i] << 32) |
-						                                        (depthRead ? 0xFFFFFFFEu - (uint32_t)winner[i] : (uint32_t)winner[i] + 1u);
+						s.keys[(py - tileY0) * TW + 2 * t + i] = ((unsigned long long)lower[i] << 32) | keyOfCommand(winner[i]);
 			}
 			__syncthreads();
 			if (MODE == 0) {
-				// Pass 2a: the lanes each item's command won, read from the keys before pass 2b
-				// overwrites them; four bits per item of this thread (at most 32 items).
-				uint64_t wonLow = 0, wonHigh = 0;
-				for (int32_t it = t, k = 0; it < items; it += NT, k++) {
-					const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
-					const int32_t j = pr / RP, rp = pr % RP;
-					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
-					QuadLanes q;
-					uint64_t mask = 0;
-					if (quadLanes(rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx, tileY0 + qy, cv.height, q)) {
-						for (int l = 0; l < 4; l++) {
-							if (q.clipSides && !q.clip[l]) continue;
-							const int32_t sl = q.slot[l];
-							const unsigned long long key = s.keys[(qy + (sl >> 1)) * TW + qx + (sl & 1)];
-							if (keyWinner(key, depthRead) == j && !(GENERAL && tileY0 + qy + 1 >= cv.height && (int)(key >> 32) != l >> 1)) mask |= 1ull << l;
-						}
-					}
-					if (k < 16) wonLow |= mask << (4 * k);
-					else wonHigh |= mask << (4 * (k - 16));
-				}
-				__syncthreads();
-				// Pass 2b: each item that won a lane evaluates its quad again (keeping pass 1's
+				// Pass 2: each item that won a lane evaluates its quad again (keeping pass 1's
 				// evaluations would cost more registers than the evaluation), writes the won lanes'
-				// depths, and leaves for every won pixel its weights (in the pixel's key, no longer
-				// read) and its command and the quad's mip level (in its colour, about to be
-				// replaced), so that pass 2c shades each pixel once with all threads busy.
-				for (int32_t it = t, k = 0; it < items; it += NT, k++) {
-					const uint32_t mask = (uint32_t)((k < 16 ? wonLow >> (4 * k) : wonHigh >> (4 * (k - 16))) & 0xFu);
-					if (!mask) continue;
+				// depths, and leaves for every won pixel its weights (in the pixel's key) and its command
+				// and the quad's mip level (in its colour, about to be replaced), so that pass 3 shades
+				// each pixel once with all threads busy.  Only a pixel's winner replaces its key, and the
+				// weight that takes the low half's place is no other command's: those halves are NaNs that
+				// no arithmetic gives, and a NaN weight is stored as the usual one.  So no barrier
+				// separates the reading of the keys from their replacement.
+				for (int32_t it = t; it < items; it += NT) {
 					const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
 					const int32_t j = pr / RP, rp = pr % RP;
 					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
+					const int32_t first = qy * TW + qx;
+					const bool oddRow = GENERAL && tileY0 + qy + 1 >= cv.height;
+					const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[first], j, oddRow);
+					if (!mask) continue;
 					QuadEval e;
 					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
 					              tileY0 + qy, cv.height, e))
 						continue;
-					int32_t pixel[4];
-					for (int l = 0; l < 4; l++) {
-						const int32_t sl = e.slot[l];
-						pixel[l] = (qy + (sl >> 1)) * TW + qx + (sl & 1);
-						if (!((mask >> l) & 1u)) continue;
-						s.depth[pixel[l]] = e.l0[l];
-						if (!fillAll) atomicOr(&s.dirty[pixel[l] >> 5], 1u << (pixel[l] & 31));
+					// The won pixels of the quad's two rows, as bits of their words.
+					const uint32_t upper = (oddRow ? mask | (mask >> 2) : mask) & 3u, lower = oddRow ? 0u : mask >> 2;
+					if (!fillAll) {
+						atomicOr(&s.dirty[first >> 5], upper << (first & 31));
+						atomicOr(&s.dirty[(first + TW) >> 5], lower << ((first + TW) & 31));
 					}
+#pragma unroll
+					for (int l = 0; l < 4; l++)
+						if ((mask >> l) & 1u) s.depth[first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1)] = e.l0[l];
 					if (colorWrite) {
 						const bool affine = (s.command[j].flags & 1) != 0;
 						float wa[4], wb[4], wc[4];
 						for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
-						const uint32_t mip = quadMip(s.si[j], textures, wa, wb, wc);
+						const uint32_t meta = (uint32_t)j | (quadMip(s.si[j], textures, wa, wb, wc) << 8);
+						atomicOr(&s.chunkWon[first >> 5], upper << (first & 31));
+						atomicOr(&s.chunkWon[(first + TW) >> 5], lower << ((first + TW) & 31));
+#pragma unroll
 						for (int l = 0; l < 4; l++) {
 							if (!((mask >> l) & 1u)) continue;
-							s.keys[pixel[l]] = ((unsigned long long)__float_as_uint(wc[l]) << 32) | __float_as_uint(wb[l]);
-							s.color[pixel[l]] = (uint32_t)j | (mip << 8);
-							atomicOr(&s.chunkWon[pixel[l] >> 5], 1u << (pixel[l] & 31));
+							const int32_t p = first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1);
+							const uint32_t weight = wb[l] == wb[l] ? __float_as_uint(wb[l]) : 0x7FC00000u;
+							s.keys[p] = ((unsigned long long)__float_as_uint(wc[l]) << 32) | weight;
+							s.color[p] = meta;
 						}
 					}
 				}
 				__syncthreads();
-				// Pass 2c: every pixel won in this chunk, shaded once.
+				// Pass 3: every pixel won in this chunk, shaded once.
 				if (colorWrite) {
 					for (int32_t p = t; p < NP; p += NT) {
 						if (!((s.chunkWon[p >> 5] >> (p & 31)) & 1u)) continue;
@@ -1822,18 +1779,12 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 					const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
 					const int32_t j = pr / RP, rp = pr % RP;
 					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
+					const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[qy * TW + qx], j, GENERAL && tileY0 + qy + 1 >= cv.height);
+					if (!mask) continue;
 					QuadEval e;
 					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
 					              tileY0 + qy, cv.height, e))
 						continue;
-					uint32_t mask = 0;
-					for (int l = 0; l < 4; l++) {
-						if (e.clipSides && !e.clip[l]) continue;
-						const int32_t sl = e.slot[l];
-						const unsigned long long key = s.keys[(qy + (sl >> 1)) * TW + qx + (sl & 1)];
-						if (keyWinner(key, depthRead) == j && !(GENERAL && tileY0 + qy + 1 >= cv.height && (int)(key >> 32) != l >> 1)) mask |= 1u << l;
-					}
-					if (!mask) continue;
 					// Depths first, so that only the weights and the won lanes' pixels outlive the quad
 					// evaluation while the colours are made.
 					uint32_t slots = 0;
@@ -1889,7 +1840,8 @@ __global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_e
 			((uint32_t *)s.textures)[i] = ((const uint32_t *)f.textures)[i];
 		__syncthreads();
 	}
-	const TextureDesc *textures = ldsTextures ? s.textures : f.textures;
+	const TextureTable textures = {(const __attribute__((address_space(3))) TextureDesc *)s.textures,
+	                               (const __attribute__((address_space(1))) TextureDesc *)f.textures, ldsTextures};
 	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 0, GENERAL>(f, tile, s, textures); });
 }
 
@@ -1905,7 +1857,7 @@ __global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_e
 	__shared__ DeferLds<TW, TH, DIFF_CHUNK, 1> s;
 	reportCounters(f);
 	if (f.counters[2]) return;
-	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 1, GENERAL>(f, tile, s, nullptr); });
+	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 1, GENERAL>(f, tile, s, TextureTable()); });
 }
 
 #define DEFERRED_SHAPE(TW, TH, P, GENERAL)                              \

@@ -149,7 +149,7 @@ __device__ __forceinline__ void sampleQuad(const TextureDesc &t, const float *u,
 	for (int l = 0; l < 4; l++) out[l] = mixSample(b[l], px[l * 4], px[l * 4 + 1], px[l * 4 + 2], px[l * 4 + 3]);
 }
 
-DH uint32_t sampleBilinear(const TextureDesc &t, float u, float v, uint32_t mip, bool highest) {
+__device__ __forceinline__ uint32_t sampleBilinear(const TextureDesc &t, float u, float v, uint32_t mip, bool highest) {
 	uint32_t scaleU = 256u << t.log2w, scaleV = 256u << t.log2h;
 	uint32_t maskX = t.maxWidthAndMask, maskY = t.maxHeightAndMask;
 	uint32_t stride = t.log2w;
@@ -167,11 +167,10 @@ DH uint32_t sampleBilinear(const TextureDesc &t, float u, float v, uint32_t mip,
 	uint32_t right = (left + 1u) & maskX, bottom = (top + 1u) & maskY;
 	left &= maskX;
 	top &= maskY;
-	const uint32_t *base = t.texels + layer;
-	uint32_t ul = __ldg(base + ((top << stride) | left));
-	uint32_t ur = __ldg(base + ((top << stride) | right));
-	uint32_t bl = __ldg(base + ((bottom << stride) | left));
-	uint32_t br = __ldg(base + ((bottom << stride) | right));
+	const uint32_t ul = loadTexel(t.texels, layer + ((top << stride) | left));
+	const uint32_t ur = loadTexel(t.texels, layer + ((top << stride) | right));
+	const uint32_t bl = loadTexel(t.texels, layer + ((bottom << stride) | left));
+	const uint32_t br = loadTexel(t.texels, layer + ((bottom << stride) | right));
 	return mixColors(mixColors(ul, ur, wx), mixColors(bl, br, wx), wy);
 }
 
@@ -241,7 +240,7 @@ struct Quad4 { float v[4]; };
 
 // getPixels_2x2 (RgbaMultiply.h:74-106) for the lanes of one quad in mask (bit l = lane l;
 // the others are left unset).  The mip level always comes from lanes 0, 1 and 2.
-DH void shadeQuad(const ShaderInputs &s, const TextureDesc *textures, const float *wa, const float *wb, const float *wc,
+__device__ __forceinline__ void shadeQuad(const ShaderInputs &s, const TextureDesc *textures, const float *wa, const float *wb, const float *wc,
                   uint32_t mask, float *r, float *g, float *b, float *a) {
 	if (s.diffuse >= 0 && s.light < 0 && s.colorless) {
 		const TextureDesc &t = textures[s.diffuse];
@@ -305,19 +304,50 @@ DH void shadeQuad(const ShaderInputs &s, const TextureDesc *textures, const floa
 	}
 }
 
+// A texture table of the visibility raster: in LDS when it is small, else in global memory.  Two typed
+// pointers and a uniform branch instead of one generic pointer, whose flat loads would go through both
+// memories' counters.
+struct TextureTable {
+	const __attribute__((address_space(3))) TextureDesc *lds;
+	const __attribute__((address_space(1))) TextureDesc *global;
+	bool inLds;
+	// What sampling reads of texture i.
+	__device__ __forceinline__ TextureDesc sampled(int32_t i) const {
+		TextureDesc d;
+		if (inLds) {
+			d.texels = lds[i].texels; d.log2w = lds[i].log2w; d.log2h = lds[i].log2h; d.startOffset = lds[i].startOffset;
+			d.maxLevelMask = lds[i].maxLevelMask; d.maxWidthAndMask = lds[i].maxWidthAndMask; d.maxHeightAndMask = lds[i].maxHeightAndMask;
+		} else {
+			d.texels = global[i].texels; d.log2w = global[i].log2w; d.log2h = global[i].log2h; d.startOffset = global[i].startOffset;
+			d.maxLevelMask = global[i].maxLevelMask; d.maxWidthAndMask = global[i].maxWidthAndMask; d.maxHeightAndMask = global[i].maxHeightAndMask;
+		}
+		return d;
+	}
+	// What the choice of the mip level reads of texture i.
+	__device__ __forceinline__ TextureDesc mipped(int32_t i) const {
+		TextureDesc d;
+		if (inLds) {
+			d.floatMaxWidth = lds[i].floatMaxWidth; d.floatMaxHeight = lds[i].floatMaxHeight; d.maxMip = lds[i].maxMip;
+		} else {
+			d.floatMaxWidth = global[i].floatMaxWidth; d.floatMaxHeight = global[i].floatMaxHeight; d.maxMip = global[i].maxMip;
+		}
+		return d;
+	}
+};
+
 // The mip level a quad samples its diffuse texture at (0 without one): texture_getMipLevelIndex
 // of lanes 0, 1 and 2's texture coordinates, as shadeQuad takes it.
-__device__ __forceinline__ uint32_t quadMip(const ShaderInputs &s, const TextureDesc *textures, const float *wa, const float *wb,
+__device__ __forceinline__ uint32_t quadMip(const ShaderInputs &s, const TextureTable &textures, const float *wa, const float *wb,
                                             const float *wc) {
 	if (s.diffuse < 0) return 0u;
 	float u[3], v[3];
 	for (int l = 0; l < 3; l++) { u[l] = interp(s.u1, wa[l], wb[l], wc[l]); v[l] = interp(s.v1, wa[l], wb[l], wc[l]); }
-	return mipLevelIndex(textures[s.diffuse], u[0], u[1], u[2], v[0], v[1], v[2]);
+	return mipLevelIndex(textures.mipped(s.diffuse), u[0], u[1], u[2], v[0], v[1], v[2]);
 }
 
 // One lane of shadeQuad followed by packSaturated, with the quad's mip level given: the same
 // operations in the same order for one pixel.
-__device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const TextureDesc *textures, float wa, float wb, float wc,
+__device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const TextureTable &textures, float wa, float wb, float wc,
                                                uint32_t mip) {
 	const bool textureOnly = s.colorless && ((s.diffuse >= 0) != (s.light >= 0));
 	float r = 0.0f, g = 0.0f, b = 0.0f, a = 0.0f;
@@ -333,7 +363,7 @@ __device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const Text
 	}
 	if (s.diffuse >= 0) {
 		float sr, sg, sb, sa;
-		unpackColor(sampleBilinear(textures[s.diffuse], interp(s.u1, wa, wb, wc), interp(s.v1, wa, wb, wc), mip, false), sr, sg, sb, sa);
+		unpackColor(sampleBilinear(textures.sampled(s.diffuse), interp(s.u1, wa, wb, wc), interp(s.v1, wa, wb, wc), mip, false), sr, sg, sb, sa);
 		if (textureOnly) {
 			r = sr; g = sg; b = sb; a = sa;
 		} else {
@@ -342,7 +372,7 @@ __device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const Text
 	}
 	if (s.light >= 0) {
 		float sr, sg, sb, sa;
-		unpackColor(sampleBilinear(textures[s.light], interp(s.u2, wa, wb, wc), interp(s.v2, wa, wb, wc), 0u, true), sr, sg, sb, sa);
+		unpackColor(sampleBilinear(textures.sampled(s.light), interp(s.u2, wa, wb, wc), interp(s.v2, wa, wb, wc), 0u, true), sr, sg, sb, sa);
 		if (textureOnly) {
 			r = sr; g = sg; b = sb; a = sa;
 		} else {
@@ -356,7 +386,7 @@ __device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const Text
 // comes from the texture coordinates of lanes 0, 1 and 2 (texture_getMipLevelIndex).
 DH float pickLane(const float *v, int l) { return l == 0 ? v[0] : (l == 1 ? v[1] : (l == 2 ? v[2] : v[3])); }
 
-DH void shadeLane(const ShaderInputs &s, const TextureDesc *textures, const float *wa, const float *wb, const float *wc, int l,
+__device__ __forceinline__ void shadeLane(const ShaderInputs &s, const TextureDesc *textures, const float *wa, const float *wb, const float *wc, int l,
                   float &r, float &g, float &b, float &a) {
 	const float la = pickLane(wa, l), lb = pickLane(wb, l), lc = pickLane(wc, l);
 	if (s.diffuse >= 0 && s.light < 0 && s.colorless) {
