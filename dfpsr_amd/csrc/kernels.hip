@@ -1396,7 +1396,7 @@ __device__ __forceinline__ RowSpan rowSpan(RowInterval r) { return RowSpan{(int1
 __device__ __forceinline__ RowInterval rowInterval(RowSpan r) { return RowInterval{r.left, r.right}; }
 
 // CHUNK: commands staged and drawn at once.  Sixteen keep a 32x16 workgroup of the RGBA8 shaders
-// within the LDS of ten workgroups per CU, the occupancy of five waves per SIMD.  The persistent
+// within the LDS of eleven workgroups per CU.  The persistent
 // grid's 32-pixel-wide tiles take 32 (at most eight workgroups per CU run anyway), and so do all
 // tiles of the differentiable shader, whose scenes are denser, so that fewer tiles need a
 // second chunk.
@@ -1404,14 +1404,15 @@ template <int TW, int TH, int P>
 constexpr int32_t colorChunk() { return P != 0 && TW * TH >= 512 ? 32 : 16; }
 constexpr int32_t DIFF_CHUNK = 32;
 
-// Threads of a visibility-raster workgroup: four pixels of the tile per thread.
+// Threads of a visibility-raster workgroup: four pixels of the tile per thread.  A 32x16 workgroup with
+// chunks of 16 keeps to 14 080 bytes of LDS, so that eleven of them fit a CU.
 template <int TW, int TH, int CH> struct DeferShape {
 	static constexpr int32_t NT = TW * TH / 4;
 	static constexpr int32_t CHUNK = CH;                   // commands per chunk
-	static constexpr int32_t LIST = 256;                    // commands sorted per round
+	static constexpr bool TIGHT = TW * TH <= 512 && CH == 16;
+	static constexpr int32_t LIST = TIGHT ? 192 : 256;     // commands sorted per round
+	static constexpr int32_t TEXTURES = TIGHT ? 8 : 16;    // texture tables up to this size are read from LDS
 };
-
-constexpr int32_t LDS_TEXTURES = 16;  // texture tables up to this size are read from LDS
 
 static_assert(sizeof(TriangleRows) % 16 == 0 && sizeof(ShaderInputs) % 16 == 0 && sizeof(Command) % 16 == 0,
               "staged records are whole 16-byte units");
@@ -1479,12 +1480,12 @@ template <int TW, int TH, int CH, int MODE> struct DeferLds {
 			PairIndex pairOfItem[ITEM_TABLE];    // the pair of each of the first ITEM_TABLE pass-1 items
 		};
 	};
-	uint32_t color[RGBA ? TW * TH : 1];          // the tile's canvas pixels as they stand
-	float depth[TW * TH];
+	float depth[TW * TH];                        // the tile's depths as they stand
+	uint32_t color[RGBA ? TW * TH : 1];          // the drawn pixels' colours
 	uint32_t dirty[TW * TH / 32];                // pixels written, one bit each
 	uint32_t chunkWon[RGBA ? TW * TH / 32 : 1];  // pixels the current chunk's commands won
 	int32_t scan[S::NT / 64];                    // wavefront totals of the prefix sums
-	TextureDesc textures[RGBA ? LDS_TEXTURES : 1];
+	TextureDesc textures[RGBA ? S::TEXTURES : 1];
 	int32_t roundInfo[4];
 	int32_t slot;
 };
@@ -1510,6 +1511,9 @@ __device__ __forceinline__ void stageToLds(T *dst, const uint8_t *src, const int
 // Waits for this thread's LDS-direct loads; a barrier then publishes them to the workgroup.
 __device__ __forceinline__ void stageWait() { __builtin_amdgcn_s_waitcnt(0); }
 
+
+// A canvas store: the pointer, read from memory, is known to be global.
+template <typename T> __device__ __forceinline__ void storeGlobal(T *p, T value) { *(__attribute__((address_space(1))) T *)p = value; }
 
 // The low half of a key of chunk command j, below which the canvas's own value (all ones) ranks first
 // and equal depths go to the earlier command.  Without a depth canvas the high half is j + 1.
@@ -1564,18 +1568,14 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 	for (int32_t p = t; p < NP; p += NT) {
 		if (f.clearInRaster) {
 			s.depth[p] = f.clearDepth;
-			if (MODE == 0) s.color[p] = f.clearColor;
 		} else {
 			const int32_t x = tileX0 + p % TW, y = tileY0 + p / TW;
 			s.depth[p] = (depthRead && x < cv.width && y < cv.height) ? cv.depth[(size_t)y * cv.depthStride + x] : 0.0f;
 		}
 	}
-	// With the fill fused in, every pixel is written back.  The differentiable shader writes its
-	// colours and ids itself, so there the dirty bits keep marking the drawn pixels: the others
-	// take the fill values at the write-back.
-	const bool fillAll = f.clearInRaster && MODE == 0;
-	const bool fillUndrawn = f.clearInRaster && MODE == 1;
-	for (int32_t w = t; w < NP / 32; w += NT) s.dirty[w] = fillAll ? ~0u : 0u;
+	// With the fill fused in, the pixels that no command draws take the fill values at the write-back.
+	for (int32_t w = t; w < NP / 32; w += NT) s.dirty[w] = 0u;
+	if (n == 0) __syncthreads();  // an empty tile only takes the fill: no round's barrier comes before the write-back
 
 	int32_t last = -1;
 	int32_t done = 0;
@@ -1736,10 +1736,8 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 						continue;
 					// The won pixels of the quad's two rows, as bits of their words.
 					const uint32_t upper = (oddRow ? mask | (mask >> 2) : mask) & 3u, lower = oddRow ? 0u : mask >> 2;
-					if (!fillAll) {
-						atomicOr(&s.dirty[first >> 5], upper << (first & 31));
-						atomicOr(&s.dirty[(first + TW) >> 5], lower << ((first + TW) & 31));
-					}
+					atomicOr(&s.chunkWon[first >> 5], upper << (first & 31));
+					atomicOr(&s.chunkWon[(first + TW) >> 5], lower << ((first + TW) & 31));
 #pragma unroll
 					for (int l = 0; l < 4; l++)
 						if ((mask >> l) & 1u) s.depth[first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1)] = e.l0[l];
@@ -1747,28 +1745,27 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 						const bool affine = (s.command[j].flags & 1) != 0;
 						float wa[4], wb[4], wc[4];
 						for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
-						const uint32_t meta = (uint32_t)j | (quadMip(s.si[j], textures, wa, wb, wc) << 8);
-						atomicOr(&s.chunkWon[first >> 5], upper << (first & 31));
-						atomicOr(&s.chunkWon[(first + TW) >> 5], lower << ((first + TW) & 31));
+						const uint32_t shade = (uint32_t)j | (quadMip(s.si[j], textures, wa, wb, wc) << 5);
 #pragma unroll
 						for (int l = 0; l < 4; l++) {
 							if (!((mask >> l) & 1u)) continue;
 							const int32_t p = first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1);
 							const uint32_t weight = wb[l] == wb[l] ? __float_as_uint(wb[l]) : 0x7FC00000u;
 							s.keys[p] = ((unsigned long long)__float_as_uint(wc[l]) << 32) | weight;
-							s.color[p] = meta;
+							s.color[p] = shade;
 						}
 					}
 				}
 				__syncthreads();
 				// Pass 3: every pixel won in this chunk, shaded once.
+				for (int32_t w = t; w < NP / 32; w += NT) s.dirty[w] |= s.chunkWon[w];
 				if (colorWrite) {
 					for (int32_t p = t; p < NP; p += NT) {
 						if (!((s.chunkWon[p >> 5] >> (p & 31)) & 1u)) continue;
-						const uint32_t meta = s.color[p];
+						const uint32_t shade = s.color[p];
 						const unsigned long long weights = s.keys[p];
 						const float wb = __uint_as_float((uint32_t)weights), wc = __uint_as_float((uint32_t)(weights >> 32));
-						s.color[p] = shadePixel(s.si[meta & 0xFFu], textures, 1.0f - (wb + wc), wb, wc, meta >> 8);
+						s.color[p] = shadePixel(s.si[shade & 31u], textures, 1.0f - (wb + wc), wb, wc, shade >> 5);
 					}
 				}
 			} else {
@@ -1808,11 +1805,11 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 
 	for (int32_t p = t; p < NP; p += NT) {
 		const bool drawn = ((s.dirty[p >> 5] >> (p & 31)) & 1u) != 0;
-		if (!drawn && !fillUndrawn) continue;
+		if (!drawn && !f.clearInRaster) continue;
 		const int32_t x = tileX0 + p % TW, y = tileY0 + p / TW;
 		if (x >= cv.width || y >= cv.height) continue;
-		if (colorWrite) cv.color[(size_t)y * cv.colorStride + x] = s.color[p];
-		if (depthRead) cv.depth[(size_t)y * cv.depthStride + x] = s.depth[p];
+		if (colorWrite) storeGlobal(cv.color + (size_t)y * cv.colorStride + x, drawn ? s.color[p] : f.clearColor);
+		if (depthRead) storeGlobal(cv.depth + (size_t)y * cv.depthStride + x, s.depth[p]);
 		if (MODE == 1 && !drawn) {  // the fill values of k_clear_canvases
 			const size_t q = (size_t)y * cv.diffStride + x;
 			*(float4 *)(cv.diffColor + q * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1822,18 +1819,21 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 	if (f.selfClean && t == 0) f.tileCount[tile] = 0;  // read by this workgroup alone, long before
 }
 
-// Five waves per SIMD: the raster is bound by latency, and the fifth wave hides more of it than a
-// larger register budget would save.  P = 1: persistent workgroups, at four waves per SIMD (a
-// persistent grid holds at most eight workgroups per CU).  The two forms are separate kernels so
+// Waves per SIMD: as many as the LDS leaves room for, since the raster waits for memory and barriers as
+// much as for its own instructions (4K terrain 138 us with ten 32x16 workgroups per CU, 133 with eleven).
+// P = 1: persistent workgroups, at four waves per SIMD (a persistent grid holds at most eight workgroups
+// per CU).  The two forms are separate kernels so
 // that each gets its own register allocation (the persistent loop keeps more values live).
+template <int TW, int TH, int P>
+constexpr int32_t rasterWaves() { return P ? 4 : (TW * TH == 512 ? 6 : 5); }
 template <int TW, int TH, int P, bool GENERAL>
-__global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_eu(P ? 4 : 5, P ? 4 : 5))) k_raster_deferred(FrameDev f) {
+__global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_eu(rasterWaves<TW, TH, P>(), rasterWaves<TW, TH, P>()))) k_raster_deferred(FrameDev f) {
 	__shared__ DeferLds<TW, TH, colorChunk<TW, TH, P>(), 0> s;
 	reportCounters(f);
 	resetNextCounters(f);
 	if (f.counters[2]) return;  // an earlier stage ran out of room: leave the canvases untouched
 	// Small texture tables are read from LDS by the shading.
-	const bool ldsTextures = f.textureCount <= LDS_TEXTURES;
+	const bool ldsTextures = f.textureCount <= DeferShape<TW, TH, colorChunk<TW, TH, P>()>::TEXTURES;
 	if (ldsTextures) {
 		constexpr int32_t W = (int32_t)(sizeof(TextureDesc) / 4);
 		for (int32_t i = threadIdx.x; i < f.textureCount * W; i += TW * TH / 4)
@@ -1845,11 +1845,11 @@ __global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_e
 	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 0, GENERAL>(f, tile, s, textures); });
 }
 
-// Waves per SIMD of the differentiable visibility raster: five for 32x16 tiles of one workgroup
-// each (20 B of scratch, 6 % faster on the 8-view fit), four for the others, where a fifth costs
-// more in scratch than it gains.
+// Waves per SIMD of the differentiable visibility raster: six for 32x16 tiles of one workgroup
+// each (16 B of scratch; 8-view fit forward raster 169 us with five, 160 with six), four for the others,
+// where more costs more in scratch than it gains.
 template <int TW, int TH, int P>
-constexpr int32_t diffWaves() { return P == 0 && TW * TH == 512 ? 5 : 4; }
+constexpr int32_t diffWaves() { return P == 0 && TW * TH == 512 ? 6 : 4; }
 
 // The differentiable forward by the visibility raster.
 template <int TW, int TH, int P, bool GENERAL>
