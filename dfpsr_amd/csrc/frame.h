@@ -193,10 +193,10 @@ private:
 	uint64_t cleanGenerations_[3] = {0, 0, 0};
 	int32_t cleanTiles_ = 0, cleanCanvases_ = 0;
 	void dropGraph();
-	// The visibility raster reproduces the in-order result when every command is Solid and each
-	// canvas's commands have one projection.
+	// The visibility raster reproduces the in-order result when each canvas's commands have one
+	// projection; the differentiable shader's only draws Solid commands.
 	bool deferredRaster(const RenderOptions &o) const {
-		return o.rasterPath == 0 && !alphaAny_ && !mixedCanvas_ && !wideCanvas_;
+		return o.rasterPath == 0 && !(alphaAny_ && o.mode == 1) && !mixedCanvas_ && !wideCanvas_;
 	}
 };
 

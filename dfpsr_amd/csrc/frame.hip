@@ -156,21 +156,23 @@ static inline int32_t blocksOf(int64_t n, int32_t size) { return (int32_t)((n + 
 static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // The visibility raster of a frame with one tile shape: RGBA8 or differentiable, one workgroup per
-// tile or persistent, for even perspective canvases alone or for any (general).
-template <int TW, int TH, int P, bool GENERAL>
-static void launchDeferredForm(const FrameDev &f, int32_t grid, hipStream_t stream) {
-	if (f.mode == 1) hipLaunchKernelGGL((k_raster_deferred_diff<TW, TH, P, GENERAL>), dim3(grid), dim3(TW * TH / 4), 0, stream, f);
-	else hipLaunchKernelGGL((k_raster_deferred<TW, TH, P, GENERAL>), dim3(grid), dim3(TW * TH / 4), 0, stream, f);
+// tile or persistent, in the form the frame needs.
+template <int TW, int TH, int P>
+static void launchDeferredForm(const FrameDev &f, int32_t grid, int32_t form, hipStream_t stream) {
+	const dim3 groups(grid), threads(TW * TH / 4);
+	if (f.mode == 1) {
+		if (form == FORM_PLAIN) hipLaunchKernelGGL((k_raster_deferred_diff<TW, TH, P, FORM_PLAIN>), groups, threads, 0, stream, f);
+		else hipLaunchKernelGGL((k_raster_deferred_diff<TW, TH, P, FORM_GENERAL>), groups, threads, 0, stream, f);
+	} else {
+		if (form == FORM_PLAIN) hipLaunchKernelGGL((k_raster_deferred<TW, TH, P, FORM_PLAIN>), groups, threads, 0, stream, f);
+		else if (form == FORM_GENERAL) hipLaunchKernelGGL((k_raster_deferred<TW, TH, P, FORM_GENERAL>), groups, threads, 0, stream, f);
+		else hipLaunchKernelGGL((k_raster_deferred<TW, TH, P, FORM_ALPHA>), groups, threads, 0, stream, f);
+	}
 }
 template <int TW, int TH>
-static void launchDeferred(const FrameDev &f, int32_t grid, int32_t persistent, bool general, hipStream_t stream) {
-	if (persistent) {
-		if (general) launchDeferredForm<TW, TH, 1, true>(f, grid, stream);
-		else launchDeferredForm<TW, TH, 1, false>(f, grid, stream);
-	} else {
-		if (general) launchDeferredForm<TW, TH, 0, true>(f, grid, stream);
-		else launchDeferredForm<TW, TH, 0, false>(f, grid, stream);
-	}
+static void launchDeferred(const FrameDev &f, int32_t grid, int32_t persistent, int32_t form, hipStream_t stream) {
+	if (persistent) launchDeferredForm<TW, TH, 1>(f, grid, form, stream);
+	else launchDeferredForm<TW, TH, 0>(f, grid, form, stream);
 }
 
 int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks, int32_t tileBlocks, bool events, int parts,
@@ -217,10 +219,11 @@ int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks,
 	} else if (deferredRaster(o)) {
 		bool general = oddCanvas_;
 		for (uint8_t p : projections_) general = general || (p & 2) != 0;
+		const int32_t form = alphaAny_ ? FORM_ALPHA : (general ? FORM_GENERAL : FORM_PLAIN);
 		switch (tileConfig_) {
-		case 1: launchDeferred<32, 16>(f, grid, persistent, general, stream); break;
-		case 2: launchDeferred<32, 32>(f, grid, persistent, general, stream); break;
-		default: launchDeferred<16, 16>(f, grid, persistent, general, stream); break;
+		case 1: launchDeferred<32, 16>(f, grid, persistent, form, stream); break;
+		case 2: launchDeferred<32, 32>(f, grid, persistent, form, stream); break;
+		default: launchDeferred<16, 16>(f, grid, persistent, form, stream); break;
 		}
 	} else if (o.mode == 1) {
 		switch (tileConfig_) {

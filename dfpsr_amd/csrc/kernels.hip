@@ -312,7 +312,7 @@ __device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, i
 				Command c;
 				const f2 is[3] = {P[0].is, P[1].is, P[2].is};
 				c.plane = weightPlanes(is, make3(P[0].cs.z, P[1].cs.z, P[2].cs.z), make3(0.0f, 1.0f, 0.0f), make3(0.0f, 0.0f, 1.0f), perspective);
-				c.task = ti; c.fan = local; c.flags = perspective ? 0 : 1;
+				c.task = ti; c.fan = local; c.flags = (perspective ? 0 : 1) | (t.filter != 0 ? 2 : 0);
 				emitCommand(f, offset, c, P, cv, si, tally, jobs, jobBase);
 			}
 			count = 1;
@@ -340,7 +340,7 @@ __device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, i
 					const f2 is[3] = {S[0].is, S[1].is, S[2].is};
 					c.plane = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), make3(va.subB, vb.subB, vc.subB),
 					                       make3(va.subC, vb.subC, vc.subC), perspective);
-					c.task = ti; c.fan = local; c.flags = perspective ? 0 : 1;
+					c.task = ti; c.fan = local; c.flags = (perspective ? 0 : 1) | (t.filter != 0 ? 2 : 0);
 					emitCommand(f, offset + count, c, S, cv, si, tally, jobs, jobBase);
 				}
 				count++;
@@ -1350,10 +1350,10 @@ template __global__ void k_raster<32, 16>(FrameDev, int32_t);
 template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 
 // ---------------------------------------------------------------------------------------
-// Visibility raster for frames whose commands are all Solid and, per canvas, all perspective or
-// all orthogonal.
+// Visibility raster for frames whose canvases hold commands of one projection each, perspective or
+// orthogonal.
 //
-// In the reference's order a pixel ends with the colour and depth of the first command
+// Of Solid commands in the reference's order, a pixel ends with the colour and depth of the first
 // reaching the best depth beyond the pixel's starting depth: a perspective command writes where
 // its 1/W is strictly greater than the depth held at that moment, an orthogonal one where its W
 // is strictly smaller (fillerTemplates.h:110-152), so the held depth is always the best value
@@ -1367,7 +1367,7 @@ template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 // thread per (command, row) for the exact rows, per (command, covered quad) for the keys and
 // per (command, covered quad) again for the shading of the lanes each command won.
 //
-// GENERAL: the frame has an orthogonal canvas or one of odd height.  An odd canvas's last row has
+// FORM_GENERAL: the frame has an orthogonal canvas or one of odd height.  An odd canvas's last row has
 // no row below, and a quad's lower
 // lanes there write the upper row's pixels after the upper lanes (fillerTemplates.h:287-323),
 // so one command can leave a depth worse than its own other candidate and the argument above
@@ -1377,9 +1377,14 @@ template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 // 73 us.  Frames of even perspective canvases take kernels without that code, which made the
 // persistent grid's 384-job batch 3 % slower.
 //
-// Frames with the Alpha filter (blending reads the colour held at that moment), canvases that
-// mix both projections (the depth test's direction changes between commands) and canvases wider
-// than 32767 pixels (rows are kept in 16 bits) take the in-order kernel above.
+// FORM_ALPHA: the frame has tasks with the Alpha filter, whose blending reads the colour held at that
+// moment.  A chunk is then drawn in runs of one filter: runs of Solid commands through the keys, runs
+// of Alpha commands by a walk in submission order with a thread per quad (blendRun).  It includes
+// FORM_GENERAL.
+//
+// Canvases that mix both projections (the depth test's direction changes between commands), canvases
+// wider than 32767 pixels (rows are kept in 16 bits) and differentiable frames with the Alpha filter
+// take the in-order kernel above.
 // ---------------------------------------------------------------------------------------
 
 
@@ -1542,11 +1547,65 @@ __device__ __forceinline__ uint32_t lanesWon(const unsigned long long *key, int3
 	return (half[0] == own ? 1u : 0u) | (half[2] == own ? 2u : 0u) | (half[2 * TW] == own ? 4u : 0u) | (half[2 * TW + 2] == own ? 8u : 0u);
 }
 
+// The Alpha filter's commands [j0, j1) of a chunk over the tile's colours and depths in LDS: a thread
+// per quad walks them in submission order (drawCommand's tests, shading and blending), no thread needs
+// another's pixels, and the commands' rows and inputs are staged, so nothing separates two commands.
+// The in-order raster, which this replaces, made each command's rows between two barriers of its own.
+template <int TW, int TH, typename Lds>
+__device__ __forceinline__ void blendRun(Lds &s, int32_t j0, int32_t j1, int32_t tileX0, int32_t tileY0, const CanvasDev &cv,
+                                         const TextureTable &textures, bool depthRead) {
+	const int32_t t = opaqueThreadIndex();
+	const int32_t qx = 2 * (t % (TW / 2)), qy = 2 * (t / (TW / 2)), first = qy * TW + qx;
+	uint32_t drawn = 0;
+	for (int32_t j = j0; j < j1; j++) {
+		QuadEval e;
+		if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx, tileY0 + qy,
+		              cv.height, e))
+			continue;
+		const bool affine = (s.command[j].flags & 1) != 0;
+		uint32_t visible = 0, old[4];
+#pragma unroll
+		for (int l = 0; l < 4; l++) {
+			const int32_t p = first + (e.slot[l] >> 1) * TW + (e.slot[l] & 1);
+			bool front = true;
+			if (depthRead) {
+				const float held = s.depth[p];
+				front = affine ? e.l0[l] < held : e.l0[l] > held;
+			}
+			if (e.clip[l] && front) visible |= 1u << l;
+			old[l] = s.color[p];
+		}
+		if (!visible) continue;
+		float wa[4], wb[4], wc[4];
+		for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
+		const uint32_t mip = quadMip(s.si[j], textures, wa, wb, wc);
+#pragma unroll
+		for (int l = 0; l < 4; l++) {
+			if (!((visible >> l) & 1u)) continue;
+			float r, g, b, a, tr, tg, tb, ta;
+			shadeChannels(s.si[j], textures, wa[l], wb[l], wc[l], mip, r, g, b, a);
+			unpackColor(old[l], tr, tg, tb, ta);
+			const float opacity = a * (1.0f / 255.0f), inv = 1.0f - opacity;
+			r = (r * opacity) + (tr * inv);
+			g = (g * opacity) + (tg * inv);
+			b = (b * opacity) + (tb * inv);
+			a = (a * opacity) + (ta * inv);
+			s.color[first + (e.slot[l] >> 1) * TW + (e.slot[l] & 1)] = packSaturated(r, g, b, a);
+			drawn |= 1u << e.slot[l];
+		}
+	}
+	if (drawn) {
+		atomicOr(&s.dirty[first >> 5], (drawn & 3u) << (first & 31));
+		atomicOr(&s.dirty[(first + TW) >> 5], (drawn >> 2) << ((first + TW) & 31));
+	}
+}
+
 // MODE 0: the RGBA8 shaders into the colour canvas.  MODE 1: the differentiable float shader
 // into the float colour canvas plus the visibility id of each pixel's winning lane.
-template <int TW, int TH, int MODE, bool GENERAL, int CH>
+template <int TW, int TH, int MODE, int FORM, int CH>
 __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW, TH, CH, MODE> &s, const TextureTable &textures) {
 	using S = DeferShape<TW, TH, CH>;
+	constexpr bool GENERAL = FORM != FORM_PLAIN, ALPHA = FORM == FORM_ALPHA;
 	constexpr int32_t NT = S::NT, CHUNK = S::CHUNK;
 	constexpr int32_t NP = TW * TH, RP = TH / 2;
 	constexpr int32_t PAIRS = DeferLds<TW, TH, CH, MODE>::PAIRS;
@@ -1571,6 +1630,10 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 		} else {
 			const int32_t x = tileX0 + p % TW, y = tileY0 + p / TW;
 			s.depth[p] = (depthRead && x < cv.width && y < cv.height) ? cv.depth[(size_t)y * cv.depthStride + x] : 0.0f;
+		}
+		if (ALPHA && colorWrite) {  // blending reads the colours that are there
+			const int32_t x = tileX0 + p % TW, y = tileY0 + p / TW;
+			s.color[p] = f.clearInRaster ? f.clearColor : (x < cv.width && y < cv.height ? cv.color[(size_t)y * cv.colorStride + x] : 0u);
 		}
 	}
 	// With the fill fused in, the pixels that no command draws take the fill values at the write-back.
@@ -1619,6 +1682,20 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				s.rows[j * TH + r] = rowSpan(triangleRow(s.tr[j], tileY0 + r));
 			}
 			__syncthreads();
+			// Runs of commands of one filter, in submission order (one run for all without the Alpha filter).
+			for (int32_t j0 = 0, j1 = cn; j0 < cn; j0 = j1) {
+			if (ALPHA && colorWrite) {
+				const int32_t lane = t & 63;
+				const uint64_t blended = __ballot(lane < cn && (s.command[lane < cn ? lane : 0].flags & 2) != 0);
+				const bool blends = ((blended >> j0) & 1u) != 0;
+				const uint64_t other = (blends ? ~blended : blended) >> j0;
+				j1 = other != 0 ? tmin(j0 + (int32_t)__builtin_ctzll(other), cn) : cn;
+				if (blends) {
+					blendRun<TW, TH>(s, j0, j1, tileX0, tileY0, cv, textures, depthRead);
+					__syncthreads();
+					continue;
+				}
+			}
 			// Keys start at the held depth with the lowest command part above every command's,
 			// so only a strictly greater depth replaces it; a NaN depth is never replaced.
 			for (int32_t p = t; p < NP; p += NT) {
@@ -1635,7 +1712,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				const int32_t pr = t * PAIRS_PER_THREAD + k;
 				const int32_t j = pr / RP, rp = pr % RP;
 				int32_t count = 0, x0 = 0;
-				if (pr < PAIRS && j < cn) {
+				if (pr < PAIRS && j < j1 && (!ALPHA || j >= j0)) {
 					const RowInterval upper = rowInterval(s.rows[j * TH + 2 * rp]), lower = rowInterval(s.rows[j * TH + 2 * rp + 1]);
 					if (upper.right > upper.left || lower.right > lower.left) {
 						const int32_t outerBlockStart = (int32_t)((uint32_t)tmin(upper.left, lower.left) & ~1u);
@@ -1688,7 +1765,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				const int32_t py = cv.height - 1, px = tileX0 + 2 * t;
 				float held[2] = {s.depth[(py - tileY0) * TW + 2 * t], s.depth[(py - tileY0) * TW + 2 * t + 1]};
 				int32_t winner[2] = {-1, -1}, lower[2] = {0, 0};
-				for (int32_t j = 0; j < cn; j++) {
+				for (int32_t j = j0; j < j1; j++) {
 					const RowSpan upperRow = s.rows[j * TH + py - tileY0];
 					if (upperRow.right <= upperRow.left) continue;
 					QuadEval e;
@@ -1798,6 +1875,7 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 				}
 			}
 			__syncthreads();
+			}
 		}
 		done += take;
 		if (take == 0) break;
@@ -1824,10 +1902,11 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 // P = 1: persistent workgroups, at four waves per SIMD (a persistent grid holds at most eight workgroups
 // per CU).  The two forms are separate kernels so
 // that each gets its own register allocation (the persistent loop keeps more values live).
-template <int TW, int TH, int P>
-constexpr int32_t rasterWaves() { return P ? 4 : (TW * TH == 512 ? 6 : 5); }
-template <int TW, int TH, int P, bool GENERAL>
-__global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_eu(rasterWaves<TW, TH, P>(), rasterWaves<TW, TH, P>()))) k_raster_deferred(FrameDev f) {
+// The Alpha form's walk keeps a quad and four colours in registers.
+template <int TW, int TH, int P, int FORM>
+constexpr int32_t rasterWaves() { return P || FORM == FORM_ALPHA ? 4 : (TW * TH == 512 ? 6 : 5); }
+template <int TW, int TH, int P, int FORM>
+__global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_eu(rasterWaves<TW, TH, P, FORM>(), rasterWaves<TW, TH, P, FORM>()))) k_raster_deferred(FrameDev f) {
 	__shared__ DeferLds<TW, TH, colorChunk<TW, TH, P>(), 0> s;
 	reportCounters(f);
 	resetNextCounters(f);
@@ -1842,7 +1921,7 @@ __global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_e
 	}
 	const TextureTable textures = {(const __attribute__((address_space(3))) TextureDesc *)s.textures,
 	                               (const __attribute__((address_space(1))) TextureDesc *)f.textures, ldsTextures};
-	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 0, GENERAL>(f, tile, s, textures); });
+	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 0, FORM>(f, tile, s, textures); });
 }
 
 // Waves per SIMD of the differentiable visibility raster: six for 32x16 tiles of one workgroup
@@ -1852,23 +1931,28 @@ template <int TW, int TH, int P>
 constexpr int32_t diffWaves() { return P == 0 && TW * TH == 512 ? 6 : 4; }
 
 // The differentiable forward by the visibility raster.
-template <int TW, int TH, int P, bool GENERAL>
+template <int TW, int TH, int P, int FORM>
 __global__ void __launch_bounds__(TW * TH / 4) __attribute__((amdgpu_waves_per_eu(diffWaves<TW, TH, P>(), diffWaves<TW, TH, P>()))) k_raster_deferred_diff(FrameDev f) {
 	__shared__ DeferLds<TW, TH, DIFF_CHUNK, 1> s;
 	reportCounters(f);
 	if (f.counters[2]) return;
-	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 1, GENERAL>(f, tile, s, TextureTable()); });
+	forEachQueuedTile(f, P, &s.slot, [&](int32_t tile) { rasterTileDeferred<TW, TH, 1, FORM>(f, tile, s, TextureTable()); });
 }
 
-#define DEFERRED_SHAPE(TW, TH, P, GENERAL)                              \
-	template __global__ void k_raster_deferred<TW, TH, P, GENERAL>(FrameDev); \
-	template __global__ void k_raster_deferred_diff<TW, TH, P, GENERAL>(FrameDev);
-#define DEFERRED_SHAPES(P, GENERAL) DEFERRED_SHAPE(16, 16, P, GENERAL) DEFERRED_SHAPE(32, 16, P, GENERAL) DEFERRED_SHAPE(32, 32, P, GENERAL)
-DEFERRED_SHAPES(0, false)
-DEFERRED_SHAPES(1, false)
-DEFERRED_SHAPES(0, true)
-DEFERRED_SHAPES(1, true)
-#undef DEFERRED_SHAPES
+#define DEFERRED_SHAPE(TW, TH, FORM)                                    \
+	template __global__ void k_raster_deferred<TW, TH, 0, FORM>(FrameDev); \
+	template __global__ void k_raster_deferred<TW, TH, 1, FORM>(FrameDev);
+#define DEFERRED_DIFF_SHAPE(TW, TH, FORM)                                    \
+	template __global__ void k_raster_deferred_diff<TW, TH, 0, FORM>(FrameDev); \
+	template __global__ void k_raster_deferred_diff<TW, TH, 1, FORM>(FrameDev);
+#define EVERY_TILE_SHAPE(KIND, FORM) KIND(16, 16, FORM) KIND(32, 16, FORM) KIND(32, 32, FORM)
+EVERY_TILE_SHAPE(DEFERRED_SHAPE, FORM_PLAIN)
+EVERY_TILE_SHAPE(DEFERRED_SHAPE, FORM_GENERAL)
+EVERY_TILE_SHAPE(DEFERRED_SHAPE, FORM_ALPHA)
+EVERY_TILE_SHAPE(DEFERRED_DIFF_SHAPE, FORM_PLAIN)
+EVERY_TILE_SHAPE(DEFERRED_DIFF_SHAPE, FORM_GENERAL)
+#undef EVERY_TILE_SHAPE
+#undef DEFERRED_DIFF_SHAPE
 #undef DEFERRED_SHAPE
 
 // The differentiable forward: the same tile walk with the float shader, persistent or not.

@@ -76,7 +76,7 @@ constexpr int32_t DENSE_PIXELS_PER_FAN = 8;
 struct __attribute__((aligned(16))) Command {
 	Projection plane;      // weight planes
 	int32_t task, fan;     // source: task and fan triangle within the task's model
-	int32_t flags;         // bit 0 = affine (orthogonal camera)
+	int32_t flags;         // bit 0 = affine (orthogonal camera), bit 1 = Alpha filter
 };
 static_assert(sizeof(Command) == 48, "three 16-byte units");
 
@@ -203,9 +203,12 @@ __global__ void k_scan_tiles_local(FrameDev f);
 __global__ void k_scan_tiles_add(FrameDev f);
 __global__ void k_bin_fill(FrameDev f);
 template <int TW, int TH> __global__ void k_raster(FrameDev f, int32_t persistent);
-template <int TW, int TH, int P, bool GENERAL> __global__ void k_raster_deferred(FrameDev f);
+// Forms of the visibility raster: even perspective canvases with Solid commands alone; any canvases;
+// any canvases and the Alpha filter.
+enum { FORM_PLAIN = 0, FORM_GENERAL = 1, FORM_ALPHA = 2 };
+template <int TW, int TH, int P, int FORM> __global__ void k_raster_deferred(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_diff(FrameDev f, int32_t persistent);
-template <int TW, int TH, int P, bool GENERAL> __global__ void k_raster_deferred_diff(FrameDev f);
+template <int TW, int TH, int P, int FORM> __global__ void k_raster_deferred_diff(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_depth(FrameDev f);
 __global__ void k_probe_edge_side(const int64_t *n, const int64_t *d, const int32_t *L, const int32_t *R, int32_t count, int32_t *out);
 template <bool DERIVE> __global__ void k_backward(FrameDev f, int32_t *heads);

@@ -345,12 +345,12 @@ __device__ __forceinline__ uint32_t quadMip(const ShaderInputs &s, const Texture
 	return mipLevelIndex(textures.mipped(s.diffuse), u[0], u[1], u[2], v[0], v[1], v[2]);
 }
 
-// One lane of shadeQuad followed by packSaturated, with the quad's mip level given: the same
-// operations in the same order for one pixel.
-__device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const TextureTable &textures, float wa, float wb, float wc,
-                                               uint32_t mip) {
+// One lane of shadeQuad, with the quad's mip level given: the same operations in the same order for
+// one pixel.
+__device__ __forceinline__ void shadeChannels(const ShaderInputs &s, const TextureTable &textures, float wa, float wb, float wc,
+                                              uint32_t mip, float &r, float &g, float &b, float &a) {
 	const bool textureOnly = s.colorless && ((s.diffuse >= 0) != (s.light >= 0));
-	float r = 0.0f, g = 0.0f, b = 0.0f, a = 0.0f;
+	r = g = b = a = 0.0f;
 	if (!textureOnly) {
 		if (s.fading) {
 			r = interp(s.red, wa, wb, wc);
@@ -379,6 +379,13 @@ __device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const Text
 			r = r * sr; g = g * sg; b = b * sb; a = a * sa;
 		}
 	}
+}
+
+// The same followed by packSaturated.
+__device__ __forceinline__ uint32_t shadePixel(const ShaderInputs &s, const TextureTable &textures, float wa, float wb, float wc,
+                                               uint32_t mip) {
+	float r, g, b, a;
+	shadeChannels(s, textures, wa, wb, wc, mip, r, g, b, a);
 	return packSaturated(r, g, b, a);
 }
 

@@ -272,6 +272,41 @@ def test_visibility_raster_of_odd_heights_and_orthogonal_cameras(api, size, canv
     assert_parity(sc, results[0], H.oracle_render(sc))
 
 
+@pytest.mark.parametrize("orthogonal", [False, True])
+@pytest.mark.parametrize("canvases", ["cd", "c", "d"])
+@pytest.mark.parametrize("size", [(50, 31), (96, 64)])
+def test_alpha_runs_between_solid_runs(api, size, canvases, orthogonal):
+    """Solid and Alpha models taking turns on one canvas (runs within one chunk of a tile, and across
+    chunks and rounds): the visibility raster with its blended runs gives the in-order raster's canvases
+    bit for bit, over held colours and depths, for every tile shape."""
+    parts = []
+    for k in range(5):
+        sc = odd_scene(size[0], size[1], orthogonal, canvases, seed=50 + k)
+        sc.filter = k % 2
+        n = [3, 4, 120, 120, 5][k]
+        sc.indices, sc.colors, sc.texcoords, sc.parts = sc.indices[:n], sc.colors[:n], sc.texcoords[:n].copy(), [S.Part(0, n, diffuse=0)]
+        sc.colors[:, :, 3] = S.Rng(60 + k).uniform(n * 4).reshape(n, 4)
+        sc.texcoords[:, :3, :2] = S.Rng(70 + k).uniform(n * 6, -1.0, 2.0).reshape(n, 3, 2)
+        sc.textures = [S.noise_checker_texture(32, k, 6, check=4)]
+        parts.append(api.GpuScene(sc))
+    held_color = S.Rng(5).u64(size[0] * size[1]).astype(np.uint32).reshape(size[1], size[0])
+    results = []
+    for tile_config in (0, 1, 2):
+        for path, persistent in ((1, 0), (0, 0), (0, 2)):
+            r = api.renderer_create()
+            api.renderer_setTuning(r, api.tuning(tile_config=tile_config, raster_path=path, persistent_per_cu=persistent))
+            color, depth = held_color.copy(), parts[0].scene.initial_depth.copy()
+            api.renderer_begin(r, api.host_image(color if "c" in canvases else None), api.host_image(depth if "d" in canvases else None))
+            for g in parts + parts[:2]:
+                g.give(r)
+            api.renderer_end(r)
+            results.append((color, depth))
+    for c, d in results[1:]:
+        assert np.array_equal(c, results[0][0]) and np.array_equal(d.view(np.uint32), results[0][1].view(np.uint32))
+    if "c" in canvases:
+        assert (results[0][0] != held_color).mean() > 0.1
+
+
 def test_canvas_with_both_projections(api):
     """A frame whose tasks mix perspective and orthogonal cameras on one canvas changes the direction of
     the depth test between commands: both raster settings draw it in order."""
