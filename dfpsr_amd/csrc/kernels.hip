@@ -138,20 +138,29 @@ __device__ __forceinline__ DiffInputs diffInputs(const TaskDev &task, int32_t fa
 	return d;
 }
 
-// Writes draw command `index` with everything the raster needs of it -- the command, its row
-// setup and (for the RGBA8 shaders) its finished shader inputs -- and enters it into every tile
-// it can touch: the columns of cut(wholeBound, canvas), the rows of the aligned raster bound
+// What the emit of a fan triangle needs of its task and canvas, read before the block's prefix sums
+// (with scalar loads where the wavefront has one task), so that no load chain starts after them.
+struct EmitTarget {
+	int32_t local, canvas, flags;  // the fan triangle's index in its task; the canvas slot; Command::flags
+	int32_t width, height, tileBase, tilesX, tilesY, dense;
+};
+__device__ __forceinline__ EmitTarget emitTarget(const FrameDev &f, int32_t g, int32_t ti) {
+	const TaskDev &t = f.tasks[ti];
+	const CanvasDev &cv = f.canvases[t.canvas];
+	return EmitTarget{g - t.fanBase, t.canvas, (t.camera.perspective != 0 ? 0 : 1) | (t.filter != 0 ? 2 : 0),
+	                  cv.width, cv.height, cv.tileBase, cv.tilesX, cv.tilesY, cv.dense};
+}
+
+// Writes draw command `index` with its row setup and enters it into every tile it can touch: the columns of cut(wholeBound, canvas), the rows of the aligned raster bound
 // (ITriangle2D.cpp:70-84).  With direct bins the index goes into the tile's list at once (in
 // any order: the raster sorts each list); otherwise the tile's count grows here and a pair
 // record (tile, slot, command) keeps the slot until the counts are scanned and the list is
 // filled from the records.
-__device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd, const Projected *P, const CanvasDev &cv,
-                            const ShaderInputs &si, BinTally &tally, BinJob *jobs, int32_t jobBase) {
+__device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd, const Projected *P, const EmitTarget &cv,
+                            BinTally &tally, BinJob *jobs, int32_t jobBase) {
 	f.commands[index] = cmd;
-	const TriangleRows tr = triangleRows(P[0].flat, P[1].flat, P[2].flat, canvasRect(cv));
+	const TriangleRows tr = triangleRows(P[0].flat, P[1].flat, P[2].flat, rectSides(0, 0, cv.width, cv.height));
 	f.triangleRows[index] = tr;
-	if (f.mode == 0) f.shaders[index] = si;
-	if (f.mode == 1) f.diffInputs[index] = diffInputs(f.tasks[cmd.task], cmd.fan);
 	int32_t tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;  // no tiles when the bound misses the canvas
 	if (tr.clipR > tr.clipL) {
 		// The columns and rows are at least 0 here, so shifts divide.
@@ -237,9 +246,20 @@ __device__ __forceinline__ TriangleCorners loadCorners(const FrameDev &f, int32_
 	return tc;
 }
 
-// What setupTriangle does with the draw commands it makes: count them, write and bin them, or
-// lower the occlusion grid under their hulls (renderer_occludeFromExistingTriangles).
-enum { SETUP_COUNT = 0, SETUP_EMIT = 1, SETUP_OCCLUDE = 2 };
+// The shading inputs of a fan triangle's draw commands, in the form of the frame's mode.
+__device__ __forceinline__ void storeFanInputs(const FrameDev &f, int32_t index, int32_t ti, int32_t local, const TriangleCorners &tc) {
+	if (f.mode == 0) f.shaders[index] = triangleShader(f.tasks[ti], tc.poly, tc.k);
+	if (f.mode == 1) f.diffInputs[index] = diffInputs(f.tasks[ti], local);
+}
+
+__device__ __forceinline__ void loadInputs(ShaderInputs &in, const TaskDev &t, int32_t, const TriangleCorners &tc) { in = triangleShader(t, tc.poly, tc.k); }
+__device__ __forceinline__ void loadInputs(DiffInputs &in, const TaskDev &t, int32_t local, const TriangleCorners &) { in = diffInputs(t, local); }
+__device__ __forceinline__ void storeInputs(const FrameDev &f, int32_t index, const ShaderInputs &in) { f.shaders[index] = in; }
+__device__ __forceinline__ void storeInputs(const FrameDev &f, int32_t index, const DiffInputs &in) { f.diffInputs[index] = in; }
+
+// What setupTriangle does with the draw commands: count them, or lower the occlusion grid under
+// their hulls (renderer_occludeFromExistingTriangles).
+enum { SETUP_COUNT = 0, SETUP_OCCLUDE = 1 };
 
 // occludeFromSortedHull of one Solid draw command's triangle (rendererAPI.cpp:218-239, with
 // the triangle's wholeBound as the pixel bound, :246-258): every cell whose four corners are
@@ -266,62 +286,39 @@ __device__ __forceinline__ bool survivesOcclusion(const FrameDev &f, const Proje
 	                            P[1].cs.z, P[2].cs.z);
 }
 
-// corners: the triangle's corners when the caller has loaded them already.  clipPoly: the
-// calling wavefront's clipped polygon in LDS.  Triangles that need clipping are rare; the
-// lanes holding one take the wavefront's polygon in turn, so that the polygon (nine
-// sub-vertices indexed at run time) lives in LDS instead of private scratch memory.
-// single: the caller has counted this triangle already and found one draw command, inside the
-// clip frustum and front-facing (the tests are not repeated).  With SETUP_COUNT, *single is set
-// when that is the case.  haveShader: shader holds the triangle's shader inputs already.
+// The draw commands of a fan triangle, counted or lowered into the occlusion grid.  clipPoly: the
+// calling wavefront's clipped polygon in LDS.  Triangles that need clipping are rare; the lanes
+// holding one take the wavefront's polygon in turn, so that the polygon (nine sub-vertices indexed
+// at run time) lives in LDS instead of private scratch memory.  *single is set where the triangle
+// makes one draw command, inside the clip frustum and front-facing.
 template <int MODE>
-__device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, int32_t ti, int32_t offset, BinTally &tally,
-                                                 ClipPolygon *clipPoly, BinJob *jobs = nullptr, int32_t jobBase = 0,
-                                                 const TriangleCorners *corners = nullptr, bool *single = nullptr,
-                                                 bool haveShader = false, ShaderInputs shader = ShaderInputs()) {
-	constexpr bool EMIT = MODE == SETUP_EMIT;
+__device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t ti, const TriangleCorners &tc, ClipPolygon *clipPoly,
+                                                 bool *single) {
 	const TaskDev &t = f.tasks[ti];
 	const CanvasDev &cv = f.canvases[t.canvas];
 	if (cv.color == nullptr && cv.depth == nullptr) return 0;
-	int32_t local = g - t.fanBase;
-	const TriangleCorners tc = corners ? *corners : loadCorners(f, g, ti);
-	const int32_t poly = tc.poly, k = tc.k;
-	const int32_t corner[3] = {0, 1 + k, 2 + k};
 	const Projected *P = tc.P;
 	const CameraParams &cam = t.camera;
-	const bool known = EMIT && single != nullptr && *single;
-	if (!known) {
-		if (triangleVisibility(P[0].cs, P[1].cs, P[2].cs, cam.cull) == VIS_HIDDEN) return 0;
-		if (t.filter != 0) {
-			const float *col = t.colors + poly * 16;
-			if (almostZero(col[corner[0] * 4 + 3]) && almostZero(col[corner[1] * 4 + 3]) && almostZero(col[corner[2] * 4 + 3])) return 0;
-		}
+	if (triangleVisibility(P[0].cs, P[1].cs, P[2].cs, cam.cull) == VIS_HIDDEN) return 0;
+	if (t.filter != 0) {
+		const float *col = t.colors + tc.poly * 16;
+		if (almostZero(col[3]) && almostZero(col[(1 + tc.k) * 4 + 3]) && almostZero(col[(2 + tc.k) * 4 + 3])) return 0;
 	}
-	int32_t count = 0;
-	const bool perspective = cam.perspective != 0;
-	ShaderInputs si;
-	if (EMIT && f.mode == 0) si = haveShader ? shader : triangleShader(t, poly, k);
-	if (known || triangleVisibility(P[0].cs, P[1].cs, P[2].cs, cam.clip) == VIS_FULL) {
-		if (known || frontFacing(P[0].flat, P[1].flat, P[2].flat)) {
-			if (MODE == SETUP_OCCLUDE) {
-				if (t.filter == 0) occludeFromCommand(f, P);
-				return 0;
-			}
-			if (!known && !survivesOcclusion(f, P)) return 0;
-			if (MODE == SETUP_COUNT && single != nullptr) *single = true;
-			if (EMIT) {
-				Command c;
-				const f2 is[3] = {P[0].is, P[1].is, P[2].is};
-				c.plane = weightPlanes(is, make3(P[0].cs.z, P[1].cs.z, P[2].cs.z), make3(0.0f, 1.0f, 0.0f), make3(0.0f, 0.0f, 1.0f), perspective);
-				c.task = ti; c.fan = local; c.flags = (perspective ? 0 : 1) | (t.filter != 0 ? 2 : 0);
-				emitCommand(f, offset, c, P, cv, si, tally, jobs, jobBase);
-			}
-			count = 1;
+	if (triangleVisibility(P[0].cs, P[1].cs, P[2].cs, cam.clip) == VIS_FULL) {
+		if (!frontFacing(P[0].flat, P[1].flat, P[2].flat)) return 0;
+		if (MODE == SETUP_OCCLUDE) {
+			if (t.filter == 0) occludeFromCommand(f, P);
+			return 0;
 		}
-	} else {
-		// The lanes here are exactly those that clip: one at a time, in lane order.
-		const uint64_t clipping = __ballot(1);
-		const int32_t me = (int32_t)(threadIdx.x & 63);
-		for (uint64_t pending = clipping; pending != 0; pending &= pending - 1) {
+		if (!survivesOcclusion(f, P)) return 0;
+		*single = true;
+		return 1;
+	}
+	// The lanes here are exactly those that clip: one at a time, in lane order.
+	int32_t count = 0;
+	const uint64_t clipping = __ballot(1);
+	const int32_t me = (int32_t)(threadIdx.x & 63);
+	for (uint64_t pending = clipping; pending != 0; pending &= pending - 1) {
 		if (me != __builtin_ctzll(pending)) continue;
 		ClipPolygon &poly9 = *clipPoly;
 		poly9.init(P[0].cs, P[1].cs, P[2].cs);
@@ -329,26 +326,67 @@ __device__ __forceinline__ int32_t setupTriangle(const FrameDev &f, int32_t g, i
 		for (int32_t i = 0; i < poly9.count - 2; i++) {
 			const SubVertex &va = poly9.v[0], &vb = poly9.v[1 + i], &vc = poly9.v[2 + i];
 			Projected S[3] = {cameraToScreen(cam, va.cs), cameraToScreen(cam, vb.cs), cameraToScreen(cam, vc.cs)};
-			if (frontFacing(S[0].flat, S[1].flat, S[2].flat)) {
-				if (MODE == SETUP_OCCLUDE) {
-					if (t.filter == 0) occludeFromCommand(f, S);
-					continue;
-				}
-				if (!survivesOcclusion(f, S)) continue;
-				if (EMIT) {
-					Command c;
-					const f2 is[3] = {S[0].is, S[1].is, S[2].is};
-					c.plane = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), make3(va.subB, vb.subB, vc.subB),
-					                       make3(va.subC, vb.subC, vc.subC), perspective);
-					c.task = ti; c.fan = local; c.flags = (perspective ? 0 : 1) | (t.filter != 0 ? 2 : 0);
-					emitCommand(f, offset + count, c, S, cv, si, tally, jobs, jobBase);
-				}
-				count++;
+			if (!frontFacing(S[0].flat, S[1].flat, S[2].flat)) continue;
+			if (MODE == SETUP_OCCLUDE) {
+				if (t.filter == 0) occludeFromCommand(f, S);
+				continue;
 			}
-		}
+			if (!survivesOcclusion(f, S)) continue;
+			count++;
 		}
 	}
 	return count;
+}
+
+// Writes the draw commands of a counted fan triangle from index offset on and bins them.  One round
+// of the loop takes every lane of the wavefront whose triangle is single (its tests are not repeated),
+// each further round one lane that clips: the code that makes a command is there once.
+// The caller has stored the shading inputs of a single triangle, so that they hold no registers here;
+// those of a clipped one are read again.
+__device__ __forceinline__ void emitTriangle(const FrameDev &f, int32_t ti, const EmitTarget &target, TriangleCorners &tc, bool single,
+                                             int32_t offset, BinTally &tally, ClipPolygon *clipPoly, BinJob *jobs,
+                                             int32_t jobBase) {
+	const CameraParams &cam = f.tasks[ti].camera;
+	const bool perspective = (target.flags & 1) == 0;
+	const int32_t me = (int32_t)(threadIdx.x & 63);
+	uint64_t clipping = __ballot(!single);
+	bool singles = true;
+#pragma clang loop unroll(disable)
+	while (singles || clipping != 0) {
+		const bool mine = singles ? single : me == __builtin_ctzll(clipping);
+		if (mine) {
+			ClipPolygon &poly9 = *clipPoly;
+			int32_t parts = 1, count = 0;
+			if (!single) {
+				poly9.init(tc.P[0].cs, tc.P[1].cs, tc.P[2].cs);
+				for (int32_t s = 0; s < cam.clip.count; s++) poly9.clip(cam.clip.planes[s]);
+				parts = poly9.count - 2;
+			}
+#pragma clang loop unroll(disable)
+			for (int32_t i = 0; i < parts; i++) {
+				Projected *S = tc.P;  // a clipped triangle's own corners are in its polygon
+				f3 subB = make3(0.0f, 1.0f, 0.0f), subC = make3(0.0f, 0.0f, 1.0f);
+				if (!single) {
+					const SubVertex &va = poly9.v[0], &vb = poly9.v[1 + i], &vc = poly9.v[2 + i];
+					S[0] = cameraToScreen(cam, va.cs);
+					S[1] = cameraToScreen(cam, vb.cs);
+					S[2] = cameraToScreen(cam, vc.cs);
+					subB = make3(va.subB, vb.subB, vc.subB);
+					subC = make3(va.subC, vb.subC, vc.subC);
+					if (!frontFacing(S[0].flat, S[1].flat, S[2].flat) || !survivesOcclusion(f, S)) continue;
+					storeFanInputs(f, offset + count, ti, target.local, tc);
+				}
+				Command c;
+				const f2 is[3] = {S[0].is, S[1].is, S[2].is};
+				c.plane = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), subB, subC, perspective);
+				c.task = ti; c.fan = target.local; c.flags = target.flags;
+				emitCommand(f, offset + count, c, S, target, tally, jobs, jobBase);
+				count++;
+			}
+		}
+		if (singles) singles = false;
+		else clipping &= clipping - 1;
+	}
 }
 
 // Exclusive prefix over one value per thread of an NT-thread workgroup (NT a multiple of 64);
@@ -389,30 +427,37 @@ __device__ int32_t blockExclusiveScan(int32_t value, int32_t &exclusive) {
 	return workgroupPrefix<SCAN_BLOCK>(value, exclusive, waveTotals);
 }
 
-// The task of fan triangle g, and whether every active lane of the wavefront has the same one.
-// A wavefront's triangles nearly always come from one task; the task index is then made
-// wave-uniform (readfirstlane) so that the task's fields -- camera planes, array bases -- are
-// read with scalar loads instead of one vector load per lane.
+// The task of fan triangle g.  A wavefront's triangles nearly always come from one task: its first
+// triangle's task is searched with scalar loads, and where that task holds the last one too, it is
+// every lane's (uniform).  Its fields -- camera planes, transform, array bases -- are then read with
+// scalar loads as well, instead of one dependent vector load per field and lane: two frustums of six
+// planes are twelve such loads in a row.
 __device__ __forceinline__ int32_t taskOf(const FrameDev &f, int32_t g, bool &uniform) {
-	const int32_t ti = findSegment(f.taskFanEnd, f.taskCount, g);
-	const int32_t first = __builtin_amdgcn_readfirstlane(ti);
-	uniform = __all(ti == first);
-	return ti;
+	const int32_t firstFan = __builtin_amdgcn_readfirstlane(g);
+	const int32_t first = __builtin_amdgcn_readfirstlane(findSegment(f.taskFanEnd, f.taskCount, firstFan));
+	uniform = tmin(firstFan + 63, f.fanTotal - 1) < f.taskFanEnd[first];
+	return uniform ? first : findSegment(f.taskFanEnd, f.taskCount, g);
 }
 
+// A count of FAN_SINGLE is one command that needs no clipping and has passed every test.
+constexpr int32_t FAN_SINGLE = -1;
 __global__ void __launch_bounds__(SCAN_BLOCK) k_setup_count(FrameDev f) {
 	__shared__ ClipPolygon clipPolys[SCAN_BLOCK / 64];
 	int32_t g = blockIdx.x * SCAN_BLOCK + threadIdx.x;
-	BinTally unused{0, 0};
 	int32_t n = 0;
+	bool single = false;
 	if (g < f.fanTotal) {
 		bool uniform;
 		const int32_t ti = taskOf(f, g, uniform);
 		ClipPolygon *poly = &clipPolys[threadIdx.x >> 6];
-		if (uniform) n = setupTriangle<SETUP_COUNT>(f, g, __builtin_amdgcn_readfirstlane(ti), 0, unused, poly);
-		else n = setupTriangle<SETUP_COUNT>(f, g, ti, 0, unused, poly);
+		if (uniform) {
+			const int32_t task = __builtin_amdgcn_readfirstlane(ti);
+			n = setupTriangle<SETUP_COUNT>(f, task, loadCorners(f, g, task), poly, &single);
+		} else {
+			n = setupTriangle<SETUP_COUNT>(f, ti, loadCorners(f, g, ti), poly, &single);
+		}
+		f.fanCount[g] = single ? FAN_SINGLE : n;
 	}
-	if (g < f.fanTotal) f.fanCount[g] = n;
 	int32_t ex;
 	int32_t total = blockExclusiveScan(n, ex);
 	if (threadIdx.x == 0) f.blockSums[blockIdx.x] = total;
@@ -513,9 +558,10 @@ __device__ __forceinline__ void setupEmit(const FrameDev &f, int32_t sumBlocks) 
 		tableTile[e] = -1;
 		tableCount[e] = 0;
 	}
-	const int32_t ti = g < f.fanTotal ? findSegment(f.taskFanEnd, f.taskCount, g) : 0;
+	int32_t ti = 0;
 	TriangleCorners corners;
-	ShaderInputs shader;
+	EmitTarget target;
+	typename std::conditional<SINGLE, ShaderInputs, DiffInputs>::type inputs;  // one pass: RGBA8 frames, two: mostly differentiable ones
 	int32_t n;
 	bool single = false;  // counted as one unclipped, front-facing command
 	if (SINGLE) {
@@ -524,15 +570,46 @@ __device__ __forceinline__ void setupEmit(const FrameDev &f, int32_t sumBlocks) 
 		// prefix sums, so that their latency overlaps them.
 		n = 0;
 		if (g < f.fanTotal) {
-			BinTally unused{0, 0};
-			corners = loadCorners(f, g, ti);
-			n = setupTriangle<SETUP_COUNT>(f, g, ti, 0, unused, &clipPolys[threadIdx.x >> 6], nullptr, 0, &corners, &single);
-			if (n > 0 && f.mode == 0) shader = triangleShader(f.tasks[ti], corners.poly, corners.k);
+			bool uniform;
+			ti = taskOf(f, g, uniform);
+			ClipPolygon *poly = &clipPolys[threadIdx.x >> 6];
+			if (uniform) {
+				const int32_t task = __builtin_amdgcn_readfirstlane(ti);
+				corners = loadCorners(f, g, task);
+				target = emitTarget(f, g, task);
+				n = setupTriangle<SETUP_COUNT>(f, task, corners, poly, &single);
+				if (single && f.mode == 0) loadInputs(inputs, f.tasks[task], target.local, corners);
+			} else {
+				corners = loadCorners(f, g, ti);
+				target = emitTarget(f, g, ti);
+				n = setupTriangle<SETUP_COUNT>(f, ti, corners, poly, &single);
+				if (single && f.mode == 0) loadInputs(inputs, f.tasks[ti], target.local, corners);
+			}
 		}
 	} else {
-		n = (g < f.fanTotal) ? f.fanCount[g] : 0;
-		// The corners are loaded before the block's prefix sums, so their latency overlaps them.
-		if (n > 0) corners = loadCorners(f, g, ti);
+		n = 0;
+		if (g < f.fanTotal) {
+			n = f.fanCount[g];
+			single = n == FAN_SINGLE;
+			if (single) n = 1;
+			bool uniform;
+			ti = taskOf(f, g, uniform);
+			// Loaded before the block's prefix sums, so that the latency overlaps them.
+			if (uniform) {
+				const int32_t task = __builtin_amdgcn_readfirstlane(ti);
+				target = emitTarget(f, g, task);
+				if (n > 0) {
+					corners = loadCorners(f, g, task);
+					if (f.mode == 1) loadInputs(inputs, f.tasks[task], target.local, corners);
+				}
+			} else {
+				target = emitTarget(f, g, ti);
+				if (n > 0) {
+					corners = loadCorners(f, g, ti);
+					if (f.mode == 1) loadInputs(inputs, f.tasks[ti], target.local, corners);
+				}
+			}
+		}
 	}
 	int32_t ex;
 	const int32_t blockCommands = blockExclusiveScan(n, ex);
@@ -568,11 +645,16 @@ __device__ __forceinline__ void setupEmit(const FrameDev &f, int32_t sumBlocks) 
 		const int32_t offset = jobBase + ex;
 		// The commands of a canvas's tasks are consecutive, so the offset at the first fan
 		// triangle of each task bounds its canvas's first command: one atomic per task.
-		if (g == f.tasks[ti].fanBase) atomicMin(&f.canvasCommandBase[f.tasks[ti].canvas], offset);
+		if (target.local == 0) atomicMin(&f.canvasCommandBase[target.canvas], offset);
 		if (n > 0) {
 			if (!SINGLE && offset + n > f.commandCapacity) atomicOr(&f.counters[2], 1);
-			else if (room) setupTriangle<SETUP_EMIT>(f, g, ti, offset, tally, &clipPolys[threadIdx.x >> 6], together ? jobs : nullptr, jobBase, &corners,
-			                                         SINGLE ? &single : nullptr, SINGLE && f.mode == 0, shader);
+			else if (room) {
+				if (single) {
+					if (f.mode == (SINGLE ? 0 : 1)) storeInputs(f, offset, inputs);
+					else storeFanInputs(f, offset, ti, target.local, corners);
+				}
+				emitTriangle(f, ti, target, corners, single, offset, tally, &clipPolys[threadIdx.x >> 6], together ? jobs : nullptr, jobBase);
+			}
 		}
 	}
 	if (together) {
@@ -684,7 +766,14 @@ __device__ __forceinline__ void setupEmit(const FrameDev &f, int32_t sumBlocks) 
 	if (threadIdx.x == 1 && blockTally[1]) atomicAdd(&f.counters[3], blockTally[1]);
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) k_setup_emit(FrameDev f, int32_t sumBlocks) { setupEmit<false>(f, sumBlocks); }
+// Bound by the latency of its loads, prefixes and atomics, not by bytes: with commands made in one
+// place, the task's fields read as scalars before the prefix and no test repeated by the second pass,
+// one pass takes 18.2 us of a 1080p terrain (20.2 before), 25.4 at 4K (31.6), 246 for 384 uneven jobs
+// (256); two passes 47 us for 8 views of 1280x720 (52) and 148 for 96 of 256x256 (199).  The second
+// pass gains from a fourth wavefront per SIMD where the blocks take several rounds of the chip (96
+// views: 115 us against 132 at three, for 28 B of scratch); the single pass does not (4K: 26.0 against
+// 25.4, the jobs 251 against 246).
+__global__ void __launch_bounds__(SCAN_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) k_setup_emit(FrameDev f, int32_t sumBlocks) { setupEmit<false>(f, sumBlocks); }
 __global__ void __launch_bounds__(SCAN_BLOCK) k_setup_single(FrameDev f) { setupEmit<true>(f, 0); }
 
 // ---------------------------------------------------------------------------------------
@@ -2450,8 +2539,9 @@ __global__ void __launch_bounds__(256) k_occlude_existing(FrameDev f) {
 	__shared__ ClipPolygon clipPolys[256 / 64];
 	const int32_t g = blockIdx.x * blockDim.x + threadIdx.x;
 	if (g >= f.fanTotal) return;
-	BinTally unused{0, 0};
-	(void)setupTriangle<SETUP_OCCLUDE>(f, g, findSegment(f.taskFanEnd, f.taskCount, g), 0, unused, &clipPolys[threadIdx.x >> 6]);
+	const int32_t ti = findSegment(f.taskFanEnd, f.taskCount, g);
+	bool single;
+	(void)setupTriangle<SETUP_OCCLUDE>(f, ti, loadCorners(f, g, ti), &clipPolys[threadIdx.x >> 6], &single);
 }
 
 // renderer_occludeFromTopRows (rendererAPI.cpp:403-474), one thread per cell: the first row of

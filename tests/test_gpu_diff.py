@@ -82,6 +82,27 @@ def test_forward_matches_oracle(api):
         assert (vis >= 0).mean() > 0.3
 
 
+def test_forward_of_clipped_triangles(api):
+    """Differentiable frames whose near plane cuts the object: clipped and whole triangles in the
+    setup's two passes give the oracle's visibility and depth."""
+    views = S.sphere_views(10, 3, 96, 64, seed=5)
+    for v in views:
+        v.near_clip = float(np.linalg.norm(np.asarray(v.cam_location[:3], np.float64))) - 0.8
+    gv = api.GpuViews(views)
+    tex = S.float_texture(64, 2)
+    print("[gpu] clipped differentiable views", flush=True)
+    r = api.DiffRenderer()
+    r.forward(gv.model, gv.views, torch.from_numpy(tex).cuda(), None, api.tuning(clear=True))
+    torch.cuda.synchronize()
+    for i, sc in enumerate(views):
+        col, vis, dep, _ = H.oracle_diff_forward(sc, tex, None)
+        assert np.array_equal(gv.visibility[i].cpu().numpy(), vis), f"view {i} visibility"
+        assert np.array_equal(gv.depth[i].cpu().numpy().view(np.uint32), dep.view(np.uint32)), f"view {i} depth"
+        close = np.isclose(gv.color[i].cpu().numpy(), col, rtol=FORWARD_RTOL, atol=1e-6)
+        assert 1.0 - close.mean() <= FORWARD_FLIP_FRACTION
+        assert (vis >= 0).any()
+
+
 def test_forward_visibility_raster_equals_in_order_raster(api):
     """The differentiable forward through the visibility raster (winner per pixel by atomic max,
     shaded once) writes the same float colours, visibility ids and depths, bit for bit, as the

@@ -498,6 +498,37 @@ def test_setup_block_with_more_commands_than_its_binning_table(api):
     assert_parity(sc, got, H.oracle_render(sc))
 
 
+@pytest.mark.parametrize("sizes", [(1,), (3, 1, 64, 2), (200, 40, 7)])
+def test_tasks_smaller_than_a_wavefront(api, sizes):
+    """Triangles given in tasks of a few at a time, clipped ones among whole ones, share the setup's
+    wavefronts and blocks: the canvases are those of one task bit for bit, and the oracle's."""
+    sc = clip_heavy_scene(triangles=300)
+    whole = S.cube_soup(width=96, height=64, triangles=300, seed=6, cam_distance=2.0, spread=0.6)
+    moved = sc.points.reshape(300, 3, 3)
+    keep = np.arange(300) % 5 != 0
+    # Whole triangles in front of the camera: the soup's, moved along the view axis.
+    moved[keep] = whole.points.reshape(300, 3, 3)[keep] + np.array([0.0, 0.0, 2.5], np.float32)
+    ref = projected_by_oracle(sc)
+    print(f"[gpu] tasks of {sizes}", flush=True)
+    want = H.oracle_render(ref)
+    cam = api.camera_create(True, sc.cam_location, sc.width, sc.height, sc.width_slope, sc.near_clip, sc.far_clip)
+    out = []
+    for split in ((300,), sizes):
+        r = api.renderer_create()
+        color, depth = np.zeros((sc.height, sc.width), np.uint32), np.zeros((sc.height, sc.width), np.float32)
+        api.renderer_begin(r, api.host_image(color), api.host_image(depth))
+        at = k = 0
+        while at < 300:
+            end = min(at + split[k % len(split)], 300)
+            api.renderer_giveTask_triangles(r, ref.projected["cs"][at:end], sc.colors[at:end, :3, :], sc.texcoords[at:end, :3, :], None, None, 0, cam)
+            at, k = end, k + 1
+        api.renderer_end(r)
+        out.append((color, depth, r.stats()[0]))
+    assert out[0][2] == out[1][2] > 300  # some triangles are split, some whole
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1].view(np.uint32), out[1][1].view(np.uint32))
+    assert_parity(sc, out[1][:2], want)
+
+
 def test_points_replaced_by_fewer_are_refused_by_every_draw(api):
     """A model whose points were replaced by fewer after its polygons were added is refused with
     an argument error by renderer_giveTask, the batch and the differentiable forward, and the
