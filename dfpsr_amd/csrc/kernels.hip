@@ -27,11 +27,8 @@ __device__ __forceinline__ Projected projectedPoint(const TaskDev &t, int32_t lo
 
 // ---------------------------------------------------------------------------------------
 // Triangle setup: renderTriangleFromData -> renderTriangleWithShader -> drawClippedTriangle
-// -> drawSubTriangle (renderCore.cpp:220-341).  Returns the number of draw commands the fan
-// triangle makes; with EMIT they are written to out[0..count).
+// -> drawSubTriangle (renderCore.cpp:220-341), one thread per fan triangle.
 // ---------------------------------------------------------------------------------------
-DH Rect canvasRect(const CanvasDev &cv) { return rectSides(0, 0, cv.width, cv.height); }
-
 // n / d for 0 <= n < 2^24 and d >= 1 with a quotient below 2^21 (a command's pair index over
 // its tile columns: at most a canvas's tiles, and its tile rows): both operands are exact in
 // float and the float quotient is within one of the integer one, which one step corrects -- no
@@ -1462,8 +1459,8 @@ template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 // so one command can leave a depth worse than its own other candidate and the argument above
 // fails for that row alone.  The row's pixels (at most one row of the bottom tiles) are walked
 // in submission order, a thread per quad; every other row goes through the keys.  A 1365x767
-// terrain frame took 379 us in order and takes 89 us here, a 1280x720 orthogonal one 333 and
-// 73 us.  Frames of even perspective canvases take kernels without that code, which made the
+// terrain frame took 379 us in order and takes 75 us here, a 1280x720 orthogonal one 333 and
+// 63 us.  Frames of even perspective canvases take kernels without that code, which made the
 // persistent grid's 384-job batch 3 % slower.
 //
 // FORM_ALPHA: the frame has tasks with the Alpha filter, whose blending reads the colour held at that
@@ -2523,8 +2520,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DERIVE
 template __global__ void k_backward<false>(FrameDev, int32_t *);
 template __global__ void k_backward<true>(FrameDev, int32_t *);
 
-// The start of a frame: zeroed counters, tile counts and fill cursors, unset canvas command
-// bases, and the projection of every model point (modelAPI.cpp:237-242), in one launch.
+// The start of a frame: zeroed counters, tile counts and fill cursors, unset canvas command bases
+// and, for differentiable frames, the next forward number.
 __global__ void k_frame_begin(FrameDev f) {
 	const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < COUNTERS) f.counters[i] = 0;

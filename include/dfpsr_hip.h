@@ -273,10 +273,12 @@ int dfpsr_hip_renderer_timing(const dfpsr_hip_renderer *renderer, float out[5]);
  * tile its own workgroup, k > 0 launches k workgroups per CU that pull tiles from a queue;
  * use_graph = 1 captures the launch sequence into a hipGraph and replays it while the work
  * is unchanged; clear = 1 fills the colour canvas with clear_color and the depth canvas with
- * clear_depth first (the caller's image_fill).  raster_path = 0 draws frames whose commands are
- * all Solid and perspective, on canvases of even height, with the visibility raster (each
- * pixel's winning command is found with atomic max over (depth, command) keys and shaded
- * once); raster_path = 1 always walks every tile's commands in order.  binning = 0 lets the
+ * clear_depth first (the caller's image_fill).  raster_path = 0 draws with the visibility raster
+ * (each pixel's winning command is found with atomic max over (depth, command) keys and shaded
+ * once; runs of Alpha commands are blended in order between runs of Solid ones), except canvases
+ * that mix perspective and orthogonal tasks, canvases wider than 32767 pixels and differentiable
+ * frames with the Alpha filter; those, and everything with raster_path = 1, walk every tile's
+ * commands in order.  binning = 0 lets the
  * setup kernel append each command to fixed-size per-tile lists (grown when a tile overflows
  * them, while they stay within a memory bound); binning = 1 always counts, scans and then fills
  * packed lists.  Results never depend on these settings. */
