@@ -161,7 +161,7 @@ private:
 	DevBuf dDiffInputs_, dDiffRecords_, dForwardNumber_;
 	std::vector<int32_t> canvasRegionEnd_;
 	int64_t recordTotal_ = 0;
-	DevBuf dCanvasBase_, dFanCount_, dBlockSums_, dCommands_, dCounters_, dTileCount_, dTileOffset_, dTileFill_, dTileList_, dTileQueue_, dPairRecords_;
+	DevBuf dCanvasBase_, dFanCount_, dBlockSums_, dCommands_, dCounters_, dTileCount_, dTileOffset_, dTileFill_, dTileList_, dTileQueue_, dLongTiles_, dPairRecords_;
 	int32_t *hostCounters_ = nullptr;
 	int32_t *hostCountersDevice_ = nullptr;
 	hipEvent_t events_[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};

@@ -202,6 +202,7 @@ int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks,
 	hipLaunchKernelGGL(k_scan_tiles_add, dim3(tileBlocks), dim3(SCAN_BLOCK), 0, stream, f);
 	hipLaunchKernelGGL(k_bin_fill, dim3(blocksOf(f.pairCapacity, 256)), dim3(256), 0, stream, f);
 	}
+	if (f.longTiles) hipLaunchKernelGGL(k_long_tiles, dim3(blocksOf(tileTotal, 256)), dim3(256), 0, stream, f);
 	if (events) HIP_TRY(hipEventRecord(events_[3], stream));
 	}
 	if (!(parts & 2)) {
@@ -299,6 +300,7 @@ int Frame::run(const RenderOptions &o) {
 	    dBlockSums_.ensure((size_t)(fanBlocks > tileBlocks ? fanBlocks : tileBlocks) * 8) != hipSuccess ||
 	    dCounters_.ensure(2 * COUNTERS * 4) != hipSuccess || dTileCount_.ensure((2 * (size_t)tileTotal + 1) * 4) != hipSuccess ||
 	    dTileOffset_.ensure(((size_t)tileTotal + 1) * 4) != hipSuccess || dTileQueue_.ensure((size_t)tileTotal * 4) != hipSuccess ||
+	    (o.persistentPerCU > 0 && dLongTiles_.ensure((size_t)tileTotal * 4) != hipSuccess) ||
 	    dCanvasBase_.ensure(2 * nC * 4) != hipSuccess)
 		return fail(-4, "device allocation failed");
 
@@ -360,6 +362,7 @@ int Frame::run(const RenderOptions &o) {
 		f.tileOffset = dTileOffset_.as<int32_t>();
 		f.tileList = dTileList_.as<int32_t>();
 		f.tileQueue = dTileQueue_.as<int32_t>();
+		f.longTiles = o.persistentPerCU > 0 && o.mode != 2 ? dLongTiles_.as<int32_t>() : nullptr;
 		f.canvasCommandBase = dCanvasBase_.as<int32_t>() + parity_ * (int32_t)nC;
 		f.pairCapacity = pairCapacity_;
 		f.pairRecords = direct ? nullptr : dPairRecords_.as<PairRecord>();

@@ -816,6 +816,24 @@ __global__ void k_bin_fill(FrameDev f) {
 	f.tileList[f.tileOffset[rec.tile] + rec.slot] = rec.command;
 }
 
+// The tiles that a persistent grid draws first (forEachQueuedTile): those with the longest lists from
+// the front of longTiles on, long ones from its back, in any order within the two.
+__global__ void __launch_bounds__(256) k_long_tiles(FrameDev f) {
+	const int32_t tile = blockIdx.x * blockDim.x + threadIdx.x;
+	const int32_t n = tile < f.tileTotal ? f.tileCount[tile] : 0;
+	const uint64_t below = (1ull << (threadIdx.x & 63)) - 1ull;
+#pragma unroll
+	for (int k = 0; k < 2; k++) {
+		const bool mine = k == 0 ? n > LONGEST_LIST : n > LONG_LIST && n <= LONGEST_LIST;
+		const uint64_t lanes = __ballot(mine);
+		if (lanes == 0) continue;
+		int32_t at = 0;
+		if ((int32_t)(threadIdx.x & 63) == __builtin_ctzll(lanes)) at = atomicAdd(&f.counters[LONG_TILES + k], __popcll(lanes));
+		at = __shfl(at, __builtin_ctzll(lanes), 64) + __popcll(lanes & below);
+		if (mine) f.longTiles[k == 0 ? at : f.tileTotal - 1 - at] = tile;
+	}
+}
+
 // ---------------------------------------------------------------------------------------
 // Tile raster / shade.
 // ---------------------------------------------------------------------------------------
@@ -1395,25 +1413,34 @@ __device__ void forEachQueuedTile(const FrameDev &f, int32_t persistent, int32_t
 	const bool allTiles = f.clearInRaster || f.binCapacity > 0;
 	const int32_t queued = allTiles ? f.tileTotal : f.counters[3];
 	const int32_t x = (int32_t)(blockIdx.x % XCDS);
-	auto visit = [&](int32_t slot) {
-		const int32_t tile = allTiles ? slot : f.tileQueue[slot];
-		if (f.clearInRaster || f.tileCount[tile] > 0) body(tile);
-	};
 	if (!persistent) {
 		const int32_t slot = xcdSlot(x, (int32_t)(blockIdx.x / XCDS));
-		if (slot < queued) visit(slot);
+		if (slot >= queued) return;
+		const int32_t tile = allTiles ? slot : f.tileQueue[slot];
+		if (f.clearInRaster || f.tileCount[tile] > 0) body(tile);
 		return;
 	}
-	// Persistent workgroups walk their own XCD's share first, then help the others.
-	for (int32_t r = 0; r < XCDS; r++) {
-		const int32_t xr = (x + r) % XCDS;
-		while (true) {
-			if (threadIdx.x == 0) *slotLds = xcdSlot(xr, atomicAdd(&f.counters[QUEUE_HEADS + QUEUE_HEAD_STRIDE * xr], 1));
+	// First the tiles with long lists (phases 0 and 1): one of 1 100 commands takes about 500 us, the time
+	// that the whole chip needs for 384 uneven jobs, and begun in tile order it ended 400 us after the
+	// other tiles (raster 913 us; 842 now, as long as the longest list of 2 029 commands takes alone).
+	// Then the others: persistent workgroups walk their own XCD's share first and help the other XCDs.
+	for (int32_t phase = 0; phase < 2 + XCDS; phase++) {
+		const bool longPhase = phase < 2;
+		const int32_t xr = (x + phase - 2) % XCDS;
+		const int32_t limit = longPhase ? f.counters[LONG_TILES + phase] : queued;
+		int32_t *head = longPhase ? &f.counters[LONG_TILES + 2 + phase] : &f.counters[QUEUE_HEADS + QUEUE_HEAD_STRIDE * xr];
+		while (limit > 0) {
+			if (threadIdx.x == 0) {
+				const int32_t ticket = atomicAdd(head, 1);
+				*slotLds = longPhase ? ticket : xcdSlot(xr, ticket);
+			}
 			__syncthreads();
 			const int32_t slot = *slotLds;
 			__syncthreads();
-			if (slot >= queued) break;
-			visit(slot);
+			if (slot >= limit) break;
+			const int32_t tile = longPhase ? f.longTiles[phase == 0 ? slot : f.tileTotal - 1 - slot] : (allTiles ? slot : f.tileQueue[slot]);
+			const int32_t n = f.tileCount[tile];
+			if (longPhase || (n <= LONG_LIST && (f.clearInRaster || n > 0))) body(tile);
 			__syncthreads();
 		}
 	}

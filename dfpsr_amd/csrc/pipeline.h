@@ -122,7 +122,7 @@ struct FrameDev {
 	                              // [6] longest tile list when a bin overflowed,
 	                              // [7] pair records, [8] most commands of one setup block when a
 	                              // single-pass block overflowed, [9..11] the adjoint's queue heads
-	                              // and flag, [QUEUE_HEADS + 32 x] XCD x's raster head
+	                              // and flag, [LONG_TILES..] k_long_tiles, [QUEUE_HEADS + 32 x] XCD x's raster head
 	int32_t blockCapacity;        // single-pass setup: command slots per setup block (0: two passes)
 	int32_t selfClean;            // the raster leaves zeroed counts for the next frame (resetNextCounters)
 	int32_t *nextCounters;        // selfClean: the counter set of the next frame
@@ -139,6 +139,7 @@ struct FrameDev {
 	int32_t pairCapacity;
 	PairRecord *pairRecords;      // pairCapacity (packed lists only)
 	int32_t *tileQueue;           // tiles with at least one command, in tile order (counters[3] of them)
+	int32_t *longTiles;           // persistent grids: tileTotal entries, the longest lists' tiles from the front, long ones' from the back
 	int32_t *canvasCommandBase;   // per canvas: index of its first draw command (visibility ids count from it)
 	int32_t *hostCounters;        // pinned host copy of counters[0..7], written by the raster kernel
 	int32_t tileW, tileH;
@@ -202,6 +203,7 @@ constexpr int32_t SETUP_SUM_BLOCKS = 2048;  // up to this many setup blocks, eac
 __global__ void k_scan_tiles_local(FrameDev f);
 __global__ void k_scan_tiles_add(FrameDev f);
 __global__ void k_bin_fill(FrameDev f);
+__global__ void k_long_tiles(FrameDev f);
 template <int TW, int TH> __global__ void k_raster(FrameDev f, int32_t persistent);
 // Forms of the visibility raster: even perspective canvases with Solid commands alone; any canvases;
 // any canvases and the Alpha filter.
@@ -239,6 +241,10 @@ constexpr int32_t SCAN_BLOCK = 256;
 // The persistent raster's per-XCD queue heads, each on a 128-byte line of its own after the
 // frame's other counters, so that the eight XCDs' tickets do not contend for one line.
 constexpr int32_t QUEUE_HEADS = 32;
+// Counters of the persistent grids' long tiles: how many are the longest and how many long, then the
+// heads of the two queues.  A long tile lists more than LONG_LIST commands, a longest LONGEST_LIST.
+constexpr int32_t LONG_TILES = 16;
+constexpr int32_t LONG_LIST = 128, LONGEST_LIST = 512;
 constexpr int32_t QUEUE_HEAD_STRIDE = 32;
 constexpr int32_t COUNTERS = QUEUE_HEADS + QUEUE_HEAD_STRIDE * XCDS;
 constexpr int32_t HOST_COUNTERS = 16;  // counters[0..15] are copied to pinned host memory

@@ -420,6 +420,33 @@ def test_tile_lists_longer_than_a_round(api, triangles):
     assert np.array_equal(depth.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("triangles", [100, 400, 1500])
+def test_persistent_grid_draws_long_lists_first(api, triangles):
+    """Tiles whose lists are short, long (over 128 commands) and longest (over 512) on one canvas: the
+    persistent grid's order of tiles changes nothing, with and without the fused fill, and no tile is
+    drawn twice or left out."""
+    near = S.cube_soup(width=200, height=70, triangles=triangles, seed=triangles, spread=0.15, cam_distance=3.0)
+    wide = S.cube_soup(width=200, height=70, triangles=200, seed=9, spread=1.2, cam_distance=3.0)
+    a, b = api.GpuScene(near), api.GpuScene(wide)
+    print(f"[gpu] persistent long lists {triangles}", flush=True)
+    for clear in (False, True):
+        out = []
+        for persistent, binning, path, tile_config in ((0, 0, 0, 1), (1, 0, 0, 1), (4, 1, 0, 1), (2, 1, 0, 0), (1, 1, 1, 2)):
+            r = api.renderer_create()
+            api.renderer_setTuning(r, api.tuning(persistent_per_cu=persistent, binning=binning, raster_path=path, tile_config=tile_config,
+                                                 clear=clear, clear_color=0x11223344, clear_depth=0.0))
+            for _ in range(2):
+                color, depth = np.full((70, 200), 7, np.uint32), np.zeros((70, 200), np.float32)
+                api.renderer_begin(r, api.host_image(color), api.host_image(depth))
+                a.give(r)
+                b.give(r)
+                api.renderer_end(r)
+                out.append((color, depth))
+        assert (out[0][1] > 0).any()
+        for color, depth in out[1:]:
+            assert np.array_equal(color, out[0][0]) and np.array_equal(depth.view(np.uint32), out[0][1].view(np.uint32))
+
+
 def test_packed_lists_grow_past_their_first_pair_capacity(api):
     """Commands whose bounds span the whole canvas touch every tile, so the frame makes more
     (tile, command) pairs than the packed lists' first capacity (four per command slot): the
