@@ -3,7 +3,7 @@
 //   zeroed, unless the previous frame's raster left them so] -> triangle setup (the corners
 //   projected, count, emit with per-command row setup, shader inputs and tile counts, in one
 //   pass or in count / scan / emit) -> [tile offsets (scan + ordered tile queue) -> list fill,
-//   for packed lists] -> tile raster.
+//   for packed lists] -> [the long tiles' queues, for persistent grids] -> tile raster.
 // Buffers that depend on data (draw commands, tile pairs) start from an estimate; a pass that
 // runs out of room raises a flag, leaves the canvases untouched, and the frame is run again
 // with the exact sizes.  With RenderOptions::graph the sequence is captured once into a
