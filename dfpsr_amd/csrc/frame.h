@@ -198,6 +198,14 @@ private:
 	bool deferredRaster(const RenderOptions &o) const {
 		return o.rasterPath == 0 && !(alphaAny_ && o.mode == 1) && !mixedCanvas_ && !wideCanvas_;
 	}
+	// The form of the visibility raster that the canvases and tasks need, FORM_IN_ORDER without it.
+	int32_t rasterForm(const RenderOptions &o) const {
+		if (!deferredRaster(o)) return FORM_IN_ORDER;
+		if (alphaAny_) return FORM_ALPHA;
+		bool general = oddCanvas_;
+		for (uint8_t p : projections_) general = general || (p & 2) != 0;
+		return general ? FORM_GENERAL : FORM_PLAIN;
+	}
 };
 
 }  // namespace dfpsr

@@ -217,14 +217,11 @@ int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks,
 		case 2: hipLaunchKernelGGL((k_raster_depth<32, 32>), dim3(xcdGrid(tileTotal)), dim3(32 * 32 / 4), 0, stream, f); break;
 		default: hipLaunchKernelGGL((k_raster_depth<16, 16>), dim3(xcdGrid(tileTotal)), dim3(16 * 16 / 4), 0, stream, f); break;
 		}
-	} else if (deferredRaster(o)) {
-		bool general = oddCanvas_;
-		for (uint8_t p : projections_) general = general || (p & 2) != 0;
-		const int32_t form = alphaAny_ ? FORM_ALPHA : (general ? FORM_GENERAL : FORM_PLAIN);
+	} else if (f.rasterForm != FORM_IN_ORDER) {
 		switch (tileConfig_) {
-		case 1: launchDeferred<32, 16>(f, grid, persistent, form, stream); break;
-		case 2: launchDeferred<32, 32>(f, grid, persistent, form, stream); break;
-		default: launchDeferred<16, 16>(f, grid, persistent, form, stream); break;
+		case 1: launchDeferred<32, 16>(f, grid, persistent, f.rasterForm, stream); break;
+		case 2: launchDeferred<32, 32>(f, grid, persistent, f.rasterForm, stream); break;
+		default: launchDeferred<16, 16>(f, grid, persistent, f.rasterForm, stream); break;
 		}
 	} else if (o.mode == 1) {
 		switch (tileConfig_) {
@@ -377,7 +374,8 @@ int Frame::run(const RenderOptions &o) {
 		// The differentiable frames fill in the raster only with 32-pixel-wide tiles: with 16x16
 		// tiles the separate fill kernel streams the float canvases faster than the one-wave
 		// workgroups' write-back of every pixel (256-view batch forward 1.61 -> 1.98 ms fused).
-		f.clearInRaster = (o.clear && (o.mode == 0 || (o.mode == 1 && f.tileW == 32)) && deferredRaster(o)) ? 1 : 0;
+		f.rasterForm = rasterForm(o);
+		f.clearInRaster = (o.clear && (o.mode == 0 || (o.mode == 1 && f.tileW == 32)) && f.rasterForm != FORM_IN_ORDER) ? 1 : 0;
 		f.clearColor = o.clearColor;
 		f.clearDepth = o.clearDepth;
 		f.mode = o.mode;
@@ -398,7 +396,7 @@ int Frame::run(const RenderOptions &o) {
 		// kernel when the frame before it cleaned the same buffers and it uses no more tiles or
 		// canvases than that frame did.
 		const bool selfClean = !o.graph && single && direct && o.persistentPerCU <= 0 &&
-		                       (o.mode == 2 || (o.mode == 0 && deferredRaster(o)));
+		                       (o.mode == 2 || (o.mode == 0 && f.rasterForm != FORM_IN_ORDER));
 		const uint64_t gens[3] = {dCounters_.generation, dTileCount_.generation, dCanvasBase_.generation};
 		const bool skipBegin = selfClean && clean_ && std::equal(gens, gens + 3, cleanGenerations_) &&
 		                       tileTotal <= cleanTiles_ && (int32_t)nC == cleanCanvases_;
@@ -416,8 +414,8 @@ int Frame::run(const RenderOptions &o) {
 		*(volatile int32_t *)&hostCounters_[2] = -1;
 
 		if (o.graph) {
-			// The graphs stay valid while the launch arguments, the options and the timing switch
-			// are the same.  Events recorded inside a graph cannot be timed, so with timing on the
+			// The graphs stay valid while the launch arguments (which hold everything that picks a
+			// kernel or a grid), the options and the timing switch are the same.  Events recorded inside a graph cannot be timed, so with timing on the
 			// sequence is captured as two graphs -- everything before the raster, and the raster --
 			// with the events recorded between their launches.
 			const uint8_t split = timing ? 1 : 0;

@@ -149,6 +149,8 @@ struct FrameDev {
 	// The visibility raster fills the canvases itself (image_fill) instead of a separate clear:
 	// it then visits every tile, and empty ones only take the fill values.
 	int32_t clearInRaster;
+	int32_t rasterForm;              // FORM_*, from the canvases' heights and the tasks' cameras and filters; here because it
+	                                 // picks the kernel, so that frames of different forms differ in their launch arguments
 	uint32_t clearColor;
 	float clearDepth;
 	// Differentiable frames (mode 1): float RGBA texture (level 0), per-point RGB multipliers
@@ -206,8 +208,8 @@ __global__ void k_bin_fill(FrameDev f);
 __global__ void k_long_tiles(FrameDev f);
 template <int TW, int TH> __global__ void k_raster(FrameDev f, int32_t persistent);
 // Forms of the visibility raster: even perspective canvases with Solid commands alone; any canvases;
-// any canvases and the Alpha filter.
-enum { FORM_PLAIN = 0, FORM_GENERAL = 1, FORM_ALPHA = 2 };
+// any canvases and the Alpha filter.  FORM_IN_ORDER: the in-order raster instead.
+enum { FORM_IN_ORDER = -1, FORM_PLAIN = 0, FORM_GENERAL = 1, FORM_ALPHA = 2 };
 template <int TW, int TH, int P, int FORM> __global__ void k_raster_deferred(FrameDev f);
 template <int TW, int TH> __global__ void k_raster_diff(FrameDev f, int32_t persistent);
 template <int TW, int TH, int P, int FORM> __global__ void k_raster_deferred_diff(FrameDev f);
