@@ -89,7 +89,8 @@ int32_t Frame::addCanvas(const CanvasHost &c) {
 	d.visibility = c.visibility;
 	d.gradColor = c.gradColor;
 	d.diffStride = c.diffStride;
-	d.affine = d.fans = d.dense = 0;
+	d.fans = 0;
+	d.affine = d.dense = 0;
 	d.recordBase = recordTotal_;
 	recordTotal_ += (int64_t)c.width * c.height;
 	if (c.height & 1) oddCanvas_ = true;
@@ -145,7 +146,7 @@ int Frame::addTask(const ModelView &m, const float *transform, const CameraParam
 	CanvasDev &cv = canvases_[(size_t)canvas];
 	if (!camera.perspective) cv.affine = 1;
 	cv.fans += m.fanCount;
-	cv.dense = (int64_t)cv.fans * DENSE_PIXELS_PER_FAN > (int64_t)cv.width * cv.height ? 1 : 0;
+	cv.dense = cv.fans * DENSE_PIXELS_PER_FAN > (int64_t)cv.width * cv.height ? 1 : 0;
 	tasks_.push_back(t);
 	taskPointEnd_.push_back(t.pointBase + m.pointCount);
 	taskFanEnd_.push_back(t.fanBase + m.fanCount);

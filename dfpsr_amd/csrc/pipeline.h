@@ -55,15 +55,17 @@ struct CanvasDev {
 	int32_t tilesX, tilesY;
 	// Differentiable frames: float RGBA colour, visibility id (command * 4 + lane or -1) and the
 	// incoming gradient of the colour, all with diffStride pixels per row.
+	int32_t diffStride;
 	float *diffColor;
 	int32_t *visibility;
 	const float *gradColor;
-	int32_t diffStride;
 	int64_t recordBase;                // differentiable frames: the canvas's first adjoint record
-	int32_t fans;                      // fan triangles of its tasks
+	int64_t fans;                      // fan triangles of its tasks
 	int32_t dense;                     // fewer than DENSE_PIXELS_PER_FAN pixels per fan triangle
 	int32_t affine;                    // its tasks' cameras are orthogonal (the smaller depth wins)
 };
+// The frame's tables are compared with the uploaded ones byte by byte.
+static_assert(__has_unique_object_representations(CanvasDev), "a canvas has no padding");
 
 // Canvases with fewer pixels than this per fan triangle are dense: the setup tests each of their
 // (command, tile) pairs for coverage (pairCovers).  A 1080p terrain has 16 pixels per triangle and
