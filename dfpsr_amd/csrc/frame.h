@@ -59,12 +59,12 @@ struct ModelView {
 	const TextureDesc *const *partLight;
 };
 
-// How a frame is run.
+// How a frame is run.  Part of a captured graph's key, so it has no padding.
 struct RenderOptions {
 	int32_t tileConfig = 0;          // tile shape, see tileConfigW/H
 	int32_t persistentPerCU = 0;     // 0: one raster workgroup per tile; k: k persistent workgroups per CU
-	bool graph = false;              // capture the launch sequence once and replay it while nothing changes
-	bool clear = false;              // fill the canvases before drawing (image_fill)
+	int32_t graph = 0;               // 1: capture the launch sequence once and replay it while nothing changes
+	int32_t clear = 0;               // 1: fill the canvases before drawing (image_fill)
 	uint32_t clearColor = 0;
 	float clearDepth = 0.0f;
 	int32_t mode = 0;                // 0: the reference's RGBA8 shaders; 1: the differentiable float shader;
@@ -72,6 +72,7 @@ struct RenderOptions {
 	int32_t rasterPath = 0;          // 0: visibility raster where the frame allows it; 1: always in order
 	int32_t binning = 0;             // 0: direct per-tile bins while they fit; 1: counted, scanned and filled lists
 };
+static_assert(sizeof(RenderOptions) == 9 * 4, "nine fields of four bytes");
 
 class Frame {
 public:
