@@ -480,6 +480,46 @@ def test_packed_lists_grow_past_their_first_pair_capacity(api):
     assert_parity(sc, first, H.oracle_render(sc))
 
 
+def test_every_buffer_of_a_dense_frame_grows(api):
+    """Thin triangles from behind the camera on a small dense canvas beside a large, nearly empty one: the
+    setup's blocks make more commands than their slots (first pass), then the bins overflow and, grown,
+    pass their bound (second pass), and the lists are packed, whose records include the many pairs that a
+    bound touches and no row covers (third pass, and a fourth with room for them)."""
+    count, w, h = 4096, 160, 128
+    rng = S.Rng(12)
+    ends = rng.uniform(count * 2, -1.0, 1.0).reshape(count, 2)
+    starts = rng.uniform(count * 2, -3.0, 3.0).reshape(count, 2)
+    pts = np.zeros((count, 3, 3), np.float32)
+    pts[:, 0, :2], pts[:, 0, 2] = starts, -0.5
+    pts[:, 1, :2], pts[:, 1, 2] = ends * 2.0, 2.0
+    pts[:, 2] = pts[:, 1] + rng.uniform(count * 3, -0.002, 0.002).reshape(count, 3)
+    away = (np.cross(pts[:, 1] - pts[:, 0], pts[:, 2] - pts[:, 0]) * pts[:, 0]).sum(1) > 0
+    pts[away] = pts[away][:, [0, 2, 1]]  # every triangle faces the camera
+    thin = clip_heavy_scene(count)
+    thin.width, thin.height, thin.points = w, h, pts.reshape(-1, 3)
+    large = S.single_triangles(8192, 8192, [[(10.0, 10.0), (10.0, 60.0), (60.0, 10.0)], [(10.0, 10.0), (60.0, 10.0), (10.0, 60.0)]])
+    g = api.GpuJobs([thin])
+    depth = torch.zeros((8192, 8192), device="cuda")
+    model = api.GpuScene(large)
+    jobs = (api.Job * 2)()
+    jobs[0] = g.jobs[0]
+    jobs[1].depth, jobs[1].model, jobs[1].camera = api.device_image(depth), model.model.handle, model.camera
+    jobs[1].transform[:] = [float(v) for v in S.identity_transform()]
+    print("[gpu] every buffer grows", flush=True)
+    b = api.Batch()
+    b.render(jobs, api.tuning())
+    assert b.stats()[3] == 4
+    got = g.image(0)
+    assert (depth > 0).any()
+    g.clear()
+    r = api.renderer_create()
+    api.renderer_setTuning(r, api.tuning(raster_path=1, binning=1))
+    g.render_plain(r)
+    want = g.image(0)
+    assert (want[1] > 0).mean() > 0.2
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1].view(np.uint32), want[1].view(np.uint32))
+
+
 def test_setup_offsets_scanned_for_many_fan_triangles(api):
     """Above 2048 setup blocks (524288 fan triangles) the command offsets come from the block
     scan kernel instead of each block summing the totals before it; both give the oracle's
