@@ -2312,6 +2312,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DERIVE
 	const int32_t t = (int32_t)threadIdx.x;
 	const int32_t forward = f.diffRecords ? *f.forwardNumber : 0;
 	bool unknown = false;  // a pixel of this thread is left to the DERIVE form
+	const uint32_t commandCount = DERIVE ? (uint32_t)f.counters[0] : 0u;
 
 	// One of the four taps of a pixel into the region's texel table; false when another texel has its place.
 	auto addToTable = [&](int32_t texel, const float4 &value) -> bool {
@@ -2413,7 +2414,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DERIVE
 				if (x + i >= cv.width || y >= cv.height) continue;
 				const int32_t id = cv.visibility[(size_t)y * cv.diffStride + x + i];
 				if (id < 0) continue;
-				const int32_t c = (id >> 2) + commandBase;
+				const int32_t c = (int32_t)((uint32_t)(id >> 2) + (uint32_t)commandBase);
 				bool known = false;
 				if (f.diffRecords) {
 					const DiffRecord rec = f.diffRecords[cv.recordBase + (int64_t)y * cv.width + x + i];
@@ -2425,7 +2426,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DERIVE
 					unknown = unknown || !known;
 					if (!known) continue;
 				} else {
-					if (known) continue;
+					// An id that a forward before the last one left, or the caller, may name no command: of a
+					// view that the last forward drew nothing in (its commandBase is unset), or of more commands.
+					if (known || (uint32_t)c >= commandCount) continue;
 					const DerivedWeights derived = derivedWeights(f.commands, f.triangleRows, c, id & 3, x + i, y, cv.height);
 					if (!derived.touches) continue;
 					weightB[i] = derived.wb;

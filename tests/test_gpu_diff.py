@@ -209,6 +209,88 @@ def test_adjoint_of_kept_and_changed_visibility(api):
         assert_close(adjoint(), base, "kept canvases")
 
 
+def test_adjoint_of_ids_that_name_no_command(api):
+    """Canvases kept from an earlier forward whose view the last one draws nothing in (turned away), and ids
+    past the last command: their pixels are left out, and the other view's gradients are what it gives
+    alone.  The bound is that of test_adjoint_of_kept_and_changed_visibility."""
+    views = small_views()[:2]
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    gv = api.GpuViews(views)
+    for i, g in enumerate(gv.grad):
+        g.copy_(torch.from_numpy(S.Rng(200 + i).uniform(g.numel(), -1.0, 1.0).reshape(tuple(g.shape))))
+    r = api.DiffRenderer()
+
+    def adjoint(renderer):
+        gt, gm = torch.zeros_like(tex), torch.zeros((gv.point_count, 3), device="cuda")
+        renderer.backward(gt, gm)
+        torch.cuda.synchronize()
+        return gt.cpu().double(), gm.cpu().double()
+
+    def assert_close(got, want):
+        for a, b in zip(got, want):
+            assert float((a - b).norm()) <= 2e-5 * float(b.norm())
+
+    print("[gpu] ids that name no command", flush=True)
+    alone = (api.View * 1)(gv.views[0])
+    r.forward(gv.model, alone, tex, None, api.tuning(clear=True))
+    want = adjoint(r)
+    r.forward(gv.model, gv.views, tex, None, api.tuning(clear=True))
+    kept = gv.visibility[1].clone()
+    assert int((kept >= 0).sum()) > 1000
+    position = np.asarray(views[1].cam_location[:3], np.float64)
+    gv.views[1].camera = api.camera_create(True, S.look_at(position, position * 2.0), views[1].width, views[1].height, views[1].width_slope)
+    r.forward(gv.model, gv.views, tex, None, api.tuning())
+    assert torch.equal(gv.visibility[1], kept)
+    assert_close(adjoint(r), want)
+    for far in (0x7FFFFFFF, 4 * int(r.stats()[0])):
+        r.forward(gv.model, alone, tex, None, api.tuning(clear=True))
+        gv.visibility[0][gv.visibility[0] < 0] = far
+        assert_close(adjoint(r), want)
+
+
+def test_adjoint_without_memory_for_records(api):
+    """Views with more pixels than the card has room for records of (1,250 of 4096x4096 that see nothing
+    and share their buffers): the forward draws, and its adjoint, which derives every weight, adds what the
+    visible view alone gives with records.  The next forward on the same object, without those views, keeps
+    records again.  The bound is that of test_adjoint_of_kept_and_changed_visibility."""
+    seen = small_views()[:1]
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    gv = api.GpuViews(seen)
+    gv.grad[0].copy_(torch.from_numpy(S.Rng(9).uniform(gv.grad[0].numel(), -1.0, 1.0).reshape(tuple(gv.grad[0].shape))))
+    side, count = 4096, 1250
+    assert count * side * side * 16 > torch.cuda.mem_get_info()[1]
+    color, grad = (torch.zeros((side, side, 4), device="cuda") for _ in range(2))
+    depth, vis = torch.zeros((side, side), device="cuda"), torch.full((side, side), -1, dtype=torch.int32, device="cuda")
+    position = np.asarray(seen[0].cam_location[:3], np.float64)
+    views = (api.View * (1 + count))()
+    views[0] = gv.views[0]
+    for i in range(1, count + 1):
+        v = views[i]
+        v.color, v.visibility, v.depth, v.grad_color = color.data_ptr(), vis.data_ptr(), depth.data_ptr(), grad.data_ptr()
+        v.width, v.height, v.stride_pixels = side, side, side
+        v.transform[:] = list(gv.views[0].transform)
+        v.camera = api.camera_create(True, S.look_at(position, position * 2.0), side, side, seen[0].width_slope)
+    t = api.tuning(tile_config=2, persistent_per_cu=4)
+
+    def adjoint(renderer, which):
+        gv.visibility[0].fill_(-1)
+        gv.depth[0].zero_()
+        renderer.forward(gv.model, which, tex, None, t)
+        gt, gm = torch.zeros_like(tex), torch.zeros((gv.point_count, 3), device="cuda")
+        renderer.backward(gt, gm, t)
+        torch.cuda.synchronize()
+        return gt.cpu().double(), gm.cpu().double()
+
+    print(f"[gpu] no room for records {count} x {side}^2", flush=True)
+    r = api.DiffRenderer()
+    want = adjoint(api.DiffRenderer(), gv.views)
+    assert float(want[0].norm()) > 0.0 and float(want[1].norm()) > 0.0
+    for which in (views, gv.views):
+        for a, b in zip(adjoint(r, which), want):
+            assert float((a - b).norm()) <= 2e-5 * float(b.norm())
+    assert int((vis >= 0).sum()) == 0
+
+
 def test_adjoint_same_for_every_tile_shape(api):
     """The adjoint walks whatever tiles the forward used: texture and multiplier gradients agree
     across tile shapes up to the order of the float atomics."""
