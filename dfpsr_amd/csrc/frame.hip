@@ -243,6 +243,7 @@ int Frame::enqueue(const FrameDev &f, const RenderOptions &o, int32_t fanBlocks,
 int Frame::prepare() {
 	prepared_ = false;
 	if (tasks_.empty() || canvases_.empty()) return 0;
+	lastRunValid_ = false;  // its tables are replaced
 	if (partTexture_.empty()) partTexture_.push_back(-1);
 	if (textures_.empty()) {
 		TextureDesc none;
@@ -287,6 +288,7 @@ int Frame::run(const RenderOptions &o) {
 	const int32_t fanTotal = taskFanEnd_.back();
 	const int32_t tileTotal = canvasTileEnd_.back();
 	if (fanTotal == 0 || tileTotal == 0) return 0;
+	lastRunValid_ = false;  // its buffers may be replaced from here on
 	const size_t nT = tasks_.size(), nC = canvases_.size();
 	uint8_t *base = (uint8_t *)dTables_.ptr;
 
