@@ -924,6 +924,7 @@ extern "C" int dfpsr_hip_batch_render(dfpsr_hip_batch *b, const dfpsr_hip_job *j
 	}
 	if (!same) {
 		b->frame.reset(o.tileConfig);
+		b->lastTileConfig = -1;  // the frame holds no whole job array until the end of this branch
 		for (int32_t i = 0; i < count; i++) {
 			const dfpsr_hip_job &j = jobs[i];
 			bool hc = hasImage(&j.color), hd = hasImage(&j.depth);
@@ -1062,6 +1063,7 @@ extern "C" int dfpsr_hip_diff_forward(dfpsr_hip_diff *d, const dfpsr_hip_model *
 		rc = checkModelIndices(model, "diff_forward");
 		if (rc) return rc;
 		d->frame.reset(o.tileConfig);
+		d->lastModel = nullptr;  // the frame holds no whole set of views until the end of this branch
 		rc = const_cast<dfpsr_hip_model *>(model)->upload();
 		if (rc) return rc;
 		for (int32_t i = 0; i < count; i++) {

@@ -74,6 +74,25 @@ def test_renderer_tuning_does_not_change_results(setup):
             assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1].view(np.uint32), ref[1].view(np.uint32)), cfg
 
 
+def test_jobs_after_a_refused_call(setup):
+    """A call that is refused for its first job leaves nothing behind: the jobs drawn before it are drawn
+    again by the next call."""
+    api, jobs, g, plain = setup
+    b = api.Batch()
+    t = api.tuning(clear=True)
+    b.render(g.jobs, t)
+    refused = (api.Job * 2)(g.jobs[0], g.jobs[1])
+    refused[0].color.stride_bytes = 2
+    with pytest.raises(api.DfpsrError):
+        b.render(refused, t)
+    g.clear()
+    print("[gpu] batch after a refused call", flush=True)
+    b.render(g.jobs, t)
+    for i in range(len(jobs)):
+        c, d = g.image(i)
+        assert np.array_equal(c, plain[i][0]) and np.array_equal(d.view(np.uint32), plain[i][1].view(np.uint32)), f"job {i}"
+
+
 def test_autotune_picks_a_swept_setting_and_keeps_images(setup):
     api, jobs, g, plain = setup
     b = api.Batch()

@@ -209,6 +209,28 @@ def test_adjoint_of_kept_and_changed_visibility(api):
         assert_close(adjoint(), base, "kept canvases")
 
 
+def test_views_after_a_refused_forward(api):
+    """A forward that is refused for its first view leaves nothing behind: the views drawn before it are
+    drawn again by the next one."""
+    gv = api.GpuViews(small_views())
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    r = api.DiffRenderer()
+    t = api.tuning(clear=True)
+    print("[gpu] forward after a refused one", flush=True)
+    r.forward(gv.model, gv.views, tex, None, t)
+    want = [v.clone() for v in gv.visibility]
+    refused = (api.View * 1)(gv.views[0])
+    refused[0].width = 0
+    with pytest.raises(api.DfpsrError):
+        r.forward(gv.model, refused, tex, None, t)
+    for v in gv.visibility:
+        v.fill_(-1)
+    r.forward(gv.model, gv.views, tex, None, t)
+    torch.cuda.synchronize()
+    for v, w in zip(gv.visibility, want):
+        assert torch.equal(v, w) and bool((w >= 0).any())
+
+
 def test_adjoint_of_ids_that_name_no_command(api):
     """Canvases kept from an earlier forward whose view the last one draws nothing in (turned away), and ids
     past the last command: their pixels are left out, and the other view's gradients are what it gives
