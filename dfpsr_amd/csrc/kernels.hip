@@ -1797,197 +1797,197 @@ __device__ void rasterTileDeferred(const FrameDev &f, int32_t tile, DeferLds<TW,
 			__syncthreads();
 			// Runs of commands of one filter, in submission order (one run for all without the Alpha filter).
 			for (int32_t j0 = 0, j1 = cn; j0 < cn; j0 = j1) {
-			if (ALPHA && colorWrite) {
-				const int32_t lane = t & 63;
-				const uint64_t blended = __ballot(lane < cn && (s.command[lane < cn ? lane : 0].flags & 2) != 0);
-				const bool blends = ((blended >> j0) & 1u) != 0;
-				const uint64_t other = (blends ? ~blended : blended) >> j0;
-				j1 = other != 0 ? tmin(j0 + (int32_t)__builtin_ctzll(other), cn) : cn;
-				if (blends) {
-					blendRun<TW, TH>(s, j0, j1, tileX0, tileY0, cv, textures, depthRead);
-					__syncthreads();
-					continue;
-				}
-			}
-			// Keys start at the held depth with the lowest command part above every command's,
-			// so only a strictly greater depth replaces it; a NaN depth is never replaced.
-			for (int32_t p = t; p < NP; p += NT) {
-				const float d = s.depth[p];
-				s.keys[p] = !depthRead ? 0ull : (d != d ? ~0ull : (((unsigned long long)(depthOrder(d) ^ flip) << 32) | 0xFFFFFFFFull));
-			}
-			if (MODE == 0)
-				for (int32_t w = t; w < NP / 32; w += NT) s.chunkWon[w] = 0u;
-			// Quads of each (command, row pair) inside the tile: the outer span of the row pair
-			// (fillShapeSuper), cut to the tile's columns.
-			int32_t pairCount[PAIRS_PER_THREAD];
-			int32_t threadSum = 0;
-			for (int32_t k = 0; k < PAIRS_PER_THREAD; k++) {
-				const int32_t pr = t * PAIRS_PER_THREAD + k;
-				const int32_t j = pr / RP, rp = pr % RP;
-				int32_t count = 0, x0 = 0;
-				if (pr < PAIRS && j < j1 && (!ALPHA || j >= j0)) {
-					const RowInterval upper = rowInterval(s.rows[j * TH + 2 * rp]), lower = rowInterval(s.rows[j * TH + 2 * rp + 1]);
-					if (upper.right > upper.left || lower.right > lower.left) {
-						const int32_t outerBlockStart = (int32_t)((uint32_t)tmin(upper.left, lower.left) & ~1u);
-						const int32_t outerBlockEnd = (int32_t)(((uint32_t)tmax(upper.right, lower.right) + 1u) & ~1u);
-						x0 = tmax(outerBlockStart, tileX0);
-						const int32_t x1 = tmin(outerBlockEnd, tileX0 + TW);
-						count = x1 > x0 ? (x1 - x0) >> 1 : 0;
+				if (ALPHA && colorWrite) {
+					const int32_t lane = t & 63;
+					const uint64_t blended = __ballot(lane < cn && (s.command[lane < cn ? lane : 0].flags & 2) != 0);
+					const bool blends = ((blended >> j0) & 1u) != 0;
+					const uint64_t other = (blends ? ~blended : blended) >> j0;
+					j1 = other != 0 ? tmin(j0 + (int32_t)__builtin_ctzll(other), cn) : cn;
+					if (blends) {
+						blendRun<TW, TH>(s, j0, j1, tileX0, tileY0, cv, textures, depthRead);
+						__syncthreads();
+						continue;
 					}
 				}
-				if (pr < PAIRS) s.pairStart[pr] = (uint8_t)(x0 - tileX0);
-				pairCount[k] = count;
-				threadSum += count;
-			}
-			int32_t before;
-			const int32_t items = workgroupPrefix<NT>(threadSum, before, s.scan);
-			for (int32_t k = 0; k < PAIRS_PER_THREAD; k++) {
-				const int32_t pr = t * PAIRS_PER_THREAD + k;
-				if (pr < PAIRS) s.pairOffset[pr] = (int16_t)before;
-				for (int32_t i = before; i < before + pairCount[k] && i < ITEM_TABLE; i++)
-					s.pairOfItem[i] = (typename DeferLds<TW, TH, CH, MODE>::PairIndex)pr;
-				before += pairCount[k];
-			}
-			if (t == 0) s.pairOffset[PAIRS] = (int16_t)items;
-			__syncthreads();
-			// Pass 1: one (command, quad) item per thread offers the covered lanes' keys.
-			for (int32_t it = t; it < items; it += NT) {
-				const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
-				const int32_t j = pr / RP, rp = pr % RP;
-				const int32_t px = tileX0 + s.pairStart[pr] + 2 * (it - s.pairOffset[pr]);
-				const int32_t py = tileY0 + 2 * rp;
-				if (GENERAL && py + 1 >= cv.height) continue;  // walked below
-				QuadEval e;
-				const bool ok = evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + 2 * rp]), rowInterval(s.rows[j * TH + 2 * rp + 1]),
-				                         px, py, cv.height, e);
-				if (!ok) continue;
-				// A lane whose row misses the quad is clipped, so a lane that counts is its own pixel.
-				unsigned long long *key = &s.keys[2 * rp * TW + px - tileX0];
-#pragma unroll
-				for (int l = 0; l < 4; l++) {
-					const float d = e.l0[l];
-					const bool offers = (!e.clipSides || e.clip[l]) && (!depthRead || d == d);
-					const uint32_t rank = depthRead ? depthOrder(d) ^ flip : (uint32_t)(j + 1);
-					if (offers) atomicMax(&key[(l >> 1) * TW + (l & 1)], ((unsigned long long)rank << 32) | keyOfCommand(j));
+				// Keys start at the held depth with the lowest command part above every command's,
+				// so only a strictly greater depth replaces it; a NaN depth is never replaced.
+				for (int32_t p = t; p < NP; p += NT) {
+					const float d = s.depth[p];
+					s.keys[p] = !depthRead ? 0ull : (d != d ? ~0ull : (((unsigned long long)(depthOrder(d) ^ flip) << 32) | 0xFFFFFFFFull));
 				}
-			}
-			// The odd canvas's last row: both lanes of a column test the depth held before the
-			// command, then the upper one writes, then the lower one (drawCommand).  The key keeps
-			// the last command that wrote and, in the high half, which of the two lanes it was.
-			if (GENERAL && (cv.height & 1) && tileY0 + TH > cv.height && t < TW / 2) {
-				const int32_t py = cv.height - 1, px = tileX0 + 2 * t;
-				float held[2] = {s.depth[(py - tileY0) * TW + 2 * t], s.depth[(py - tileY0) * TW + 2 * t + 1]};
-				int32_t winner[2] = {-1, -1}, lower[2] = {0, 0};
-				for (int32_t j = j0; j < j1; j++) {
-					const RowSpan upperRow = s.rows[j * TH + py - tileY0];
-					if (upperRow.right <= upperRow.left) continue;
-					QuadEval e;
-					if (!evalQuad(s.command[j].plane, rowInterval(upperRow), rowInterval(s.rows[j * TH + py - tileY0 + 1]), px, py, cv.height, e)) continue;
-#pragma unroll
-					for (int i = 0; i < 2; i++) {
-						const float old = held[i];
-#pragma unroll
-						for (int half = 0; half < 2; half++) {
-							const int l = 2 * half + i;
-							if (!e.clip[l]) continue;
-							if (depthRead && !(cv.affine ? e.l0[l] < old : e.l0[l] > old)) continue;
-							held[i] = e.l0[l];
-							winner[i] = j;
-							lower[i] = half;
+				if (MODE == 0)
+					for (int32_t w = t; w < NP / 32; w += NT) s.chunkWon[w] = 0u;
+				// Quads of each (command, row pair) inside the tile: the outer span of the row pair
+				// (fillShapeSuper), cut to the tile's columns.
+				int32_t pairCount[PAIRS_PER_THREAD];
+				int32_t threadSum = 0;
+				for (int32_t k = 0; k < PAIRS_PER_THREAD; k++) {
+					const int32_t pr = t * PAIRS_PER_THREAD + k;
+					const int32_t j = pr / RP, rp = pr % RP;
+					int32_t count = 0, x0 = 0;
+					if (pr < PAIRS && j < j1 && (!ALPHA || j >= j0)) {
+						const RowInterval upper = rowInterval(s.rows[j * TH + 2 * rp]), lower = rowInterval(s.rows[j * TH + 2 * rp + 1]);
+						if (upper.right > upper.left || lower.right > lower.left) {
+							const int32_t outerBlockStart = (int32_t)((uint32_t)tmin(upper.left, lower.left) & ~1u);
+							const int32_t outerBlockEnd = (int32_t)(((uint32_t)tmax(upper.right, lower.right) + 1u) & ~1u);
+							x0 = tmax(outerBlockStart, tileX0);
+							const int32_t x1 = tmin(outerBlockEnd, tileX0 + TW);
+							count = x1 > x0 ? (x1 - x0) >> 1 : 0;
 						}
 					}
+					if (pr < PAIRS) s.pairStart[pr] = (uint8_t)(x0 - tileX0);
+					pairCount[k] = count;
+					threadSum += count;
 				}
-#pragma unroll
-				for (int i = 0; i < 2; i++)
-					if (winner[i] >= 0)
-						s.keys[(py - tileY0) * TW + 2 * t + i] = ((unsigned long long)lower[i] << 32) | keyOfCommand(winner[i]);
-			}
-			__syncthreads();
-			if (MODE == 0) {
-				// Pass 2: each item that won a lane evaluates its quad again (keeping pass 1's
-				// evaluations would cost more registers than the evaluation), writes the won lanes'
-				// depths, and leaves for every won pixel its weights (in the pixel's key) and its command
-				// and the quad's mip level (in its colour, about to be replaced), so that pass 3 shades
-				// each pixel once with all threads busy.  Only a pixel's winner replaces its key, and the
-				// weight that takes the low half's place is no other command's: those halves are NaNs that
-				// no arithmetic gives, and a NaN weight is stored as the usual one.  So no barrier
-				// separates the reading of the keys from their replacement.
+				int32_t before;
+				const int32_t items = workgroupPrefix<NT>(threadSum, before, s.scan);
+				for (int32_t k = 0; k < PAIRS_PER_THREAD; k++) {
+					const int32_t pr = t * PAIRS_PER_THREAD + k;
+					if (pr < PAIRS) s.pairOffset[pr] = (int16_t)before;
+					for (int32_t i = before; i < before + pairCount[k] && i < ITEM_TABLE; i++)
+						s.pairOfItem[i] = (typename DeferLds<TW, TH, CH, MODE>::PairIndex)pr;
+					before += pairCount[k];
+				}
+				if (t == 0) s.pairOffset[PAIRS] = (int16_t)items;
+				__syncthreads();
+				// Pass 1: one (command, quad) item per thread offers the covered lanes' keys.
 				for (int32_t it = t; it < items; it += NT) {
 					const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
 					const int32_t j = pr / RP, rp = pr % RP;
-					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
-					const int32_t first = qy * TW + qx;
-					const bool oddRow = GENERAL && tileY0 + qy + 1 >= cv.height;
-					const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[first], j, oddRow);
-					if (!mask) continue;
+					const int32_t px = tileX0 + s.pairStart[pr] + 2 * (it - s.pairOffset[pr]);
+					const int32_t py = tileY0 + 2 * rp;
+					if (GENERAL && py + 1 >= cv.height) continue;  // walked below
 					QuadEval e;
-					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
-					              tileY0 + qy, cv.height, e))
-						continue;
-					// The won pixels of the quad's two rows, as bits of their words.
-					const uint32_t upper = (oddRow ? mask | (mask >> 2) : mask) & 3u, lower = oddRow ? 0u : mask >> 2;
-					atomicOr(&s.chunkWon[first >> 5], upper << (first & 31));
-					atomicOr(&s.chunkWon[(first + TW) >> 5], lower << ((first + TW) & 31));
-#pragma unroll
-					for (int l = 0; l < 4; l++)
-						if ((mask >> l) & 1u) s.depth[first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1)] = e.l0[l];
+					const bool ok = evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + 2 * rp]), rowInterval(s.rows[j * TH + 2 * rp + 1]),
+					                         px, py, cv.height, e);
+					if (!ok) continue;
+					// A lane whose row misses the quad is clipped, so a lane that counts is its own pixel.
+					unsigned long long *key = &s.keys[2 * rp * TW + px - tileX0];
+	#pragma unroll
+					for (int l = 0; l < 4; l++) {
+						const float d = e.l0[l];
+						const bool offers = (!e.clipSides || e.clip[l]) && (!depthRead || d == d);
+						const uint32_t rank = depthRead ? depthOrder(d) ^ flip : (uint32_t)(j + 1);
+						if (offers) atomicMax(&key[(l >> 1) * TW + (l & 1)], ((unsigned long long)rank << 32) | keyOfCommand(j));
+					}
+				}
+				// The odd canvas's last row: both lanes of a column test the depth held before the
+				// command, then the upper one writes, then the lower one (drawCommand).  The key keeps
+				// the last command that wrote and, in the high half, which of the two lanes it was.
+				if (GENERAL && (cv.height & 1) && tileY0 + TH > cv.height && t < TW / 2) {
+					const int32_t py = cv.height - 1, px = tileX0 + 2 * t;
+					float held[2] = {s.depth[(py - tileY0) * TW + 2 * t], s.depth[(py - tileY0) * TW + 2 * t + 1]};
+					int32_t winner[2] = {-1, -1}, lower[2] = {0, 0};
+					for (int32_t j = j0; j < j1; j++) {
+						const RowSpan upperRow = s.rows[j * TH + py - tileY0];
+						if (upperRow.right <= upperRow.left) continue;
+						QuadEval e;
+						if (!evalQuad(s.command[j].plane, rowInterval(upperRow), rowInterval(s.rows[j * TH + py - tileY0 + 1]), px, py, cv.height, e)) continue;
+	#pragma unroll
+						for (int i = 0; i < 2; i++) {
+							const float old = held[i];
+	#pragma unroll
+							for (int half = 0; half < 2; half++) {
+								const int l = 2 * half + i;
+								if (!e.clip[l]) continue;
+								if (depthRead && !(cv.affine ? e.l0[l] < old : e.l0[l] > old)) continue;
+								held[i] = e.l0[l];
+								winner[i] = j;
+								lower[i] = half;
+							}
+						}
+					}
+	#pragma unroll
+					for (int i = 0; i < 2; i++)
+						if (winner[i] >= 0)
+							s.keys[(py - tileY0) * TW + 2 * t + i] = ((unsigned long long)lower[i] << 32) | keyOfCommand(winner[i]);
+				}
+				__syncthreads();
+				if (MODE == 0) {
+					// Pass 2: each item that won a lane evaluates its quad again (keeping pass 1's
+					// evaluations would cost more registers than the evaluation), writes the won lanes'
+					// depths, and leaves for every won pixel its weights (in the pixel's key) and its command
+					// and the quad's mip level (in its colour, about to be replaced), so that pass 3 shades
+					// each pixel once with all threads busy.  Only a pixel's winner replaces its key, and the
+					// weight that takes the low half's place is no other command's: those halves are NaNs that
+					// no arithmetic gives, and a NaN weight is stored as the usual one.  So no barrier
+					// separates the reading of the keys from their replacement.
+					for (int32_t it = t; it < items; it += NT) {
+						const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
+						const int32_t j = pr / RP, rp = pr % RP;
+						const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
+						const int32_t first = qy * TW + qx;
+						const bool oddRow = GENERAL && tileY0 + qy + 1 >= cv.height;
+						const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[first], j, oddRow);
+						if (!mask) continue;
+						QuadEval e;
+						if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
+						              tileY0 + qy, cv.height, e))
+							continue;
+						// The won pixels of the quad's two rows, as bits of their words.
+						const uint32_t upper = (oddRow ? mask | (mask >> 2) : mask) & 3u, lower = oddRow ? 0u : mask >> 2;
+						atomicOr(&s.chunkWon[first >> 5], upper << (first & 31));
+						atomicOr(&s.chunkWon[(first + TW) >> 5], lower << ((first + TW) & 31));
+	#pragma unroll
+						for (int l = 0; l < 4; l++)
+							if ((mask >> l) & 1u) s.depth[first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1)] = e.l0[l];
+						if (colorWrite) {
+							const bool affine = (s.command[j].flags & 1) != 0;
+							float wa[4], wb[4], wc[4];
+							for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
+							const uint32_t shade = (uint32_t)j | (quadMip(s.si[j], textures, wa, wb, wc) << 5);
+	#pragma unroll
+							for (int l = 0; l < 4; l++) {
+								if (!((mask >> l) & 1u)) continue;
+								const int32_t p = first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1);
+								const uint32_t weight = wb[l] == wb[l] ? __float_as_uint(wb[l]) : 0x7FC00000u;
+								s.keys[p] = ((unsigned long long)__float_as_uint(wc[l]) << 32) | weight;
+								s.color[p] = shade;
+							}
+						}
+					}
+					__syncthreads();
+					// Pass 3: every pixel won in this chunk, shaded once.
+					for (int32_t w = t; w < NP / 32; w += NT) s.dirty[w] |= s.chunkWon[w];
 					if (colorWrite) {
-						const bool affine = (s.command[j].flags & 1) != 0;
-						float wa[4], wb[4], wc[4];
-						for (int l = 0; l < 4; l++) laneWeights(e, l, affine, wa[l], wb[l], wc[l]);
-						const uint32_t shade = (uint32_t)j | (quadMip(s.si[j], textures, wa, wb, wc) << 5);
-#pragma unroll
+						for (int32_t p = t; p < NP; p += NT) {
+							if (!((s.chunkWon[p >> 5] >> (p & 31)) & 1u)) continue;
+							const uint32_t shade = s.color[p];
+							const unsigned long long weights = s.keys[p];
+							const float wb = __uint_as_float((uint32_t)weights), wc = __uint_as_float((uint32_t)(weights >> 32));
+							s.color[p] = shadePixel(s.si[shade & 31u], textures, 1.0f - (wb + wc), wb, wc, shade >> 5);
+						}
+					}
+				} else {
+					// Pass 2 of the differentiable shader: the same items, evaluated again; each writes
+					// the lanes whose pixels its command won, with the quad's weights as in the in-order
+					// walk.  A pixel has one winner, so exactly one item writes it.
+					for (int32_t it = t; it < items; it += NT) {
+						const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
+						const int32_t j = pr / RP, rp = pr % RP;
+						const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
+						const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[qy * TW + qx], j, GENERAL && tileY0 + qy + 1 >= cv.height);
+						if (!mask) continue;
+						QuadEval e;
+						if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
+						              tileY0 + qy, cv.height, e))
+							continue;
+						// Depths first, so that only the weights and the won lanes' pixels outlive the quad
+						// evaluation while the colours are made.
+						uint32_t slots = 0;
 						for (int l = 0; l < 4; l++) {
 							if (!((mask >> l) & 1u)) continue;
-							const int32_t p = first + (oddRow ? 0 : (l >> 1) * TW) + (l & 1);
-							const uint32_t weight = wb[l] == wb[l] ? __float_as_uint(wb[l]) : 0x7FC00000u;
-							s.keys[p] = ((unsigned long long)__float_as_uint(wc[l]) << 32) | weight;
-							s.color[p] = shade;
+							const int32_t sl = e.slot[l];
+							const int32_t p = (qy + (sl >> 1)) * TW + qx + (sl & 1);
+							s.depth[p] = e.l0[l];
+							atomicOr(&s.dirty[p >> 5], 1u << (p & 31));
+							slots |= (uint32_t)sl << (2 * l);
 						}
+						const int32_t id = (s.list[c0 + j] - f.canvasCommandBase[ci]) * 4;
+						shadeDiffLanes(f, s.command[j], f.diffInputs[s.list[c0 + j]], e, mask, slots, id, forward, cv, tileX0 + qx, tileY0 + qy);
 					}
 				}
 				__syncthreads();
-				// Pass 3: every pixel won in this chunk, shaded once.
-				for (int32_t w = t; w < NP / 32; w += NT) s.dirty[w] |= s.chunkWon[w];
-				if (colorWrite) {
-					for (int32_t p = t; p < NP; p += NT) {
-						if (!((s.chunkWon[p >> 5] >> (p & 31)) & 1u)) continue;
-						const uint32_t shade = s.color[p];
-						const unsigned long long weights = s.keys[p];
-						const float wb = __uint_as_float((uint32_t)weights), wc = __uint_as_float((uint32_t)(weights >> 32));
-						s.color[p] = shadePixel(s.si[shade & 31u], textures, 1.0f - (wb + wc), wb, wc, shade >> 5);
-					}
-				}
-			} else {
-				// Pass 2 of the differentiable shader: the same items, evaluated again; each writes
-				// the lanes whose pixels its command won, with the quad's weights as in the in-order
-				// walk.  A pixel has one winner, so exactly one item writes it.
-				for (int32_t it = t; it < items; it += NT) {
-					const int32_t pr = it < ITEM_TABLE ? (int32_t)s.pairOfItem[it] : segmentOf(s.pairOffset, PAIRS, it);
-					const int32_t j = pr / RP, rp = pr % RP;
-					const int32_t qx = s.pairStart[pr] + 2 * (it - s.pairOffset[pr]), qy = 2 * rp;
-					const uint32_t mask = lanesWon<TW, GENERAL>(&s.keys[qy * TW + qx], j, GENERAL && tileY0 + qy + 1 >= cv.height);
-					if (!mask) continue;
-					QuadEval e;
-					if (!evalQuad(s.command[j].plane, rowInterval(s.rows[j * TH + qy]), rowInterval(s.rows[j * TH + qy + 1]), tileX0 + qx,
-					              tileY0 + qy, cv.height, e))
-						continue;
-					// Depths first, so that only the weights and the won lanes' pixels outlive the quad
-					// evaluation while the colours are made.
-					uint32_t slots = 0;
-					for (int l = 0; l < 4; l++) {
-						if (!((mask >> l) & 1u)) continue;
-						const int32_t sl = e.slot[l];
-						const int32_t p = (qy + (sl >> 1)) * TW + qx + (sl & 1);
-						s.depth[p] = e.l0[l];
-						atomicOr(&s.dirty[p >> 5], 1u << (p & 31));
-						slots |= (uint32_t)sl << (2 * l);
-					}
-					const int32_t id = (s.list[c0 + j] - f.canvasCommandBase[ci]) * 4;
-					shadeDiffLanes(f, s.command[j], f.diffInputs[s.list[c0 + j]], e, mask, slots, id, forward, cv, tileX0 + qx, tileY0 + qy);
-				}
-			}
-			__syncthreads();
 			}
 		}
 		done += take;
