@@ -417,7 +417,7 @@ int Frame::run(const RenderOptions &o) {
 		f.gridH = gridH_;
 		lastRun_ = f;
 		lastRunValid_ = false;
-		// The raster kernel copies counters[0..7] into pinned host memory as it starts; the
+		// The raster kernel copies counters[0..15] into pinned host memory as it starts; the
 		// sentinel, written before anything of the frame is launched, shows whether it did.
 		*(volatile int32_t *)&hostCounters_[2] = -1;
 

@@ -61,10 +61,11 @@ __device__ __forceinline__ int32_t jobOfPair(const BinJob *jobs, int32_t count, 
 // Whether a command's rows can cover a pixel of the w x h tile whose first pixel is (x0, y0); asked
 // for every (command, tile) pair of a dense canvas.  There most triangles are smaller than the pixel
 // spacing and many cover no pixel centre, or none of a tile that their bound touches; a tile sorts,
-// stages and walks every command it lists, so the longest lists bound the frame.  384 uneven jobs:
-// 1 505 512 pairs and a longest list of 5 593 become 1 092 084 and 1 180, the frame 6.2 -> 2.0 ms;
-// 96 views of 256x256: raster 632 -> 358 us.  Where triangles are larger the test does not pay: a
-// 1080p terrain loses a quarter of its pairs, but its raster gains 2 us and its setup loses as much.
+// stages and walks every command it lists, so the longest lists bound the frame.  384 uneven jobs, without
+// and with the test: 1 502 446 pairs and a longest list of 5 593, 1 311 070 and 2 029 (blocks that clip
+// much bin without it); raster 2 006 and 823 us, setup 250 and 245.  96 views of 256x256: raster 388 and
+// 294 us, setup 125 and 148.  Where triangles are larger the test does not pay: a 1080p terrain loses a
+// quarter of its pairs, but its raster gains 2 us and its setup loses as much.
 //
 // A right edge ends row r at trunc(m / a), m = c - b * r (EdgeRows), so it keeps column x >= 1 exactly
 // when m >= a * x, and column 0 when m > -a (truncation); a left edge starts it after trunc(m / a) and
@@ -148,11 +149,11 @@ __device__ __forceinline__ EmitTarget emitTarget(const FrameDev &f, int32_t g, i
 	                  cv.width, cv.height, cv.tileBase, cv.tilesX, cv.tilesY, cv.dense};
 }
 
-// Writes draw command `index` with its row setup and enters it into every tile it can touch: the columns of cut(wholeBound, canvas), the rows of the aligned raster bound
-// (ITriangle2D.cpp:70-84).  With direct bins the index goes into the tile's list at once (in
-// any order: the raster sorts each list); otherwise the tile's count grows here and a pair
-// record (tile, slot, command) keeps the slot until the counts are scanned and the list is
-// filled from the records.
+// Writes draw command `index` with its row setup and enters it into every tile it can touch: the
+// columns of cut(wholeBound, canvas), the rows of the aligned raster bound (ITriangle2D.cpp:70-84).
+// With direct bins the index goes into the tile's list at once (in any order: the raster sorts each
+// list); otherwise the tile's count grows here and a pair record (tile, slot, command) keeps the slot
+// until the counts are scanned and the list is filled from the records.
 __device__ void emitCommand(const FrameDev &f, int32_t index, const Command &cmd, const Projected *P, const EmitTarget &cv,
                             BinTally &tally, BinJob *jobs, int32_t jobBase) {
 	f.commands[index] = cmd;
@@ -376,7 +377,7 @@ __device__ __forceinline__ void emitTriangle(const FrameDev &f, int32_t ti, cons
 				Command c;
 				const f2 is[3] = {S[0].is, S[1].is, S[2].is};
 				c.plane = weightPlanes(is, make3(S[0].cs.z, S[1].cs.z, S[2].cs.z), subB, subC, perspective);
-				c.task = ti; c.fan = target.local; c.flags = target.flags;
+				c.task = ti; c.flags = target.flags;
 				emitCommand(f, offset + count, c, S, target, tally, jobs, jobBase);
 				count++;
 			}
@@ -1260,9 +1261,9 @@ __device__ __attribute__((noinline)) int32_t roundThreshold(const int32_t *src, 
 // the list fits CAP, otherwise the commands in (last, threshold] for a threshold that keeps the round
 // within CAP.  The threshold comes from a histogram of the remaining indices: the bins up to it hold
 // at most CAP of them; when the first bin in use alone holds more, its range is cut into bins in turn
-// (down to single indices, which are distinct).  A round reads the list twice or thrice; searching
-// the threshold by halving the index range read it 31 times, more than half the time of the tiles
-// with over 256 commands (a list of 1 100: 676 of 1 122 us).  Every one of the workgroup's NT threads
+// (down to single indices, which are distinct).  A round reads the list three times (lowest and highest
+// index, histogram, collection) and once more for each range cut again; searching the threshold by
+// halving the index range read it 31 times, more than half the time of the tiles with over 256 commands (a list of 1 100: 676 of 1 122 us).  Every one of the workgroup's NT threads
 // calls it; hist holds ROUND_BINS entries that are free here; returns the round's size.
 template <int NT, int CAP = TILE_SORT_CAP>
 __device__ int32_t nextRound(const int32_t *src, int32_t n, int32_t done, int32_t &last, int32_t *list, int32_t *roundInfo, int32_t *hist) {
@@ -1474,26 +1475,27 @@ template __global__ void k_raster<32, 32>(FrameDev, int32_t);
 // commands in order: every covered lane of every command offers the key (depth order << 32 |
 // ~command) to the pixel with an LDS atomic max -- the order reversed on orthogonal canvases --
 // and only the winning command is shaded for each pixel, with the same quad
-// evaluation, weights and mip selection as the in-order walk.  Without a depth canvas the key
-// is the command alone and the last covering command wins.  Commands run in chunks per tile;
+// evaluation, weights and mip selection as the in-order walk.  Without a depth canvas the high
+// half is the command's number, so the last covering command wins.  Commands run in chunks per tile;
 // each chunk starts from the depths the previous one left.  Work is spread densely: one
 // thread per (command, row) for the exact rows, per (command, covered quad) for the keys and
 // per (command, covered quad) again for the shading of the lanes each command won.
 //
 // FORM_GENERAL: the frame has an orthogonal canvas or one of odd height.  An odd canvas's last row has
-// no row below, and a quad's lower
-// lanes there write the upper row's pixels after the upper lanes (fillerTemplates.h:287-323),
-// so one command can leave a depth worse than its own other candidate and the argument above
-// fails for that row alone.  The row's pixels (at most one row of the bottom tiles) are walked
-// in submission order, a thread per quad; every other row goes through the keys.  A 1365x767
-// terrain frame took 379 us in order and takes 75 us here, a 1280x720 orthogonal one 333 and
-// 63 us.  Frames of even perspective canvases take kernels without that code, which made the
-// persistent grid's 384-job batch 3 % slower.
+// no row below, and a quad's lower lanes there write the upper row's pixels after the upper lanes
+// (fillerTemplates.h:287-323), so one command can leave a depth worse than its own other candidate and
+// the argument above fails for that row alone.  The row's pixels (at most one row of the bottom tiles)
+// are walked in submission order, a thread per quad; every other row goes through the keys.  Whole
+// frames, while such frames were drawn in order and now: 1365x767 terrain 349 and 72 us, 1280x720
+// orthogonal terrain 297 and 63 us.  Frames of even perspective canvases take kernels without that
+// code, which made the persistent grid's 384-job batch 3 % slower.
 //
 // FORM_ALPHA: the frame has tasks with the Alpha filter, whose blending reads the colour held at that
 // moment.  A chunk is then drawn in runs of one filter: runs of Solid commands through the keys, runs
 // of Alpha commands by a walk in submission order with a thread per quad (blendRun).  It includes
-// FORM_GENERAL.
+// FORM_GENERAL.  One Alpha task is enough, and runs may be short: 1 000 objects of one triangle over a
+// terrain at 1280x720, Solid and Alpha in turn, take the raster 51 us (135 in order), 10 objects of 100
+// triangles 46 (147), and 64 jobs with one Alpha task among them 352 us (302 without it, 2 037 in order).
 //
 // Canvases that mix both projections (the depth test's direction changes between commands), canvases
 // wider than 32767 pixels (rows are kept in 16 bits) and differentiable frames with the Alpha filter
@@ -1523,7 +1525,11 @@ constexpr int32_t colorChunk() { return P != 0 && TW * TH >= 512 ? 32 : 16; }
 constexpr int32_t DIFF_CHUNK = 32;
 
 // Threads of a visibility-raster workgroup: four pixels of the tile per thread.  A 32x16 workgroup with
-// chunks of 16 keeps to 14 080 bytes of LDS, so that eleven of them fit a CU.
+// chunks of 16 keeps to 14 080 bytes of LDS, so that eleven of them fit a CU.  The smaller limits that
+// this takes cost nothing that shows, with 256 and 16 against 192 and 8: raster of a 1080p terrain with 8,
+// 12 and 16 textures 52.9, 53.1 and 53.8 against 52.0, 52.7 and 53.4 us (16x16 tiles 56.9, 57.4 and 57.9
+// against 53.4, 53.3 and 53.2); 256x256 canvases with tile lists of 60 to 130 commands on average,
+// 141 to 282 against 139 to 281 us (16x16 tiles 157 to 320 against 158 to 325).
 template <int TW, int TH, int CH> struct DeferShape {
 	static constexpr int32_t NT = TW * TH / 4;
 	static constexpr int32_t CHUNK = CH;                   // commands per chunk

@@ -366,8 +366,13 @@ int dfpsr_hip_diff_forward(dfpsr_hip_diff *diff, const dfpsr_hip_model *model, c
                            int32_t view_count, const float *texture, int32_t log2w, int32_t log2h,
                            const float *multipliers, const dfpsr_hip_tuning *tuning);
 /* Adjoint of the last forward with its visibility fixed: adds dL/dtexture (texture layout) and
- * dL/dmultipliers (point_count x 3) from every view's grad_color, recomputing each pixel's
- * interpolants.  Either output may be NULL.  Float atomics: sums are order-dependent. */
+ * dL/dmultipliers (point_count x 3) from every view's grad_color.  Either output may be NULL.
+ * Float atomics: sums are order-dependent.  The weights of a pixel come from a record of 16 bytes
+ * that the forward leaves for every pixel it draws.  The object keeps room for one record per pixel
+ * of all views, from the first forward in which every view has a grad_color until it is destroyed.
+ * They are derived again where there is no such record: without that memory, and for pixels whose
+ * visibility id is not the one the last forward wrote there.  Ids that name no draw command of the
+ * last forward are left out. */
 int dfpsr_hip_diff_backward(dfpsr_hip_diff *diff, float *grad_texture, float *grad_multipliers,
                             const dfpsr_hip_tuning *tuning);
 int dfpsr_hip_diff_stats(const dfpsr_hip_diff *diff, int64_t out[4]);
