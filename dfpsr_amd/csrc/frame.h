@@ -179,6 +179,9 @@ private:
 	int32_t gridW_ = 0, gridH_ = 0;
 	FrameDev lastRun_;
 	bool lastRunValid_ = false;
+	bool lastRunEmpty_ = false;  // a differentiable run without tasks (no view sees the model)
+	// Fills the canvases of a frame without tasks.
+	int clearCanvases(const RenderOptions &o);
 	hipGraph_t bwdGraph_ = nullptr;
 	hipGraphExec_t bwdGraphExec_ = nullptr;
 	std::vector<uint8_t> bwdGraphKey_;

@@ -280,9 +280,34 @@ int Frame::prepare() {
 	return 0;
 }
 
+int Frame::clearCanvases(const RenderOptions &o) {
+	lastRunValid_ = false;  // its tables are replaced
+	uploadedTables_.clear();
+	const size_t nC = canvases_.size(), offTileEnd = align256(nC * sizeof(CanvasDev)), total = offTileEnd + nC * 4;
+	if (dTables_.ensure(total) != hipSuccess) return fail(-4, "device allocation failed");
+	tables_.assign(total, 0);
+	std::memcpy(&tables_[0], canvases_.data(), nC * sizeof(CanvasDev));
+	std::memcpy(&tables_[offTileEnd], canvasTileEnd_.data(), nC * 4);
+	HIP_TRY(hipMemcpyAsync(dTables_.ptr, tables_.data(), total, hipMemcpyHostToDevice, stream));
+	FrameDev f;
+	std::memset(&f, 0, sizeof(f));
+	f.canvases = (const CanvasDev *)dTables_.ptr;
+	f.canvasCount = (int32_t)nC;
+	f.canvasTileEnd = (const int32_t *)((const uint8_t *)dTables_.ptr + offTileEnd);
+	f.tileTotal = canvasTileEnd_.back();
+	f.tileW = tileConfigW(tileConfig_);
+	f.tileH = tileConfigH(tileConfig_);
+	hipLaunchKernelGGL(k_clear_canvases, dim3(f.tileTotal), dim3(256), 0, stream, f, o.clearColor, o.clearDepth);
+	HIP_TRY(hipGetLastError());
+	HIP_TRY(hipStreamSynchronize(stream));
+	return 0;
+}
+
 int Frame::run(const RenderOptions &o) {
 	stats[0] = stats[1] = stats[2] = stats[3] = 0;
 	for (float &m : stageMs) m = 0.0f;
+	lastRunEmpty_ = o.mode == 1 && tasks_.empty();
+	if (tasks_.empty() && !canvases_.empty() && canvasTileEnd_.back() > 0 && o.clear) return clearCanvases(o);
 	if (!prepared_ || tasks_.empty() || canvases_.empty()) return 0;
 	const int32_t pointTotal = taskPointEnd_.back();
 	const int32_t fanTotal = taskFanEnd_.back();
@@ -556,6 +581,7 @@ int Frame::occludeExisting(float *deviceGrid, int32_t gridW, int32_t gridH) {
 static constexpr int32_t ADJOINT_UNITS_PER_CU = 8;
 
 int Frame::backward(float *gradTexture, float *gradMultipliers, const RenderOptions &o) {
+	if (lastRunEmpty_) return 0;  // nothing was drawn
 	if (!lastRunValid_ || lastRun_.mode != 1) return fail(-2, "backward needs a differentiable forward pass first");
 	FrameDev f = lastRun_;
 	f.gradTexture = gradTexture;

@@ -93,6 +93,44 @@ def test_jobs_after_a_refused_call(setup):
         assert np.array_equal(c, plain[i][0]) and np.array_equal(d.view(np.uint32), plain[i][1].view(np.uint32)), f"job {i}"
 
 
+def test_frames_that_show_nothing_are_cleared(setup):
+    """With the fill on, a frame without any visible task still fills its canvases, and a frame after it
+    draws as ever: the renderer with and without a task out of view, and a batch."""
+    api, jobs, g, plain = setup
+    sc = S.cube_soup(width=50, height=34, triangles=40, seed=3)
+    scene = api.GpuScene(sc)
+    behind = S.identity_transform()
+    behind[2] = -50.0
+    print("[gpu] frames that show nothing", flush=True)
+    r = api.renderer_create()
+    api.renderer_setTuning(r, api.tuning(clear=True, clear_color=0x01020304, clear_depth=0.5))
+    want = api.render_scene(sc, r)
+    for tasks in (0, 1):
+        color, depth = np.full((34, 50), 7, np.uint32), np.full((34, 50), 7, np.float32)
+        api.renderer_begin(r, api.host_image(color), api.host_image(depth))
+        for _ in range(tasks):
+            api.renderer_giveTask(r, scene.model, behind, scene.camera)
+        api.renderer_end(r)
+        assert (color == 0x01020304).all() and (depth == 0.5).all()
+        again = api.render_scene(sc, r)
+        assert np.array_equal(again[0], want[0]) and np.array_equal(again[1], want[1])
+    b = api.Batch()
+    two = (api.Job * 2)(g.jobs[0], g.jobs[1])
+    for j in two:
+        j.transform[:] = [float(v) for v in behind]
+    g.colors[0].fill_(7)
+    g.depths[1].fill_(7.0)
+    b.render(two, api.tuning(clear=True, clear_color=0x01020304, clear_depth=0.5))
+    for i in range(2):
+        c, d = g.image(i)
+        assert (c == 0x01020304).all() and (d == 0.5).all()
+    g.clear()
+    b.render(g.jobs, api.tuning(clear=True))
+    for i in range(len(jobs)):
+        c, d = g.image(i)
+        assert np.array_equal(c, plain[i][0]) and np.array_equal(d.view(np.uint32), plain[i][1].view(np.uint32)), f"job {i}"
+
+
 def test_autotune_picks_a_swept_setting_and_keeps_images(setup):
     api, jobs, g, plain = setup
     b = api.Batch()

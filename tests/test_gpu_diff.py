@@ -231,6 +231,31 @@ def test_views_after_a_refused_forward(api):
         assert torch.equal(v, w) and bool((w >= 0).any())
 
 
+@pytest.mark.parametrize("tile_config", [0, 1])
+def test_views_that_see_nothing(api, tile_config):
+    """A forward whose views all turned away still clears them, and its adjoint adds nothing, also after a
+    forward that drew."""
+    views = small_views()[:2]
+    gv = api.GpuViews(views)
+    tex = torch.from_numpy(S.float_texture(64, 5)).cuda()
+    for g in gv.grad:
+        g.fill_(1.0)
+    r = api.DiffRenderer()
+    print("[gpu] views that see nothing", flush=True)
+    r.forward(gv.model, gv.views, tex, None, api.tuning(clear=True, tile_config=tile_config))
+    assert all(bool((v >= 0).any()) for v in gv.visibility)
+    for i, sc in enumerate(views):
+        position = np.asarray(sc.cam_location[:3], np.float64)
+        gv.views[i].camera = api.camera_create(True, S.look_at(position, position * 2.0), sc.width, sc.height, sc.width_slope)
+    r.forward(gv.model, gv.views, tex, None, api.tuning(clear=True, clear_depth=0.25, tile_config=tile_config))
+    gt = torch.zeros_like(tex)
+    r.backward(gt, None)
+    torch.cuda.synchronize()
+    assert not bool(gt.any())
+    for i in range(len(views)):
+        assert bool((gv.visibility[i] == -1).all()) and not bool(gv.color[i].any()) and bool((gv.depth[i] == 0.25).all())
+
+
 def test_adjoint_of_ids_that_name_no_command(api):
     """Canvases kept from an earlier forward whose view the last one draws nothing in (turned away), and ids
     past the last command: their pixels are left out, and the other view's gradients are what it gives
