@@ -260,7 +260,10 @@ int Frame::prepare() {
 	offTextures_ = align256(offRegionEnd_ + nC * 4);
 	const size_t offParts = align256(offTextures_ + textures_.size() * sizeof(TextureDesc));
 	const size_t total = align256(offParts + partTexture_.size() * 4);
-	if (dTables_.ensure(total) != hipSuccess) return fail(-4, "device allocation failed");
+	if (dTables_.ensure(total) != hipSuccess) {
+		uploadedTables_.clear();  // they are gone
+		return fail(-4, "device allocation failed");
+	}
 	uint8_t *base = (uint8_t *)dTables_.ptr;
 	tables_.assign(total, 0);
 	for (size_t i = 0; i < nT; i++) tasks_[i].partTexture = (const int32_t *)(base + offParts) + partTextureOffset_[i];
@@ -273,6 +276,7 @@ int Frame::prepare() {
 	std::memcpy(&tables_[offTextures_], textures_.data(), textures_.size() * sizeof(TextureDesc));
 	std::memcpy(&tables_[offParts], partTexture_.data(), partTexture_.size() * 4);
 	if (tables_ != uploadedTables_) {
+		uploadedTables_.clear();
 		HIP_TRY(hipMemcpyAsync(dTables_.ptr, tables_.data(), total, hipMemcpyHostToDevice, stream));
 		uploadedTables_ = tables_;
 	}
